@@ -114,5 +114,13 @@ def check(fn: str, code: int) -> None:
         raise ShadyHipError(fn, code, lib().st_last_error().decode())
 
 
+_bound: dict = {}  # entry points by name, bound once
+
+
 def call(fn: str, *args) -> None:
-    check(fn, getattr(lib(), fn)(*args))
+    f = _bound.get(fn)
+    if f is None:
+        f = _bound[fn] = getattr(lib(), fn)
+    code = f(*args)
+    if code != ST_OK:
+        check(fn, code)

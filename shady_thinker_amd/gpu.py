@@ -38,12 +38,17 @@ class GpuContext:
         call("st_context_create", device, ctypes.byref(handle))
         self.handle = handle
         self._stream = None
+        # the current stream's handle without a Stream object around it (0.1
+        # instead of 1 us, on every call)
+        torch.cuda.current_stream(self.device)  # (initialises torch's side of the device)
+        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+        self._raw_stream = raw or (lambda index: torch.cuda.current_stream(index).cuda_stream)
         self.sync_stream()
 
     # -- stream -------------------------------------------------------------
     def sync_stream(self) -> None:
         """Follow torch's current stream (called before every kernel)."""
-        s = self.torch.cuda.current_stream(self.device).cuda_stream
+        s = self._raw_stream(self.device.index)
         if s != self._stream:
             call("st_context_set_stream", self.handle, s)
             self._stream = s

@@ -14,17 +14,17 @@ qweight int32 [K/8, N], scales f16 [K/gs, N], optional qzeros int32
 """
 from __future__ import annotations
 
+import torch
+
 from ._lib import ST_F16, ST_F32, ST_FLAG_TILED, call, lib
 from .gpu import ptr
 from .weights import GptqWeight, Int8Weight
 
 
 def _xdtype(t) -> int:
-    import torch
-
-    if t.dtype == torch.float32:
+    if t.dtype is torch.float32:
         return ST_F32
-    if t.dtype == torch.float16:
+    if t.dtype is torch.float16:
         return ST_F16
     raise TypeError(f"activation dtype {t.dtype} (need float32 or float16)")
 
@@ -37,7 +37,10 @@ def _rows(t, k: int) -> int:
 
 # Argument checks the C ABI cannot make: it receives bare pointers, so a
 # wrong dtype or a short buffer would be read or written past its end on the
-# device. Every helper checks its tensors here before the call.
+# device. Every helper checks its tensors here before the call. A small call's
+# kernel takes 4-5 us, so the checks of the common case are one expression of
+# cheap tensor queries (0.4 us instead of 2 per weight, MI355X host); only a
+# failing call goes on to _need, which finds out what is wrong.
 def _need(t, name: str, dtypes, numel: int) -> None:
     if t is None:
         raise ValueError(f"{name} is required")
@@ -49,30 +52,41 @@ def _need(t, name: str, dtypes, numel: int) -> None:
         raise ValueError(f"{name}: {t.numel()} elements, need at least {numel}")
 
 
-def _torch():
-    import torch
-
-    return torch
+_I32, _F16, _F32 = torch.int32, torch.float16, torch.float32
+_ACT = (_F32, _F16)
+_ACT16 = (_F16,)
+_OUT32 = (_F32,)
 
 
 def _check_gptq(qweight, scales, qzeros, perm, k: int, n: int, group_size: int, flags: int) -> None:
-    torch = _torch()
     if group_size <= 0 or k <= 0 or n <= 0 or k % group_size or k % 8 or n % 8:
         raise ValueError(f"GPTQ weight {k} x {n}, group size {group_size}: K and N multiples of 8, K of the group")
-    words = lib().st_gptq_i4_tiled_words(k, n, group_size) if flags & ST_FLAG_TILED else k // 8 * n
-    _need(qweight, "qweight", (torch.int32,), words)
-    _need(scales, "scales", (torch.float16,), k // group_size * n)
+    g = k // group_size
+    # (tiled: st_gptq_i4_tiled_words)
+    words = (n + 15) // 16 * 16 * (k // 8) if flags & ST_FLAG_TILED else k // 8 * n
+    if (qweight is not None and scales is not None
+            and qweight.dtype is _I32 and qweight.numel() >= words and qweight.is_contiguous()
+            and scales.dtype is _F16 and scales.numel() >= g * n and scales.is_contiguous()
+            and (qzeros is None or qzeros.dtype is _I32 and qzeros.numel() >= g * (n // 8) and qzeros.is_contiguous())
+            and (perm is None or perm.dtype is _I32 and perm.numel() >= k and perm.is_contiguous())):
+        return
+    _need(qweight, "qweight", (_I32,), words)
+    _need(scales, "scales", (_F16,), g * n)
     if qzeros is not None:
-        _need(qzeros, "qzeros", (torch.int32,), k // group_size * (n // 8))
+        _need(qzeros, "qzeros", (_I32,), g * (n // 8))
     if perm is not None:
-        _need(perm, "perm", (torch.int32,), k)
+        _need(perm, "perm", (_I32,), k)
 
 
-def _check_io(x, k: int, out, n: int, x_dtypes=None, out_dtypes=None, name: str = "input") -> int:
-    torch = _torch()
-    _need(x, name, x_dtypes or (torch.float32, torch.float16), 0)
+def _check_io(x, k: int, out, n: int, x_dtypes=_ACT, out_dtypes=_OUT32, name: str = "input") -> int:
+    if x is not None and out is not None and x.dtype in x_dtypes and out.dtype in out_dtypes:
+        numel = x.numel()
+        m = numel // k
+        if m and m * k == numel and out.numel() >= m * n and x.is_contiguous() and out.is_contiguous():
+            return m
+    _need(x, name, x_dtypes, 0)
     m = _rows(x, k)
-    _need(out, "output", out_dtypes or (torch.float32,), m * n)
+    _need(out, "output", out_dtypes, m * n)
     return m
 
 
@@ -89,9 +103,8 @@ def gptq_matvec(gpu, name: str, input, qweight, scales, output, k: int, n: int, 
 def fused_silu_gptq_down(gpu, gate_out, up_out, down_qw, down_sc, output, k: int, n: int, group_size: int = 128,
                          qzeros=None, perm=None, flags: int = 0) -> None:
     """output = (silu(gate_out) * up_out) . dequant(W_down)  (src/model.rs:383-408)."""
-    torch = _torch()
     _check_gptq(down_qw, down_sc, qzeros, perm, k, n, group_size, flags)
-    m = _check_io(gate_out, k, output, n, x_dtypes=(torch.float32,), name="gate_out")
+    m = _check_io(gate_out, k, output, n, x_dtypes=_OUT32, name="gate_out")
     _need(up_out, "up_out", (torch.float32,), m * k)
     gpu.sync_stream()
     call("st_gptq_i4_silu_matvec", gpu.handle, ptr(gate_out), ptr(up_out), ptr(down_qw), ptr(down_sc),
@@ -113,8 +126,6 @@ def gptq_dequant(gpu, qweight, scales, out, k: int, n: int, group_size: int = 12
                  flags: int = 0) -> None:
     """out[k, n] = dequant(W) in out's dtype (float32 exact, bfloat16 RNE as
     src/weights.rs:257-313)."""
-    import torch
-
     od = {torch.float32: 0, torch.bfloat16: 2}.get(out.dtype)
     if od is None:
         raise TypeError(f"dequant output dtype {out.dtype}")
@@ -130,7 +141,6 @@ def gptq_dequant(gpu, qweight, scales, out, k: int, n: int, group_size: int = 12
 def int8_matvec(gpu, x, w, scale, y, k: int, n: int, flags: int = 0) -> None:
     """y[M, n] = x[M, k] . (w[n, k]^T * scale[n]) (INT8 per-channel); flags
     ST_FLAG_TILED when w is in the layout of st_int8_repack."""
-    torch = _torch()
     m = _check_io(x, k, y, n)
     nbytes = lib().st_int8_tiled_bytes(k, n) if flags & ST_FLAG_TILED else k * n
     _need(w, "w", (torch.int8,), nbytes)
@@ -143,8 +153,7 @@ def int8_gemm(gpu, a, w, scale, c, k: int, n: int, flags: int = 0) -> None:
     """c[M, n] = a[M, k] (f16) . (w[n, k]^T * scale[n]): the INT8 prefill
     GEMM (W8A16 on f16 MFMA), c float32 or float16; flags ST_FLAG_TILED when
     w is in the layout of st_int8_repack."""
-    torch = _torch()
-    m = _check_io(a, k, c, n, x_dtypes=(torch.float16,), out_dtypes=(torch.float32, torch.float16), name="a")
+    m = _check_io(a, k, c, n, x_dtypes=_ACT16, out_dtypes=_ACT, name="a")
     nbytes = lib().st_int8_tiled_bytes(k, n) if flags & ST_FLAG_TILED else k * n
     _need(w, "w", (torch.int8,), nbytes)
     _need(scale, "scale", (torch.float32,), n)
@@ -156,10 +165,8 @@ def int8_gemm(gpu, a, w, scale, c, k: int, n: int, flags: int = 0) -> None:
 def gptq_gemm(gpu, a, qweight, scales, c, k: int, n: int, group_size: int = 128, qzeros=None, perm=None,
               flags: int = 0) -> None:
     """c[M, n] = a[M, k] (f16) . dequant(W), c float32 or float16."""
-    import torch
-
     _check_gptq(qweight, scales, qzeros, perm, k, n, group_size, flags)
-    m = _check_io(a, k, c, n, x_dtypes=(torch.float16,), out_dtypes=(torch.float32, torch.float16), name="a")
+    m = _check_io(a, k, c, n, x_dtypes=_ACT16, out_dtypes=_ACT, name="a")
     cd = ST_F32 if c.dtype == torch.float32 else ST_F16
     gpu.sync_stream()
     call("st_gptq_i4_gemm", gpu.handle, ptr(a), ptr(qweight), ptr(scales), ptr(qzeros), ptr(perm), ptr(c), cd, m,
@@ -172,11 +179,9 @@ def gate_up_gemm(gpu, a, gate_qw, gate_sc, up_qw, up_sc, gate_out, up_out, k: in
     float32 or float16 (one dtype), from one pass over a (f16): the M-token
     gate and up projections of src/model.rs:803-811, each bit for bit what
     gptq_gemm gives for that weight."""
-    import torch
-
     _check_gptq(gate_qw, gate_sc, gate_qz, perm, k, n, group_size, flags)
     _check_gptq(up_qw, up_sc, up_qz, perm, k, n, group_size, flags)
-    m = _check_io(a, k, gate_out, n, x_dtypes=(torch.float16,), out_dtypes=(torch.float32, torch.float16), name="a")
+    m = _check_io(a, k, gate_out, n, x_dtypes=_ACT16, out_dtypes=_ACT, name="a")
     _need(up_out, "up_out", (gate_out.dtype,), m * n)
     cd = ST_F32 if gate_out.dtype == torch.float32 else ST_F16
     gpu.sync_stream()
@@ -189,10 +194,8 @@ def fused_silu_gptq_gemm(gpu, gate_out, up_out, down_qw, down_sc, output, k: int
     """output[M, n] = (silu(gate_out) * up_out)[M, k] . dequant(W): the
     M-token form of fused_silu_gptq_down (src/model.rs:383-408) through the
     prefill GEMM; gate_out and up_out f16, output float32 or float16."""
-    import torch
-
     _check_gptq(down_qw, down_sc, qzeros, perm, k, n, group_size, flags)
-    m = _check_io(gate_out, k, output, n, x_dtypes=(torch.float16,), out_dtypes=(torch.float32, torch.float16),
+    m = _check_io(gate_out, k, output, n, x_dtypes=_ACT16, out_dtypes=_ACT,
                   name="gate_out")
     if up_out.shape != gate_out.shape:
         raise ValueError("gate_out and up_out: float16 tensors of one shape")
@@ -206,8 +209,6 @@ def fused_silu_gptq_gemm(gpu, gate_out, up_out, down_qw, down_sc, output, k: int
 def bf16_matvec(gpu, x, w, y, k: int, n: int) -> None:
     """y[M, n] = x[M, k] . w^T, w bf16 [n, k] (Model::bf16_lm_head,
     src/model.rs:455-468 / bf16_matvec.wgsl). x f32 or f16, y f32, M <= 8."""
-    import torch
-
     m = _check_io(x, k, y, n)
     _need(w, "w", (torch.bfloat16, torch.int16, torch.uint16), n * k)
     gpu.sync_stream()
@@ -223,14 +224,14 @@ def linear(gpu, x, w, y) -> None:
     if isinstance(w, GptqWeight):
         m = _rows(x, w.K)
         if m > 32:
-            xa = x if x.dtype == _torch().float16 else x.to(_torch().float16)
+            xa = x if x.dtype == _F16 else x.to(_F16)
             gptq_gemm(gpu, xa, w.qweight, w.scales, y, w.K, w.N, w.group_size, w.qzeros, w.perm, w.flags)
         else:
             gptq_matvec(gpu, "linear", x, w.qweight, w.scales, y, w.K, w.N, w.group_size, w.qzeros, w.perm, w.flags)
     elif isinstance(w, Int8Weight):
         m = _rows(x, w.K)
         if m > 32:
-            xa = x if x.dtype == _torch().float16 else x.to(_torch().float16)
+            xa = x if x.dtype == _F16 else x.to(_F16)
             int8_gemm(gpu, xa, w.w, w.scale, y, w.K, w.N, w.flags)
         else:
             int8_matvec(gpu, x, w.w, w.scale, y, w.K, w.N, w.flags)
