@@ -105,11 +105,11 @@ typedef enum {
     ST_TUNE_NO_KSPLIT,         /* 1: no split-K of several-token decode on few tiles */
     ST_TUNE_SPLIT_TILES_CU,    /* several-token decode: split K up to this many tiles per CU */
     ST_TUNE_TOKEN_BLOCK,       /* decode: tokens per launch (1..16) */
-    ST_TUNE_I4MM_MIN_M,        /* GPTQ decode: fewest tokens for the f16-MFMA kernel (default 5 on more tiles than CUs, 9 on fewer) */
-    ST_TUNE_I4MM_MIN_TILES,    /* GPTQ decode: fewest 16-column tiles for the f16-MFMA kernel */
+    ST_TUNE_I4MM_MIN_M,        /* GPTQ decode: fewest tokens for the f16-MFMA kernels (default 5; on at most one tile per CU 3 with act-order, 9 with K below 2048) */
+    ST_TUNE_I4MM_MIN_TILES,    /* GPTQ decode: fewest 16-column tiles for the f16-MFMA kernels */
     ST_TUNE_I8MM_MIN_M,        /* INT8 decode: fewest tokens for the f16-MFMA kernel */
-    ST_TUNE_GEMM_CB,           /* prefill GEMM: 32-column blocks per wave (1 or 2) */
-    ST_TUNE_GEMM_NO_SPLIT,     /* 1: prefill GEMM without split-K */
+    ST_TUNE_GEMM_CB,           /* prefill GEMM: 32-column blocks per wave (1 or 2); set, the skinny kernel takes no GEMM call */
+    ST_TUNE_GEMM_NO_SPLIT,     /* 1: prefill GEMM without split-K; set (0 or 1), the skinny kernel takes no GEMM call */
     ST_TUNE_STREAM_WAVES,      /* streaming decode kernel: waves per workgroup (8 or 16) */
     ST_TUNE_STREAM_TILES_WG,   /* streaming decode kernel: 16-column tiles per workgroup (0: a workgroup per CU) */
     ST_TUNE_STREAM_SYNC,       /* streaming decode kernel: ring blocks between workgroup barriers (0: none) */
@@ -117,7 +117,7 @@ typedef enum {
     ST_TUNE_I4MM_WAVES,        /* f16-MFMA GPTQ decode: 16 forces 16-wave workgroups (default: 12 when the tiles use at most 12) */
     ST_TUNE_I4MM_PAIR,         /* f16-MFMA gate/up: 0 gives each wave one source (default 1: both sources of a tile per wave) */
     ST_TUNE_I4MM_PREPASS,      /* f16-MFMA GPTQ decode, f32 x: 1 splits x in a pre-pass launch (default: in the kernel, unless act-order) */
-    ST_TUNE_I4MM_SPLIT_TILES,  /* f16-MFMA GPTQ decode on at most one 16-column tile per CU: tiles per workgroup, K split across workgroups (0: limb kernels) */
+    ST_TUNE_I4MM_SPLIT_TILES,  /* f16-MFMA GPTQ decode on at most one 16-column tile per CU: 0 keeps the limb kernels */
     ST_TUNE_COUNT
 } st_tune;
 int st_context_set_tune(st_context *ctx, int knob, int value);
@@ -177,12 +177,12 @@ int st_flush(st_context *ctx);
  * Requires K % group_size == 0, group_size in {64, 128, 256}, N % 8 == 0,
  * 1 <= M <= 32, 16-byte aligned qweight and x. Accumulation: exact integer
  * products of the nibbles with a 3 x 8-bit split of x scaled by a power of
- * two per group, f32 across groups (rel-L2 vs f64 ~1e-7). For 5-32 tokens
- * on tiled weights when N has more 16-column tiles than the GPU has CUs, and
- * 9-32 when it has fewer (then with K split across workgroups and partial
- * sums in the context workspace), with or without perm: f16 MFMA on exact
- * (q - z) and x (f16 x as is; f32 x split into two f16 parts per 128 k while
- * it is staged, or with perm by a pre-pass into the context workspace), f32
+ * two per group, f32 across groups (rel-L2 vs f64 ~1e-7). From 5 tokens on
+ * tiled weights (with at most one 16-column tile per CU from 3 under perm and
+ * from 9 with K below 2048; then K may be split across workgroups, partial sums in the
+ * context workspace): f16 MFMA on exact (q - z) and x (f16 x as is; f32 x
+ * scaled by a power of two and split into two f16 parts; with perm x is
+ * gathered into the context workspace first), f32
  * sums, rel-L2 vs f64 ~1e-7, the weights read once for up to 32 tokens. The
  * same rule applies to st_gptq_i4_gate_up_silu. */
 int st_gptq_i4_matvec(st_context *ctx, const void *x, int x_dtype,

@@ -105,14 +105,30 @@ inline void launch(st_context *ctx, F kernel, dim3 grid, dim3 block, size_t lds,
 // Multi-token INT8 matvec with f16 x on f16 MFMA (i8mm.hip); the caller
 // (st_int8_matvec) has checked the arguments.
 int int8_mm_f16(st_context *ctx, const void *x, const int8_t *w, const float *scale, float *y, int M, int K, int N);
-// Multi-token GPTQ int4 matvec / gate-up on f16 MFMA (i4mm.hip), tiled
-// weights (act-order through perm, or NULL), M <= 16; checked by the caller.
-// -1: not taken (a K split whose partials do not fit the workspace).
-// On at most one 16-column tile per CU it takes groups of kI4mmSplitTiles
-// tiles with K split across workgroups (0: the integer-limb kernels).
-constexpr int kI4mmSplitTiles = 8;
+// Two to eight tokens of GPTQ int4 matvec / gate-up on wide linears, f16 MFMA
+// (i4mm.hip), tiled weights (act-order through perm, or NULL); checked by the
+// caller.
 int int4_mm_f16(st_context *ctx, const void *x, bool x_f32, const int32_t *perm, const uint32_t *const qw[2],
                 const uint16_t *const sc[2], const uint32_t *const qz[2], int zoff, float *y, int M, int K, int N,
                 int gs, int nsrc);
+
+// Skinny GPTQ int4 GEMM with x held in registers (i4xs.hpp), tiled weights.
+// The caller has checked the arguments (K % 128 == 0, alignment, 32-bit
+// offsets of x and the weights). -1, having launched nothing: not taken (the
+// workspace holds neither the gathered x nor the K slices' partial sums).
+struct XsCall {
+    const void *x, *xb;  // xb: x is silu(x) * xb
+    bool x_f16;
+    const int32_t *perm;
+    const uint32_t *qw[2];
+    const uint16_t *sc[2];
+    const uint32_t *qz[2];  // both or neither of two sources
+    int zoff;
+    void *y;
+    bool y_f16;
+    int M, K, N, gs, nsrc;  // nsrc 2: y = silu(gate) * up
+    bool round_w = false;   // f16 x, one source: weights rounded to f16 as the prefill GEMM's
+};
+int int4_xs(st_context *ctx, const XsCall &c);
 
 }  // namespace st

@@ -749,6 +749,18 @@ struct GptqOperand {
     void *c;
 };
 
+// Calls that the skinny kernel takes (i4xs.hpp, tiled weights): up to 160
+// tokens, and up to 256 on weights of at most 2^24 values, whose GEMM is mostly
+// its launches (pre-pass, tiles, split-K reduction). GEMM / skinny, us in a
+// graph with cold weights (MI355X): 33 tokens 4096 x 4096 16.5 / 8.5, 4096 x
+// 14336 27.8 / 17.1, 11008 x 4096 26.5 / 17.4; 128 tokens 24.8 / 11.2, 33.7 /
+// 27.5, 30.8 / 27.4; 160 tokens 25.6 / 16.7, 46.3 / 38.6, 41.6 / 38.3; 256
+// tokens 30.9 / 18.5, 47.0 / 46.4, 44.2 / 53.4.
+bool use_skinny(const st_context *ctx, int M, int K, int N, uint32_t flags) {
+    return (flags & ST_FLAG_TILED) && (M <= 160 || (M <= 256 && (long long)K * N <= (1 << 24))) &&
+           st::tune(ctx, ST_TUNE_GEMM_CB, -1) < 0 && st::tune(ctx, ST_TUNE_GEMM_NO_SPLIT, -1) < 0;
+}
+
 // The prefill GEMM behind the entry points: u == NULL for a . dequant(W),
 // else silu(a) * u . dequant(W); with w1 (u == NULL) also C1 = a . dequant(W1)
 // from the same pre-processed A.
@@ -777,6 +789,19 @@ int gemm_impl(const char *fn, st_context *ctx, const uint16_t *a, const uint16_t
         return st::fail(ST_ERR_WORKSPACE, "%s: needs %zu B of workspace for A (st_context_reserve_workspace)", fn,
                         need);
     if (perm && !st::aligned16(perm)) return st::fail(ST_ERR_ALIGN, "%s: perm must be 16-byte aligned", fn);
+    if (use_skinny(ctx, M, K, N, flags)) {
+        st::XsCall x{a, u, true, perm, {qweight, nullptr}, {scales, nullptr}, {qzeros, nullptr},
+                     (flags & ST_FLAG_ZEROS_PLUS_ONE) ? 1 : 0, c, c_dtype == ST_F16, M, K, N, group_size, 1, true};
+        int rc = st::int4_xs(ctx, x);
+        if (rc == ST_OK && w1) {
+            x.qw[0] = w1->qweight;
+            x.sc[0] = w1->scales;
+            x.qz[0] = w1->qzeros;
+            x.y = w1->c;
+            rc = st::int4_xs(ctx, x);
+        }
+        if (rc != -1) return rc;
+    }
     _Float16 *A = reinterpret_cast<_Float16 *>(ctx->ws);
     float *rsc = u ? reinterpret_cast<float *>(reinterpret_cast<char *>(ctx->ws) + rsc_off) : nullptr;
     st::launch(ctx, prep_a_kernel, dim3(M), dim3(256), (size_t)K * sizeof(_Float16),

@@ -1,10 +1,14 @@
-// Multi-token GPTQ int4 decode on f16 MFMA (a skinny GEMM), for 2..32
-// tokens on tiled weights (st_gptq_i4_repack; act-order x
-// through a pre-pass):
+// Few-token GPTQ int4 decode on f16 MFMA for wide linears (a skinny GEMM of
+// 16 rows: 2..8 tokens of f32 x, 2..16 of f16) on tiled weights
+// (st_gptq_i4_repack; act-order x through a pre-pass):
 //   y[m, n]  = sum_g s[g, n] * sum_{k in g} (q[k, n] - z[g, n]) * x[m, k]
 //   (st_gptq_i4_matvec), or silu(gate) * up of two such sums
 //   (st_gptq_i4_gate_up_silu). Semantics of gptq_matvec.wgsl:51-58 and
 //   fused_gate_up_silu_4t.wgsl:24-90; the reference runs one token at a time.
+// i4xs.hpp, which holds x in registers, takes everything else from a few
+// tokens on; here x is shared through LDS chunk by chunk, which starts the
+// weights' arithmetic earlier when there is little of it (the launch rule
+// and both sides' times are at launch_f16 in qmv.hip).
 //
 //  * Exact products: (q - z) is an integer in [-15, 15], exact in f16 (the
 //    f16 1024 bias: 1024 + q, minus 1024 + z). f16 x is used as is. f32 x is
@@ -25,9 +29,6 @@
 //    LDS (double buffered, one chunk ahead); each wave keeps a ring of three
 //    chunks of weights, scales and zeros, two in flight while it computes
 //    one. Partial sums meet in LDS in a fixed order.
-//  * On at most one tile per CU (narrow linears): groups of tiles with K
-//    split across workgroups, whole chunks per slice; each slice's sums go
-//    to the workspace and i4mm_reduce_kernel adds them in slice order.
 #include "common.hpp"
 
 #include <algorithm>
@@ -49,7 +50,6 @@ constexpr int kTileN = 16;
 constexpr int kRsrcWord3 = 0x00020000;     // raw 32-bit buffer data (gfx9-class)
 constexpr unsigned kNoLoad = 0x80000000u;  // buffer offset past every resource: reads 0, touches no memory
 constexpr int kMaxTilesPerWg = 8;
-constexpr int kMaxSplit = 16;  // K slices of a split launch
 
 // v_and_or_b32 with both constants in registers (a VOP3 takes no literal).
 __device__ __forceinline__ unsigned and_or(unsigned a, unsigned m, unsigned c) {
@@ -169,7 +169,7 @@ __global__ __launch_bounds__(256) void i4mm_prep_kernel(const float *__restrict_
 
 // XM: f16 x (0), the pre-pass output (1: xp, pe, two f16 rows per token) or
 // f32 x split at staging (2);
-// NSRC: 1 (matvec) or 2 (gate/up); MB: 16-row MFMA blocks; KCU: 128-k units
+// NSRC: 1 (matvec) or 2 (gate/up); KCU: 128-k units
 // per staged chunk; GW: units per wave per chunk (S = KCU / GW waves per tile
 // and source).
 // NW waves per workgroup: 16, or 12 when the workgroup's tiles use at most 12
@@ -178,18 +178,19 @@ __global__ __launch_bounds__(256) void i4mm_prep_kernel(const float *__restrict_
 // weight of a tile, so every x fragment read from LDS and every load
 // address serves two MFMA chains.
 // HZ: some source has zero points (without, no zero words are loaded: z = 8).
-template <int XM, int NSRC, int MB, int GS, int KCU, int GW, int NW, bool PAIR, bool HZ>
+template <int XM, int NSRC, int GS, int KCU, int GW, int NW, bool PAIR, bool HZ>
 __global__ __launch_bounds__(64 * NW) void i4mm_kernel(const void *__restrict__ x, const float *__restrict__ pe,
                                                         const uint32_t *__restrict__ qw0,
                                                         const uint16_t *__restrict__ sc0, const uint32_t *__restrict__ qz0,
                                                         const uint32_t *__restrict__ qw1, const uint16_t *__restrict__ sc1,
                                                         const uint32_t *__restrict__ qz1, int zoff, float *__restrict__ y,
-                                                        int M, int K, int N, int ntiles, float *__restrict__ part, int ks) {
+                                                        int M, int K, int N, int ntiles) {
     // XM: 0 f16 x; 1 f32 x split by i4mm_prep_kernel (hi / lo rows and
     // factors in the workspace); 2 f32 x split here, at staging, with the
     // same arithmetic (no pre-pass launch)
     constexpr bool F32X = XM != 0;
     constexpr bool RAW = XM == 2;
+    constexpr int MB = 1;                 // 16-row MFMA blocks
     constexpr int kKC = 128 * KCU;        // k per staged chunk
     constexpr int kPitch = kKC + 8;       // halves per LDS row (16-byte pad: fragment rows on distinct banks)
     constexpr int S = KCU / GW;
@@ -225,19 +226,14 @@ __global__ __launch_bounds__(64 * NW) void i4mm_kernel(const void *__restrict__ 
     // weight, scale and zero resources in VGPRs, every load of them in a
     // waterfall loop.
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // K split (ks > 1): workgroup b takes K slice b % ks of tile group b / ks
-    const int kslice = blockIdx.x % ks, ngrp = gridDim.x / ks, grp = blockIdx.x / ks;
-    const int t0 = (int)((long long)grp * ntiles / ngrp);
-    const int t1 = (int)((long long)(grp + 1) * ntiles / ngrp);
+    const int t0 = (int)((long long)blockIdx.x * ntiles / gridDim.x);
+    const int t1 = (int)((long long)(blockIdx.x + 1) * ntiles / gridDim.x);
     const int tb = PAIR ? wave / S : wave / (NSRC * S), src = PAIR ? 0 : (wave / S) % NSRC, slice = wave % S;
     const bool active = t0 + tb < t1;
     const int T = min(t0 + tb, ntiles - 1);
     const int G = K / GS;
     const int units = K / 128;
-    // this slice's chunks [cb, ce), its units below uend, its k below kend
-    const int nch_all = (units + KCU - 1) / KCU;
-    const int cb = kslice * nch_all / ks, ce = (kslice + 1) * nch_all / ks;
-    const int uend = min(units, ce * KCU), kend = min(K, ce * kKC);
+    const int nch = (units + KCU - 1) / KCU;
     const int q = lane >> 4, r16 = lane & 15;
     const int n = min(kTileN * T + r16, N - 1);  // this lane's column (the last tile's padding repeats N - 1)
 
@@ -276,7 +272,7 @@ __global__ __launch_bounds__(64 * NW) void i4mm_kernel(const void *__restrict__ 
             for (int j = 0; j < XLR; ++j) {
                 const int i = j * kThr + tid;
                 const int t = i / (kKC / 8), k = c * kKC + 8 * (i % (kKC / 8));
-                const bool ok = i < RITEMS && t < M && k < kend;
+                const bool ok = i < RITEMS && t < M && k < K;
                 const unsigned o = ok ? (unsigned)(t * K + k) * 4u : kNoLoad;
                 xr[2 * j] = __builtin_amdgcn_raw_buffer_load_b128(rx, o, 0, 0);
                 xr[2 * j + 1] = __builtin_amdgcn_raw_buffer_load_b128(rx, ok ? o + 16u : kNoLoad, 0, 0);
@@ -287,12 +283,12 @@ __global__ __launch_bounds__(64 * NW) void i4mm_kernel(const void *__restrict__ 
         for (int j = 0; j < XL; ++j) {
             const int i = j * kThr + tid;
             const int row = i / (kKC / 8), k = c * kKC + 8 * (i % (kKC / 8));
-            const bool ok = i < XITEMS && row < nrows && k < kend;
+            const bool ok = i < XITEMS && row < nrows && k < K;
             xr[j] = __builtin_amdgcn_raw_buffer_load_b128(rx, ok ? (unsigned)(row * K + k) * 2u : kNoLoad, 0, 0);
         }
         if constexpr (F32X) {
             const int t = tid % PT, u = c * KCU + tid / PT;
-            const bool ok = tid < KCU * PT && t < M && u < uend;
+            const bool ok = tid < KCU * PT && t < M && u < units;
             pr = __builtin_amdgcn_raw_buffer_load_b32(rp, ok ? (unsigned)(t * units + u) * 4u : kNoLoad, 0, 0);
         }
     };
@@ -350,7 +346,7 @@ __global__ __launch_bounds__(64 * NW) void i4mm_kernel(const void *__restrict__ 
         for (int gi = 0; gi < GW; ++gi) {
             Unit<GS> &du = dsts[gi][ps];
             const int u = c * KCU + slice * GW + gi;
-            const bool ok = active && u < uend;
+            const bool ok = active && u < units;
             if constexpr (GS == 64) {
                 unsigned o0 = ok ? (unsigned)(((T * G + 2 * u) * 64 + lane) * 8) : kNoLoad;
                 asm volatile("" : "+v"(o0));
@@ -467,10 +463,10 @@ __global__ __launch_bounds__(64 * NW) void i4mm_kernel(const void *__restrict__ 
     // c - 2 into ring slot c % 3. Six chunks per trip so that every buffer
     // index is compile-time; loads are unconditional (past the end they read
     // nothing), so the compiler's wait counts are the same on every path.
-    load_x(xr2[0], pr2[0], cb);
-    if constexpr (XS == 2) load_x(xr2[1], pr2[1], cb + 1);
-    load_u(ur[0], cb);
-    load_u(ur[1], cb + 1);
+    load_x(xr2[0], pr2[0], 0);
+    if constexpr (XS == 2) load_x(xr2[1], pr2[1], 1);
+    load_u(ur[0], 0);
+    load_u(ur[1], 1);
     store_x(xr2[0], pr2[0], xs0, ps0);
     lds_barrier();
     auto chunk = [&](auto P, int c) {
@@ -484,17 +480,17 @@ __global__ __launch_bounds__(64 * NW) void i4mm_kernel(const void *__restrict__ 
         store_x(xr2[(p + 1) % XS], pr2[(p + 1) % XS], p % 2 ? xs0 : xs1, p % 2 ? ps0 : ps1);  // chunk c + 1
         lds_barrier();
     };
-    for (int c = cb; c < ce; c += 6) {
+    for (int c = 0; c < nch; c += 6) {
         chunk(std::integral_constant<int, 0>{}, c);
-        if (c + 1 >= ce) break;
+        if (c + 1 >= nch) break;
         chunk(std::integral_constant<int, 1>{}, c + 1);
-        if (c + 2 >= ce) break;
+        if (c + 2 >= nch) break;
         chunk(std::integral_constant<int, 2>{}, c + 2);
-        if (c + 3 >= ce) break;
+        if (c + 3 >= nch) break;
         chunk(std::integral_constant<int, 3>{}, c + 3);
-        if (c + 4 >= ce) break;
+        if (c + 4 >= nch) break;
         chunk(std::integral_constant<int, 4>{}, c + 4);
-        if (c + 5 >= ce) break;
+        if (c + 5 >= nch) break;
         chunk(std::integral_constant<int, 5>{}, c + 5);
     }
 
@@ -527,10 +523,7 @@ __global__ __launch_bounds__(64 * NW) void i4mm_kernel(const void *__restrict__ 
             }
             const int m = F32X ? TPB * mb + 2 * q + i : 16 * mb + 4 * q + i;
             if (m >= M) continue;
-            if (ks > 1) {  // the slice's sums, to i4mm_reduce_kernel
-#pragma unroll
-                for (int sr = 0; sr < NSRC; ++sr) part[((size_t)(kslice * NSRC + sr) * M + m) * N + nc] = v[sr];
-            } else if constexpr (NSRC == 2) {
+            if constexpr (NSRC == 2) {
                 y[(size_t)m * N + nc] = silu_f(v[0]) * v[1];
             } else {
                 y[(size_t)m * N + nc] = v[0];
@@ -538,54 +531,22 @@ __global__ __launch_bounds__(64 * NW) void i4mm_kernel(const void *__restrict__ 
         }
 }
 
-// K split: y = epilogue(sum over slices s < ks of part[s][src]), the slices
-// added in order (deterministic), the epilogue silu(gate) * up for two sources.
-template <int NSRC>
-__global__ __launch_bounds__(256) void i4mm_reduce_kernel(const float *__restrict__ part, float *__restrict__ y, int MN,
-                                                          int ks) {
-    const int idx = blockIdx.x * 256 + threadIdx.x;
-    if (idx >= MN) return;
-    float t[kMaxSplit][NSRC];  // every slice's load issued before the first add
-#pragma unroll
-    for (int s = 0; s < kMaxSplit; ++s)
-#pragma unroll
-        for (int sr = 0; sr < NSRC; ++sr) t[s][sr] = s < ks ? part[(size_t)(s * NSRC + sr) * MN + idx] : 0.f;
-    float v[NSRC];
-#pragma unroll
-    for (int sr = 0; sr < NSRC; ++sr) {
-        v[sr] = 0.f;
-#pragma unroll
-        for (int s = 0; s < kMaxSplit; ++s)
-            if (s < ks) v[sr] += t[s][sr];
-    }
-    y[idx] = NSRC == 2 ? silu_f(v[0]) * v[1] : v[0];
-}
-
-template <int XM, int NSRC, int MB, int GS>
+template <int XM, int NSRC, int GS>
 int launch_gs(st_context *ctx, const void *x, const float *pe, const uint32_t *const *qw, const uint16_t *const *sc,
               const uint32_t *const *qz, int zoff, float *y, int M, int K, int N, int ntiles, int G, int wpt, int nw,
-              bool pair, float *part, int ks) {
-    const dim3 grid(G * ks);
+              bool pair) {
+    const dim3 grid(G);
     const bool hz = qz[0] || (NSRC == 2 && qz[1]);
 #define ST_I4MM_P(KCU_, GW_, NW_, PAIR_)                                                                           \
     do {                                                                                                           \
         if (hz)                                                                                                    \
-            st::launch(ctx, (i4mm_kernel<XM, NSRC, MB, GS, KCU_, GW_, NW_, PAIR_, true>), grid, dim3(64 * NW_), 0,  \
-                       x, pe, qw[0], sc[0], qz[0], qw[1], sc[1], qz[1], zoff, y, M, K, N, ntiles, part, ks);    \
+            st::launch(ctx, (i4mm_kernel<XM, NSRC, GS, KCU_, GW_, NW_, PAIR_, true>), grid, dim3(64 * NW_), 0,  \
+                       x, pe, qw[0], sc[0], qz[0], qw[1], sc[1], qz[1], zoff, y, M, K, N, ntiles);    \
         else                                                                                                       \
-            st::launch(ctx, (i4mm_kernel<XM, NSRC, MB, GS, KCU_, GW_, NW_, PAIR_, false>), grid, dim3(64 * NW_), 0, \
-                       x, pe, qw[0], sc[0], qz[0], qw[1], sc[1], qz[1], zoff, y, M, K, N, ntiles, part, ks);    \
+            st::launch(ctx, (i4mm_kernel<XM, NSRC, GS, KCU_, GW_, NW_, PAIR_, false>), grid, dim3(64 * NW_), 0, \
+                       x, pe, qw[0], sc[0], qz[0], qw[1], sc[1], qz[1], zoff, y, M, K, N, ntiles);    \
     } while (0)
 #define ST_I4MM(KCU_, GW_, NW_) ST_I4MM_P(KCU_, GW_, NW_, false)
-    // 17-32 tokens of f32 x (64 MFMA rows): 2-unit chunks (the two x buffers
-    // of 4-unit chunks would not fit the LDS)
-    if constexpr (MB == 4) {
-        if (nw == 12)
-            ST_I4MM(2, 1, 12);
-        else
-            ST_I4MM(2, 1, 16);
-        return st::launch_check("i4mm_kernel");
-    } else {
         // gate/up with both sources in a wave: wpt is then waves per tile pair
         if constexpr (NSRC == 2 && GS != 64) {  // (group 64 with two sources per wave spills)
             if (pair) {
@@ -618,7 +579,6 @@ int launch_gs(st_context *ctx, const void *x, const float *pe, const uint32_t *c
                 ST_I4MM(2, 1, 16);
         }
         return st::launch_check("i4mm_kernel");
-    }
 #undef ST_I4MM
 #undef ST_I4MM_P
 }
@@ -637,72 +597,36 @@ __global__ __launch_bounds__(256) void i4mm_gather_kernel(const uint16_t *__rest
     *reinterpret_cast<u32x4 *>(xg + i) = v;
 }
 
-template <int XM, int NSRC, int MB>
-int launch_mb(st_context *ctx, const void *x, const float *pe, const uint32_t *const *qw, const uint16_t *const *sc,
-              const uint32_t *const *qz, int zoff, float *y, int M, int K, int N, int gs, int ntiles, int G, int wpt,
-              int nw, bool pair, float *part, int ks) {
-    switch (gs) {
-        case 64:  // (four 16-row blocks with group 64 spill: the entry point takes 16-token blocks)
-            if constexpr (MB == 4)
-                return st::fail(ST_ERR_UNSUPPORTED, "int4_mm_f16: group 64 with %d tokens of f32 x", M);
-            else
-                return launch_gs<XM, NSRC, MB, 64>(ctx, x, pe, qw, sc, qz, zoff, y, M, K, N, ntiles, G, wpt, nw, pair, part,
-                                                   ks);
-        case 128:
-            return launch_gs<XM, NSRC, MB, 128>(ctx, x, pe, qw, sc, qz, zoff, y, M, K, N, ntiles, G, wpt, nw, pair, part, ks);
-        default:
-            return launch_gs<XM, NSRC, MB, 256>(ctx, x, pe, qw, sc, qz, zoff, y, M, K, N, ntiles, G, wpt, nw, pair, part, ks);
-    }
-}
-
 template <int XM, int NSRC>
 int launch_src(st_context *ctx, const void *x, const float *pe, const uint32_t *const *qw, const uint16_t *const *sc,
                const uint32_t *const *qz, int zoff, float *y, int M, int K, int N, int gs, int ntiles, int G, int wpt,
-               int nw, bool pair, float *part, int ks) {
-    // tokens per 16-row block: 8 (f32 x: hi and lo rows) or 16; four blocks
-    // only with f32 x (17-32 tokens)
-    const int mb = (M * (XM ? 2 : 1) + 15) / 16;
-    int rc;
-    if (mb <= 1)
-        rc = launch_mb<XM, NSRC, 1>(ctx, x, pe, qw, sc, qz, zoff, y, M, K, N, gs, ntiles, G, wpt, nw, pair, part, ks);
-    else if (mb <= 2)
-        rc = launch_mb<XM, NSRC, 2>(ctx, x, pe, qw, sc, qz, zoff, y, M, K, N, gs, ntiles, G, wpt, nw, pair, part, ks);
-    else if constexpr (XM != 0)
-        rc = launch_mb<XM, NSRC, 4>(ctx, x, pe, qw, sc, qz, zoff, y, M, K, N, gs, ntiles, G, wpt, nw, pair, part, ks);
-    else
-        return st::fail(ST_ERR_SHAPE, "int4_mm_f16: %d tokens", M);
-    if (rc || ks == 1) return rc;
-    const int mn = M * N;
-    st::launch(ctx, (i4mm_reduce_kernel<NSRC>), dim3((mn + 255) / 256), dim3(256), 0, part, y, mn, ks);
-    return st::launch_check("i4mm_reduce_kernel");
+               int nw, bool pair) {
+    switch (gs) {
+        case 64: return launch_gs<XM, NSRC, 64>(ctx, x, pe, qw, sc, qz, zoff, y, M, K, N, ntiles, G, wpt, nw, pair);
+        case 128: return launch_gs<XM, NSRC, 128>(ctx, x, pe, qw, sc, qz, zoff, y, M, K, N, ntiles, G, wpt, nw, pair);
+        default: return launch_gs<XM, NSRC, 256>(ctx, x, pe, qw, sc, qz, zoff, y, M, K, N, ntiles, G, wpt, nw, pair);
+    }
 }
 
 }  // namespace
 
 namespace st {
 
-// Arguments are checked by the entry points (tiled weights, M <= 16, K %
-// 128 == 0, K % group_size == 0, N % 8 == 0, alignment, 32-bit offsets).
-// Returns -1, having launched nothing, when the shape would split K and the
-// slices' partial sums do not fit the workspace (the caller then takes the
-// integer-limb kernels).
+// Arguments are checked by the entry points (tiled weights, at most 16 MFMA
+// rows, K % 128 == 0, K % group_size == 0, N % 8 == 0, alignment, 32-bit
+// offsets).
 // perm (act-order, may be NULL): x is read as x[:, perm[k]], by the f32
 // pre-pass or, for f16 x, by a gather pass into the workspace.
 int int4_mm_f16(st_context *ctx, const void *x, bool x_f32, const int32_t *perm, const uint32_t *const qw[2],
                 const uint16_t *const sc[2], const uint32_t *const qz[2], int zoff, float *y, int M, int K, int N,
                 int gs, int nsrc) {
+    if (M * (x_f32 ? 2 : 1) > 16) return fail(ST_ERR_SHAPE, "int4_mm_f16: %d tokens", M);
     const int ntiles = (N + kTileN - 1) / kTileN;
     const int maxt = kMaxTilesPerWg / nsrc;  // tiles per workgroup: each tile (and source) keeps >= 2 waves
-    // At most one tile per CU: groups of split_tiles tiles, K split across
-    // workgroups so that the grid fills the CUs (0: one workgroup per tile)
-    const int split_tiles =
-        ntiles <= ctx->num_cus ? std::min(tune(ctx, ST_TUNE_I4MM_SPLIT_TILES, kI4mmSplitTiles), maxt) : 0;
-    int G = std::max(std::min(ctx->num_cus, ntiles), (ntiles + maxt - 1) / maxt);
-    if (split_tiles > 0) G = (ntiles + split_tiles - 1) / split_tiles;
+    const int G = std::max(std::min(ctx->num_cus, ntiles), (ntiles + maxt - 1) / maxt);
     const int tbmax = (ntiles + G - 1) / G;
     int wpt = 2;  // waves per tile and source: a power of two, wpt * nsrc * tbmax <= 16
     while (wpt < 8 && 2 * wpt * nsrc * tbmax <= kWaves) wpt *= 2;
-    if (x_f32 && M > 16) wpt = 2;  // 17-32 tokens of f32 x: 2-unit chunks only
     if (wpt * nsrc * tbmax > kWaves) return fail(ST_ERR_SHAPE, "int4_mm_f16: %d tiles per workgroup", tbmax);
     // 12-wave workgroups when the tiles use at most 12 waves (gate/up with 3
     // tile pairs per workgroup): idle waves would still issue the loop's VALU
@@ -711,8 +635,8 @@ int int4_mm_f16(st_context *ctx, const void *x, bool x_f32, const int32_t *perm,
     // of 12 waves (wpt becomes waves per tile pair: 3 pairs of 4 waves, or
     // 5-6 pairs of 2)
     bool pair = false;
-    if (nsrc == 2 && gs != 64 && !(x_f32 && M > 16) && tune(ctx, ST_TUNE_I4MM_PAIR, 1) != 0 &&
-        tune(ctx, ST_TUNE_I4MM_WAVES, 0) != 16) {  // (not four 16-row blocks: both sources' sums would spill)
+    if (nsrc == 2 && gs != 64 && tune(ctx, ST_TUNE_I4MM_PAIR, 1) != 0 &&
+        tune(ctx, ST_TUNE_I4MM_WAVES, 0) != 16) {
         int wpp = 2;
         while (wpp < 4 && 2 * wpp * tbmax <= 12) wpp *= 2;
         if (wpp * tbmax >= 10 && wpp * tbmax <= 12) {
@@ -726,22 +650,6 @@ int int4_mm_f16(st_context *ctx, const void *x, bool x_f32, const int32_t *perm,
     // f32 x without act-order: split inside the kernel (XM 2); with
     // act-order, or when the setting asks for it, by the pre-pass (XM 1)
     const bool split_in = x_f32 && !perm && tune(ctx, ST_TUNE_I4MM_PREPASS, 0) != 1;
-    // K slices (whole chunks each) and their f32 partials in the workspace,
-    // after what the pre-pass or the gather writes there
-    int ks = 1;
-    float *part = nullptr;
-    if (split_tiles > 0) {
-        const int kcu = pair ? (wpt >= 4 ? 4 : 2) : (wpt >= 8 && gs != 64 ? 8 : (wpt >= 4 ? 4 : 2));
-        const int nch = (K / 128 + kcu - 1) / kcu;
-        ks = std::max(1, std::min({ctx->num_cus / G, kMaxSplit, nch}));
-        if (ks > 1) {
-            const size_t pre = x_f32 && !split_in ? (((size_t)2 * M * K * 2 + 255) & ~size_t(255)) + (size_t)M * (K / 128) * 4
-                                                  : (perm ? (size_t)M * K * 2 : 0);
-            const size_t off = (pre + 255) & ~size_t(255);
-            if (!ctx->ws || off + (size_t)ks * nsrc * M * N * sizeof(float) > ctx->ws_bytes) return -1;  // not taken
-            part = reinterpret_cast<float *>(reinterpret_cast<char *>(ctx->ws) + off);
-        }
-    }
     if (x_f32 && !split_in) {  // the pre-pass writes [2M, K] f16 rows and [M, K / 128] factors into the workspace
         const size_t xbytes = ((size_t)2 * M * K * 2 + 255) & ~size_t(255);
         if (!ctx->ws || xbytes + (size_t)M * (K / 128) * 4 > ctx->ws_bytes)
@@ -762,13 +670,13 @@ int int4_mm_f16(st_context *ctx, const void *x, bool x_f32, const int32_t *perm,
         xa = xg;
     }
     if (split_in)
-        return nsrc == 2 ? launch_src<2, 2>(ctx, xa, pe, qw, sc, qz, zoff, y, M, K, N, gs, ntiles, G, wpt, nw, pair, part, ks)
-                         : launch_src<2, 1>(ctx, xa, pe, qw, sc, qz, zoff, y, M, K, N, gs, ntiles, G, wpt, nw, pair, part, ks);
+        return nsrc == 2 ? launch_src<2, 2>(ctx, xa, pe, qw, sc, qz, zoff, y, M, K, N, gs, ntiles, G, wpt, nw, pair)
+                         : launch_src<2, 1>(ctx, xa, pe, qw, sc, qz, zoff, y, M, K, N, gs, ntiles, G, wpt, nw, pair);
     if (nsrc == 2)
-        return x_f32 ? launch_src<1, 2>(ctx, xa, pe, qw, sc, qz, zoff, y, M, K, N, gs, ntiles, G, wpt, nw, pair, part, ks)
-                     : launch_src<0, 2>(ctx, xa, pe, qw, sc, qz, zoff, y, M, K, N, gs, ntiles, G, wpt, nw, pair, part, ks);
-    return x_f32 ? launch_src<1, 1>(ctx, xa, pe, qw, sc, qz, zoff, y, M, K, N, gs, ntiles, G, wpt, nw, pair, part, ks)
-                 : launch_src<0, 1>(ctx, xa, pe, qw, sc, qz, zoff, y, M, K, N, gs, ntiles, G, wpt, nw, pair, part, ks);
+        return x_f32 ? launch_src<1, 2>(ctx, xa, pe, qw, sc, qz, zoff, y, M, K, N, gs, ntiles, G, wpt, nw, pair)
+                     : launch_src<0, 2>(ctx, xa, pe, qw, sc, qz, zoff, y, M, K, N, gs, ntiles, G, wpt, nw, pair);
+    return x_f32 ? launch_src<1, 1>(ctx, xa, pe, qw, sc, qz, zoff, y, M, K, N, gs, ntiles, G, wpt, nw, pair)
+                 : launch_src<0, 1>(ctx, xa, pe, qw, sc, qz, zoff, y, M, K, N, gs, ntiles, G, wpt, nw, pair);
 }
 
 }  // namespace st

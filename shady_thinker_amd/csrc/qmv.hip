@@ -66,38 +66,54 @@ __global__ __launch_bounds__(256) void repack8_kernel(const int8_t *__restrict__
     reinterpret_cast<uint4 *>(out)[idx] = *reinterpret_cast<const uint4 *>(w + (size_t)n * K + k0);
 }
 
-// The GPTQ entry points take the f16-MFMA kernel (tiled weights, with or
-// without act-order, f32 or f16 x) from kI4mmMinM tokens on when N has more
-// 16-column tiles than the GPU has CUs, and from kI4mmSplitMinM tokens on
-// (groups of tiles, K split across workgroups) when it has fewer. Measured
-// against the integer-limb kernels (kernel durations, MI355X): at 5 tokens
-// configs[4] q|k|v 9.45 -> 7.61 us, gate/up 12.44 -> 9.58, the lm_head
-// 77.3 -> 51.3, Llama-7B gate/up 14.95 -> 11.86; at 4 tokens the lm_head
-// stays on the streaming kernel (39.3 against 50.9 us). On few tiles the
-// limb kernels' fused split-K reduction keeps 5-8 tokens (configs[4] o at 8
-// tokens 9.24 against 10.27 us); at 9-16 tokens the split kernel wins
-// (o 11.8 -> 10.5, down 16.4 -> 12.3, Llama-7B down 21.8 -> 13.7 us).
-constexpr int kI4mmMinM = 5;
-constexpr int kI4mmSplitMinM = 9;
+// The GPTQ entry points take an f16-MFMA kernel (tiled weights, with or
+// without act-order) from a few tokens on. Times (us per call in a graph, cold
+// weights, MI355X; integer-limb kernels against i4xs.hpp):
+//   narrow linears (at most one 16-column tile per CU)
+//     4096 x 4096           4 tokens  6.3 /  7.7   8 tokens  8.8 /  7.7
+//     11008 x 4096                   10.6 / 11.6             13.6 / 12.1
+//     silu(a) b, 4096 x 4096          8.4 /  9.3              9.9 /  9.6
+//     act-order 4096 x 4096          14.4 /  9.7             13.1 /  9.9
+//     act-order 4096 x 4096 2 tokens  7.9 /  9.5
+//   wide: 2560 x 151936     4 tokens 39   / 42     5 tokens 77   / 42
+// so from 5 tokens on, with act-order on narrow linears from 3 (the limb
+// kernels gather x in every workgroup); narrow linears with K below 2048 keep
+// the limb kernels to 8 tokens.
+constexpr int kF16MinM = 5;
+constexpr int kF16MinMActOrder = 3;
+constexpr int kF16MinMShortK = 9;
+constexpr int kF16ShortK = 2048;
 
-// mmax: 16, or 32 for one source (17-32 tokens in one launch, the weights
-// read once; the integer-limb kernels take 16-token blocks)
-bool use_i4mm(const st_context *ctx, const QmvParams &p, bool tiled, int xm, int mmax = 16) {
+// Wide linears whose tokens fill 16 MFMA rows or less (8 tokens of f32 x, 16
+// of f16): i4mm.hip, except for one source of at least 3 tiles per CU (8
+// tokens of f32 x, i4mm / i4xs: 2560 x 10240 7.5 / 8.4 us, gate/up 2560 x
+// 9728 9.8 / 11.8, gate/up 4096 x 11008 13.6 / 14.5; 4096 x 14336 12.9 / 11.3,
+// 2560 x 151936 53.8 / 43.3). Above 16 rows i4xs took every shape measured.
+bool use_i4mm(const st_context *ctx, const QmvParams &p, int ntiles, int nsrc, int xm) {
+    return xm != XM_SILU && ntiles > ctx->num_cus && p.M <= (xm == XM_F32 ? 8 : 16) &&
+           (nsrc == 2 || ntiles < 3 * ctx->num_cus);
+}
+
+// -1: not taken.
+int launch_f16(st_context *ctx, const QmvParams &p, bool tiled, int nsrc, int xm) {
     const int ntiles = (p.N + kTileN - 1) / kTileN;
     const bool few = ntiles <= ctx->num_cus;
-    const int min_m = std::max(2, st::tune(ctx, ST_TUNE_I4MM_MIN_M, few ? kI4mmSplitMinM : kI4mmMinM));
+    const int dflt = !few ? kF16MinM : p.perm ? kF16MinMActOrder : p.K < kF16ShortK ? kF16MinMShortK : kF16MinM;
+    const int min_m = std::max(2, st::tune(ctx, ST_TUNE_I4MM_MIN_M, dflt));
     const int min_tiles = st::tune(ctx, ST_TUNE_I4MM_MIN_TILES, ctx->num_cus + 1);
-    const bool split = few && st::tune(ctx, ST_TUNE_I4MM_SPLIT_TILES, st::kI4mmSplitTiles) > 0;
-    return tiled && (xm == XM_F32 || xm == XM_F16) && p.M <= mmax && p.M >= min_m && (ntiles >= min_tiles || split) &&
-           p.K % 128 == 0 && (size_t)ntiles * kTileN * p.K / 2 < (size_t(1) << 31);
+    const bool split = few && st::tune(ctx, ST_TUNE_I4MM_SPLIT_TILES, 1) > 0;
+    if (!tiled || p.M < min_m || (ntiles < min_tiles && !split) || p.K % 128 ||
+        (size_t)ntiles * kTileN * p.K / 2 >= (size_t(1) << 31) || (size_t)p.M * p.K * 4 >= (size_t(1) << 31))
+        return -1;
+    if (use_i4mm(ctx, p, ntiles, nsrc, xm))
+        return st::int4_mm_f16(ctx, p.x, xm == XM_F32, p.perm, p.qw, p.sc, p.qz, p.zoff, p.y, p.M, p.K, p.N, p.gs, nsrc);
+    const st::XsCall c{p.x, xm == XM_SILU ? p.xb : nullptr, xm == XM_F16, p.perm, {p.qw[0], p.qw[1]}, {p.sc[0], p.sc[1]},
+                       {p.qz[0], p.qz[1]}, p.zoff, p.y, false, p.M, p.K, p.N, p.gs, nsrc};
+    return st::int4_xs(ctx, c);
 }
 
 int launch_i4(st_context *ctx, QmvParams &p, bool tiled, int nsrc, int xm) {
-    if (use_i4mm(ctx, p, tiled, xm)) {
-        const int rc = st::int4_mm_f16(ctx, p.x, xm == XM_F32, p.perm, p.qw, p.sc, p.qz, p.zoff, p.y, p.M, p.K, p.N,
-                                       p.gs, nsrc);
-        if (rc != -1) return rc;  // (-1: the K split's partials do not fit the workspace)
-    }
+    if (const int rc = launch_f16(ctx, p, tiled, nsrc, xm); rc != -1) return rc;
     p.units = p.K / p.gs;
     p.ntiles = (p.N + kTileN - 1) / kTileN;
     // the tiled kernels address the weights with 32-bit buffer offsets
@@ -132,6 +148,14 @@ int by_token_blocks(const st_context *ctx, QmvParams &p, int xm, F &&launch) {
         if (int rc = launch(q)) return rc;
     }
     return ST_OK;
+}
+
+// A GPTQ call of up to 32 tokens: one f16-MFMA launch when it is taken, else
+// blocks of tokens (each of which may still be taken).
+int launch_i4_blocks(st_context *ctx, QmvParams &p, bool tiled, int nsrc, int xm) {
+    if (p.M > kTokenBlock && st::tune(ctx, ST_TUNE_TOKEN_BLOCK, 0) == 0)
+        if (const int rc = launch_f16(ctx, p, tiled, nsrc, xm); rc != -1) return rc;
+    return by_token_blocks(ctx, p, xm, [&](QmvParams &q) { return launch_i4(ctx, q, tiled, nsrc, xm); });
 }
 
 int check_i4(const char *fn, int M, int K, int N, int gs, int mmax) {
@@ -171,14 +195,7 @@ int st_gptq_i4_matvec(st_context *ctx, const void *x, int x_dtype, const uint32_
     p.zoff = (flags & ST_FLAG_ZEROS_PLUS_ONE) ? 1 : 0;
     const bool tiled = flags & ST_FLAG_TILED;
     const int xm = x_dtype == ST_F32 ? XM_F32 : XM_F16;
-    // 17-32 tokens in one f16-MFMA launch when it takes the call (not group
-    // 64 with f32 x: its four 16-row blocks would spill)
-    if (M > kTokenBlock && !(group_size == 64 && xm == XM_F32) && use_i4mm(ctx, p, tiled, xm, 2 * kTokenBlock)) {
-        const int rc = st::int4_mm_f16(ctx, p.x, xm == XM_F32, p.perm, p.qw, p.sc, p.qz, p.zoff, p.y, p.M, p.K, p.N,
-                                       p.gs, 1);
-        if (rc != -1) return rc;  // (-1: the K split's partials do not fit the workspace)
-    }
-    return by_token_blocks(ctx, p, xm, [&](QmvParams &q) { return launch_i4(ctx, q, tiled, 1, xm); });
+    return launch_i4_blocks(ctx, p, tiled, 1, xm);
 }
 
 int st_gptq_i4_matvec_noalloc(st_context *ctx, const void *x, int x_dtype, const uint32_t *qweight,
@@ -227,7 +244,7 @@ int st_gptq_i4_silu_matvec(st_context *ctx, const float *a, const float *b, cons
     p.gs = group_size;
     p.zoff = (flags & ST_FLAG_ZEROS_PLUS_ONE) ? 1 : 0;
     const bool tiled = flags & ST_FLAG_TILED;
-    return by_token_blocks(ctx, p, XM_SILU, [&](QmvParams &q) { return launch_i4(ctx, q, tiled, 1, XM_SILU); });
+    return launch_i4_blocks(ctx, p, tiled, 1, XM_SILU);
 }
 
 int st_gptq_i4_gate_up_silu(st_context *ctx, const void *x, int x_dtype, const uint32_t *qweight_gate,
@@ -261,12 +278,7 @@ int st_gptq_i4_gate_up_silu(st_context *ctx, const void *x, int x_dtype, const u
     p.zoff = (flags & ST_FLAG_ZEROS_PLUS_ONE) ? 1 : 0;
     const bool tiled = flags & ST_FLAG_TILED;
     const int xm = x_dtype == ST_F32 ? XM_F32 : XM_F16;
-    if (M > kTokenBlock && !(group_size == 64 && xm == XM_F32) && use_i4mm(ctx, p, tiled, xm, 2 * kTokenBlock)) {
-        const int rc = st::int4_mm_f16(ctx, p.x, xm == XM_F32, p.perm, p.qw, p.sc, p.qz, p.zoff, p.y, p.M, p.K, p.N,
-                                       p.gs, 2);
-        if (rc != -1) return rc;
-    }
-    return by_token_blocks(ctx, p, xm, [&](QmvParams &q) { return launch_i4(ctx, q, tiled, 2, xm); });
+    return launch_i4_blocks(ctx, p, tiled, 2, xm);
 }
 
 size_t st_gptq_i4_tiled_words(int K, int N, int group_size) {
