@@ -108,7 +108,7 @@ typedef enum {
     ST_TUNE_I4MM_MIN_M,        /* GPTQ decode: fewest tokens for the f16-MFMA kernels (default 5; on at most one tile per CU 3 with act-order, 9 with K below 2048) */
     ST_TUNE_I4MM_MIN_TILES,    /* GPTQ decode: fewest 16-column tiles for the f16-MFMA kernels */
     ST_TUNE_I8MM_MIN_M,        /* INT8 decode: fewest tokens for the f16-MFMA kernel */
-    ST_TUNE_GEMM_CB,           /* prefill GEMM: 32-column blocks per wave (1 or 2); set, the skinny kernel takes no GEMM call */
+    ST_TUNE_GEMM_CB,           /* prefill GEMM: workgroup tile of 128 (1), 256 (2) or 512 (3) columns; set, the skinny kernel takes no GEMM call */
     ST_TUNE_GEMM_NO_SPLIT,     /* 1: prefill GEMM without split-K; set (0 or 1), the skinny kernel takes no GEMM call */
     ST_TUNE_STREAM_WAVES,      /* streaming decode kernel: waves per workgroup (8 or 16) */
     ST_TUNE_STREAM_TILES_WG,   /* streaming decode kernel: 16-column tiles per workgroup (0: a workgroup per CU) */

@@ -20,8 +20,9 @@
 //    buffered one tile ahead. A DMA instruction fills 1 KiB of LDS lane by
 //    lane, so rows are not padded: row r's 16-byte chunk c sits at chunk
 //    c ^ (r % 16), which makes the MFMA fragment reads conflict-free.
-//  * Workgroup tile 128 (M) x 256 (N), 4 waves side by side along N, each
-//    wave 128 x 64 = 4 x 2 MFMA blocks of 32 x 32: every converted B
+//  * Workgroup tile 128 (M) x 512, 256 or 128 (N), 8 or 4 waves side by side
+//    along N, each wave 128 x 64 = 4 x 2 MFMA blocks of 32 x 32 (128 x 32 in
+//    the smallest): every converted B
 //    fragment feeds 4 MFMAs, every A fragment read from LDS feeds 2, and no
 //    B column is converted twice in a workgroup. 128 accumulator registers,
 //    two waves per SIMD; B words and the next k-step's A fragments are read
@@ -53,21 +54,11 @@ typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int BM = 128;              // rows of A per workgroup
-constexpr int BN = 256;              // columns per workgroup
-constexpr int WN = 4;                // waves along N (1 along M)
-constexpr int RB = 4, CB = 2;        // 32 x 32 MFMA blocks per wave (rows, columns)
+constexpr int RB = 4;                // 32 x 32 MFMA blocks per wave along M (along N: CB)
 constexpr int KT = 128;              // k per LDS tile
-constexpr int kThreads = 256;
-#ifndef ST_GEMM_VPM
-#define ST_GEMM_VPM 3  // VALU instructions scheduled after each MFMA
-#endif
-#ifndef ST_GEMM_WAVES
-#define ST_GEMM_WAVES 2
-#endif
-constexpr int kWavesPerSimd = ST_GEMM_WAVES;
+constexpr int kVpm = 3;              // VALU instructions scheduled after each MFMA
 // Buffer resource word 3 for gfx9-class GPUs: raw (untyped) 32-bit data.
 constexpr int kRsrcWord3 = 0x00020000;
-constexpr int kDmaPerWave = BM * KT * 2 / 1024 / (kThreads / 64);  // 1 KiB A DMAs per wave per tile (8)
 
 // v_and_or_b32 with both constants in VGPRs (a VOP3 on gfx9 takes no
 // literal, and at most one SGPR), so the compiler cannot split it in two.
@@ -118,19 +109,20 @@ __device__ __forceinline__ half8 bytes_to_b(unsigned w0, unsigned w1) {
     return __builtin_bit_cast(half8, r);
 }
 
-// CB_ = 32-column MFMA blocks per wave: 2 (workgroup tile 128 x 256) or 1
-// (128 x 128, for grids whose 128 x 256 tiles would leave CUs idle).
+// A workgroup is WN waves side by side along N, CB 32-column MFMA blocks each
+// (workgroup tile 128 x 32 CB WN: 128 x 128, 128 x 256 or 128 x 512).
 // I8: qw is INT8 w (row-major [N, K] or st_int8_repack's tiles), sc / qz /
 // zoff unused, chs the f32 channel scales.
-template <int GS, bool TILED, bool F16OUT, int CB_, bool I8>
-__global__ __launch_bounds__(kThreads, kWavesPerSimd) void gemm_kernel(const _Float16 *__restrict__ A, const uint32_t *__restrict__ qw,
+template <int GS, bool TILED, bool F16OUT, int CB, int WN, bool I8>
+__global__ __launch_bounds__(64 * WN, 2) void gemm_kernel(const _Float16 *__restrict__ A, const uint32_t *__restrict__ qw,
                                                            const uint16_t *__restrict__ sc, const uint32_t *__restrict__ qz,
                                                            int zoff, const float *__restrict__ rsc, const float *__restrict__ chs,
                                                            void *__restrict__ C, int M, int K, int N, int kps,
                                                            float *__restrict__ part, int vec, const uint32_t *qw1,
                                                            const uint16_t *sc1, const uint32_t *qz1, void *C1) {
-    constexpr int CB = CB_;            // (hides the namespace-scope defaults)
     constexpr int BN = 32 * CB * WN;
+    constexpr int kDmaPerWave = BM * KT * 2 / 1024 / WN;  // 1 KiB A DMAs per wave per tile (8 or 4)
+    constexpr int kDmaSteps = I8 ? 2 : 4;                 // k-steps over which they are issued
     // Two separate arrays (not one [2][...]) so that alias analysis can tell
     // the stage being read from the stage the DMA is filling; otherwise every
     // LDS read waits for the in-flight DMA.
@@ -166,8 +158,7 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void gemm_kernel(const _Fl
         C = C1;
     }
     const int m0 = mt * BM, n0 = nt * BN;
-    const int nw = n0 + 32 * CB * (wave % WN);  // this wave's columns
-    const int mw = 32 * RB * (wave / WN);       // and its rows within the tile
+    const int nw = n0 + 32 * CB * wave;  // this wave's columns
 
     int col[CB];
 #pragma unroll
@@ -185,17 +176,18 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void gemm_kernel(const _Fl
     // A DMA j of this wave fills tile rows 4 (8 wave + j) .. +3; lane i
     // writes LDS chunk i % 16 of row + i / 16, i.e. logical chunk
     // (i % 16) ^ (row % 16). Rows past M - 1 repeat row M - 1.
-    auto a_dma = [&](auto STAGE, int kt) {
+    auto a_dma1 = [&](auto STAGE, int kt, int j) {
         _Float16 *as = decltype(STAGE)::value ? As1 : As0;
+        const int r = 4 * (kDmaPerWave * wave + j) + (lane >> 4);
+        const int c = (lane & 15) ^ (r & 15);
+        const int voff = (min(m0 + r, M - 1) * K + 8 * c) * 2;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            ra, (__attribute__((address_space(3))) void *)&as[(4 * (kDmaPerWave * wave + j)) * KT], 16, voff, kt * KT * 2,
+            0, 0);
+    };
+    auto a_dma = [&](auto STAGE, int kt) {
 #pragma unroll
-        for (int j = 0; j < kDmaPerWave; ++j) {
-            const int r = 4 * (kDmaPerWave * wave + j) + (lane >> 4);
-            const int c = (lane & 15) ^ (r & 15);
-            const int voff = (min(m0 + r, M - 1) * K + 8 * c) * 2;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                ra, (__attribute__((address_space(3))) void *)&as[(4 * (kDmaPerWave * wave + j)) * KT], 16, voff,
-                kt * KT * 2, 0, 0);
-        }
+        for (int j = 0; j < kDmaPerWave; ++j) a_dma1(STAGE, kt, j);
     };
     // B words: bw[buffer][t][cb] is the word of k-step t (16 k) for this
     // lane's column block cb; koff(t) is where its 8 k sit in the A tile.
@@ -352,7 +344,6 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void gemm_kernel(const _Fl
         // previous tile's loads are still in flight.
         const int kn = min(kt + 1, kt1 - 1);
         load_groups(BUF ^ 1, kn);
-        a_dma(std::integral_constant<int, BUF ^ 1>{}, kn);  // stage BUF ^ 1 was last read before the previous barrier
         constexpr int RBUF = I8 ? 0 : BUF;                  // the B buffer this tile reads
         if constexpr (!I8) load_b(bw[BUF ^ 1], kn);
         // Keep the prefetch here: left alone, the scheduler sinks these loads
@@ -361,7 +352,7 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void gemm_kernel(const _Fl
         __builtin_amdgcn_sched_barrier(0);
         half8 af[RB];
         auto read_a1 = [&](int t, int rb) {
-            const int row = mw + rb * 32 + l32;
+            const int row = rb * 32 + l32;
             const _Float16 *as = BUF ? As1 : As0;
             af[rb] = *reinterpret_cast<const half8 *>(&as[row * KT + 8 * (kchunk(t) ^ (row & 15))]);
         };
@@ -383,6 +374,18 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void gemm_kernel(const _Fl
 #pragma unroll
         for (int t = 0; t < KT / 16; ++t) {
             const int cur = t & 1;
+            // The next tile's A DMAs, over its first four steps (INT8, whose
+            // weights' loads are spread too: two; stage BUF ^ 1 was last read
+            // before the previous barrier). Issued all at the tile's start,
+            // the waves queued for the address unit (16 loads of 16 cycles
+            // each per wave) before their first MFMA. 256 tiles of 128 x 128
+            // x 2560: 34.3 -> 28.6 us; 304 of 128 x 256: 72 -> 68.
+            if (t < kDmaSteps) {
+                constexpr int n = kDmaPerWave / kDmaSteps;
+#pragma unroll
+                for (int j = 0; j < n; ++j) a_dma1(std::integral_constant<int, BUF ^ 1>{}, kn, n * t + j);
+                __builtin_amdgcn_sched_barrier(0);
+            }
             // INT8: piece (t - 1) / 2 of the next K tile, into the registers
             // its k-steps used here (both converted by step t - 1), pinned at
             // the top of the step: left alone, the scheduler sank these loads
@@ -408,12 +411,13 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void gemm_kernel(const _Fl
                 for (int i = 0; i < RB * CB; ++i) {
                     __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                   // one MFMA
                     if (i % CB == CB - 1) __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // its row block's next A
-                    __builtin_amdgcn_sched_group_barrier(0x002, ST_GEMM_VPM, 0);         // VALU
+                    __builtin_amdgcn_sched_group_barrier(0x002, kVpm, 0);         // VALU
                 }
             }
         }
         // vmcnt(0): the next tile's A DMAs (and GPTQ B words) landed. INT8:
-        // the 4 CB piece loads issued after the DMAs may stay in flight.
+        // the 4 CB piece loads issued after the last DMAs (steps 1, 3, 5 and
+        // 7) may stay in flight.
         __builtin_amdgcn_s_waitcnt(I8 ? 0x0F70 + 4 * CB : 0x0F70);
         __syncthreads();
     };
@@ -429,8 +433,8 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void gemm_kernel(const _Fl
     // its channel scale here. 32 x 32 block: lane l holds column l % 32, rows
     // 8 (i / 4) + 4 (l / 32) + i % 4.
     if (vec) {
-        // Staged through LDS, 32 rows at a time: each wave writes its 32 x 32 CB
-        // block into a region of its own (rows padded by 16 bytes) and reads it
+        // Staged through LDS, SR rows at a time: each wave writes its rows x 32 CB
+        // columns into a region of its own (rows padded by 16 bytes) and reads it
         // back as 16-byte row chunks, so C is written in whole lines (16 stores
         // per lane for f16 C instead of 128 2-byte ones). The A tiles are free:
         // the last K tile ended with a barrier after every wave's last read.
@@ -441,29 +445,31 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void gemm_kernel(const _Fl
             constexpr int PITCH = WC * (int)sizeof(T) + 16;  // bytes per staged row
             constexpr int EPC = 16 / (int)sizeof(T);         // elements per chunk
             constexpr int CPR = WC / EPC;                    // chunks per row
-            static_assert(2 * 32 * PITCH <= (int)sizeof(As0), "staging region");
-            char *stg = reinterpret_cast<char *>((wave & 2) ? As1 : As0) + (wave & 1) * 32 * PITCH;
+            constexpr int SR = WN == 8 && sizeof(T) == 4 ? 16 : 32;  // rows per pass (eight waves' f32 rows: half)
+            static_assert(WN / 2 * SR * PITCH <= (int)sizeof(As0), "staging region");
+            char *stg = reinterpret_cast<char *>((wave & (WN / 2)) ? As1 : As0) + (wave & (WN / 2 - 1)) * SR * PITCH;
             T *dst = part ? reinterpret_cast<T *>(part + (size_t)split * M * N) : static_cast<T *>(C);
             float cs[CB];
 #pragma unroll
             for (int cb = 0; cb < CB; ++cb) cs[cb] = I8 ? chs[min(nw + 32 * cb + l32, N - 1)] : 1.0f;
 #pragma unroll
-            for (int rb = 0; rb < RB; ++rb) {
+            for (int rs = 0; rs < RB * 32 / SR; ++rs) {  // rows SR rs .. of the tile: row block rb, its registers i0 ..
+                const int rb = rs * SR / 32, i0 = rs * SR % 32 / 2;
 #pragma unroll
                 for (int cb = 0; cb < CB; ++cb)
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) {
+                    for (int i = 0; i < SR / 2; ++i) {
                         const int r = 8 * (i >> 2) + 4 * hi + (i & 3);
-                        float v = rsc ? acc[rb][cb][i] * rsc[min(m0 + mw + rb * 32 + r, M - 1)] : acc[rb][cb][i];
+                        float v = rsc ? acc[rb][cb][i0 + i] * rsc[min(m0 + SR * rs + r, M - 1)] : acc[rb][cb][i0 + i];
                         if constexpr (I8) v *= cs[cb];
                         *reinterpret_cast<T *>(stg + r * PITCH + (32 * cb + l32) * (int)sizeof(T)) = (T)v;
                     }
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the wave's block is in LDS
 #pragma unroll
-                for (int q = 0; q < 32 * CPR / 64; ++q) {
+                for (int q = 0; q < SR * CPR / 64; ++q) {
                     const int ch = q * 64 + lane, row = ch / CPR, cc = ch % CPR;
                     const u32x4 v = *reinterpret_cast<const u32x4 *>(stg + row * PITCH + 16 * cc);
-                    const int m = m0 + mw + rb * 32 + row, n = nw + EPC * cc;
+                    const int m = m0 + SR * rs + row, n = nw + EPC * cc;
                     if (m >= M) continue;
                     if (n + EPC <= N) {
                         *reinterpret_cast<u32x4 *>(dst + (size_t)m * N + n) = v;
@@ -491,7 +497,7 @@ __global__ __launch_bounds__(kThreads, kWavesPerSimd) void gemm_kernel(const _Fl
             const float cs = I8 ? chs[n] : 1.0f;
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
-                const int m = m0 + mw + rb * 32 + 8 * (i >> 2) + 4 * hi + (i & 3);
+                const int m = m0 + rb * 32 + 8 * (i >> 2) + 4 * hi + (i & 3);
                 if (m >= M) continue;
                 float v = rsc ? acc[rb][cb][i] * rsc[m] : acc[rb][cb][i];
                 if constexpr (I8) v *= cs;
@@ -591,7 +597,7 @@ __global__ __launch_bounds__(256) void prep_a_kernel(const _Float16 *__restrict_
     }
 }
 
-constexpr int kMaxSplit = 8;  // K splits of a small GEMM grid (plan_split)
+constexpr int kMaxSplit = 8;  // K splits of a small GEMM grid (plan_gemm)
 
 // C[m, n] = sum over s < S of part[s, m, n] (fixed order: deterministic).
 template <bool F16OUT>
@@ -656,24 +662,31 @@ int vec_ok(const GemmArgs &g, const Split &sp) {
     return st::aligned16(g.C) && (!g.C1 || st::aligned16(g.C1)) && g.N % (g.f16out ? 8 : 4) == 0;
 }
 
-template <int GS, bool TILED, int CBL, bool I8>
-int launch_cb(st_context *ctx, const GemmArgs &g, const Split &sp) {
-    const int T = ((g.M + BM - 1) / BM) * ((g.N + 32 * CBL * WN - 1) / (32 * CBL * WN)) * (g.C1 ? 2 : 1);
-    const dim3 grid(T * sp.S);
+// Workgroup tiles: columns of one workgroup.
+enum Tile { kTile128 = 0, kTile256 = 1, kTile512 = 2 };
+constexpr int tile_columns(int tile) { return 128 << tile; }
+int tile_count(int M, int N, int tile) {
+    return ((M + BM - 1) / BM) * ((N + tile_columns(tile) - 1) / tile_columns(tile));
+}
+
+template <int GS, bool TILED, int CB, int WN, bool I8>
+int launch_cb(st_context *ctx, const GemmArgs &g, const Split &sp, int T) {
+    const dim3 grid(T * sp.S), block(64 * WN);
     if (g.f16out)
-        st::launch(ctx, (gemm_kernel<GS, TILED, true, CBL, I8>), grid, dim3(kThreads), 0, g.A, g.qw, g.sc,
-                           g.qz, g.zoff, g.rsc, g.chs, g.C, g.M, g.K, g.N, sp.kps, sp.part, vec_ok(g, sp), g.qw1, g.sc1,
-                           g.qz1, g.C1);
+        st::launch(ctx, (gemm_kernel<GS, TILED, true, CB, WN, I8>), grid, block, 0, g.A, g.qw, g.sc, g.qz, g.zoff, g.rsc, g.chs,
+                   g.C, g.M, g.K, g.N, sp.kps, sp.part, vec_ok(g, sp), g.qw1, g.sc1, g.qz1, g.C1);
     else
-        st::launch(ctx, (gemm_kernel<GS, TILED, false, CBL, I8>), grid, dim3(kThreads), 0, g.A, g.qw, g.sc,
-                           g.qz, g.zoff, g.rsc, g.chs, g.C, g.M, g.K, g.N, sp.kps, sp.part, vec_ok(g, sp), g.qw1, g.sc1,
-                           g.qz1, g.C1);
+        st::launch(ctx, (gemm_kernel<GS, TILED, false, CB, WN, I8>), grid, block, 0, g.A, g.qw, g.sc, g.qz, g.zoff, g.rsc, g.chs,
+                   g.C, g.M, g.K, g.N, sp.kps, sp.part, vec_ok(g, sp), g.qw1, g.sc1, g.qz1, g.C1);
     return st::launch_check("gemm_kernel");
 }
 
 template <int GS, bool TILED, bool I8 = false>
-int launch_gs(st_context *ctx, const GemmArgs &g, int cb, const Split &sp) {
-    const int rc = cb == 1 ? launch_cb<GS, TILED, 1, I8>(ctx, g, sp) : launch_cb<GS, TILED, 2, I8>(ctx, g, sp);
+int launch_gs(st_context *ctx, const GemmArgs &g, int tile, const Split &sp) {
+    const int T = tile_count(g.M, g.N, tile) * (g.C1 ? 2 : 1);
+    const int rc = tile == kTile128   ? launch_cb<GS, TILED, 1, 4, I8>(ctx, g, sp, T)
+                   : tile == kTile256 ? launch_cb<GS, TILED, 2, 4, I8>(ctx, g, sp, T)
+                                      : launch_cb<GS, TILED, 2, 8, I8>(ctx, g, sp, T);
     if (rc) return rc;
     const int M = g.M, N = g.N;
     const bool f16out = g.f16out;
@@ -691,50 +704,73 @@ int launch_gs(st_context *ctx, const GemmArgs &g, int cb, const Split &sp) {
 }
 
 template <bool TILED>
-int launch_tiled(st_context *ctx, const GemmArgs &g, int gs, int cb, const Split &sp) {
+int launch_tiled(st_context *ctx, const GemmArgs &g, int gs, int tile, const Split &sp) {
     switch (gs) {
-        case 64: return launch_gs<64, TILED>(ctx, g, cb, sp);
-        case 128: return launch_gs<128, TILED>(ctx, g, cb, sp);
-        default: return launch_gs<256, TILED>(ctx, g, cb, sp);
+        case 64: return launch_gs<64, TILED>(ctx, g, tile, sp);
+        case 128: return launch_gs<128, TILED>(ctx, g, tile, sp);
+        default: return launch_gs<256, TILED>(ctx, g, tile, sp);
     }
 }
 
-// 32-column blocks per wave: 1 (128 x 128 tiles) when 128 x 256 tiles would
-// give at most one workgroup per CU (then two waves per SIMD instead of
-// one); ST_TUNE_GEMM_CB forces 1 or 2. INT8 keeps the wide tiles down to
-// half a workgroup per CU (configs[2]'s weight: M = 512, 216 wide tiles,
-// 85 -> 76-78 us; M = 384, 162 tiles, 72-74 -> 69 us; at M = 256, 108
-// tiles, the narrow ones win).
-int pick_cb(st_context *ctx, int M, int N, bool i8) {
-    const int f = st::tune(ctx, ST_TUNE_GEMM_CB, 0);
-    if (f == 1 || f == 2) return f;
-    const int T2 = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
-    if (i8) return 2 * T2 >= ctx->num_cus ? 2 : 1;
-    return T2 <= ctx->num_cus ? 1 : 2;
+// Time (us) of one 128-k step of n workgroup tiles that run at once, from
+// sweeps of 200-2048 rows on weights of 2048 x 2560 to 2560 x 19456 (MI355X).
+// Up to a tile per CU its own pipeline bounds it (more CUs at work lower the
+// clock a little); beyond, two share a CU, and from about 1.1 PFLOP/s on the
+// chip as a whole does.
+double step_us(bool i8, int tile, int n, int ncu) {
+    switch (tile) {
+        case kTile128:
+            if (n <= ncu) return i8 ? 0.8 + 0.0012 * n : 0.85 + 0.0017 * n;
+            return std::max(1.85, (i8 ? 0.0037 : 0.0039) * n);
+        case kTile256:
+            if (n <= ncu) return i8 ? 1.15 + 0.0025 * n : 1.5 + 0.0024 * n;
+            return std::max(i8 ? 3.2 : 3.25, (i8 ? 0.0075 : 0.008) * n);
+        default: return std::max(i8 ? 2.2 : 2.35, (i8 ? 0.0139 : 0.0152) * n);
+    }
 }
 
-// Split K when the tiles alone fill at most half the CUs (the f32 partials
-// cost S * M * N * 8 bytes of extra traffic, which measured a loss at
-// configs[3] M = 512, 224 tiles): S splits of an even number of K tiles
-// each, as many as fill the workgroup slots (two per CU), at most 8, each at
-// least 4 K tiles, within the workspace left after A'.
-Split plan_split(st_context *ctx, int M, int K, int N, int cb, size_t ws_used) {
-    Split sp{1, K / KT, nullptr};
-    const int T = ((M + BM - 1) / BM) * ((N + 32 * cb * WN - 1) / (32 * cb * WN));
-    const int slots = 2 * ctx->num_cus;
-    const int ntiles = K / KT;
-    if (2 * T > ctx->num_cus || ntiles < 8 || st::tune(ctx, ST_TUNE_GEMM_NO_SPLIT, 0)) return sp;
-    int S = std::min({kMaxSplit, (slots + T - 1) / T, ntiles / 4});
+struct GemmPlan {
+    int tile;
+    Split sp;
+};
+
+// The workgroup tile and the K splits with the least estimated time: rounds of
+// as many tiles as fit the chip (two 128- or 256-column workgroups per CU, one
+// of 512), the last one smaller; a split adds its reduction, S f32 partials
+// of C written and read. At most kMaxSplit splits of an even number of at
+// least 4 K tiles, within the workspace left after A'. GEMM_CB forces the tile
+// (1, 2, 3), GEMM_NO_SPLIT = 1 no split.
+// Before (128 columns up to a 256-column tile per CU, then 256; splits
+// whenever tiles filled half the CUs or less) and now, us with the pre-pass:
+// 512 rows 2560 x 19456 72 -> 60, 768 rows 83 -> 77, 1024 rows 4096 x 14336
+// 122 -> 114, 2048 rows 237 -> 225, 512 rows 2048 x 2560 25 -> 20.
+GemmPlan plan_gemm(st_context *ctx, bool i8, int M, int K, int N, size_t ws_used, bool split = true) {
+    const int ncu = ctx->num_cus, ntiles = K / KT;
+    const int force = st::tune(ctx, ST_TUNE_GEMM_CB, 0);
+    const int smax = !split || st::tune(ctx, ST_TUNE_GEMM_NO_SPLIT, 0) == 1 ? 1 : std::min(kMaxSplit, ntiles / 4);
     const size_t off = (ws_used + 255) & ~size_t(255);
-    while (S > 1 && off + (size_t)S * M * N * sizeof(float) > ctx->ws_bytes) --S;
-    if (S <= 1) return sp;
-    int kps = (ntiles + S - 1) / S;
-    kps += kps & 1;
-    sp.S = (ntiles + kps - 1) / kps;
-    sp.kps = kps;
-    sp.part = sp.S > 1 ? reinterpret_cast<float *>(reinterpret_cast<char *>(ctx->ws) + off) : nullptr;
-    if (sp.S == 1) sp.kps = ntiles;
-    return sp;
+    GemmPlan best{kTile128, {1, ntiles, nullptr}};
+    double least = 1e30;
+    for (int tile = kTile128; tile <= kTile512; ++tile) {
+        if (force >= 1 && force <= 3 && tile != force - 1) continue;
+        const int T = tile_count(M, N, tile), slots = tile == kTile512 ? ncu : 2 * ncu;
+        for (int s = 1; s <= std::max(1, smax); ++s) {
+            if (s > 1 && off + (size_t)s * M * N * sizeof(float) > ctx->ws_bytes) break;
+            int kps = (ntiles + s - 1) / s;
+            if (s > 1) kps += kps & 1;
+            const int S = (ntiles + kps - 1) / kps;
+            if (S != s) continue;
+            const long long n = (long long)T * S;
+            double us = kps * ((n / slots) * step_us(i8, tile, slots, ncu) + (n % slots ? step_us(i8, tile, (int)(n % slots), ncu) : 0.0));
+            if (S > 1) us += 3.0 + 2e-6 * S * M * N;
+            if (us < least) {
+                least = us;
+                best.tile = tile;
+                best.sp = Split{S, kps, S > 1 ? reinterpret_cast<float *>(reinterpret_cast<char *>(ctx->ws) + off) : nullptr};
+            }
+        }
+    }
+    return best;
 }
 
 }  // namespace
@@ -809,36 +845,32 @@ int gemm_impl(const char *fn, st_context *ctx, const uint16_t *a, const uint16_t
     if (int rc = st::launch_check("prep_a_kernel")) return rc;
     GemmArgs g{A, qweight, scales, qzeros, (flags & ST_FLAG_ZEROS_PLUS_ONE) ? 1 : 0, rsc, nullptr, c,
                c_dtype == ST_F16, M, K, N};
-    auto run = [&](const GemmArgs &ga, int cb, const Split &sp) {
-        return (flags & ST_FLAG_TILED) ? launch_tiled<true>(ctx, ga, group_size, cb, sp)
-                                       : launch_tiled<false>(ctx, ga, group_size, cb, sp);
+    auto run = [&](const GemmArgs &ga, int tile, const Split &sp) {
+        return (flags & ST_FLAG_TILED) ? launch_tiled<true>(ctx, ga, group_size, tile, sp)
+                                       : launch_tiled<false>(ctx, ga, group_size, tile, sp);
     };
-    const int cb = pick_cb(ctx, M, N, false);
-    const Split sp = plan_split(ctx, M, K, N, cb, need);
-    if (w1) {
-        // Both weights' tiles in one grid when neither that grid nor one
-        // weight's alone splits K (the partials are laid out for one C, and
-        // a split changes the order of the f32 sums, so the results would no
-        // longer be those of st_gptq_i4_gemm); otherwise two launches on A.
-        const int cb2 = pick_cb(ctx, M, 2 * N, false);
-        const Split sp2 = plan_split(ctx, M, K, 2 * N, cb2, need);
-        if (sp2.S == 1 && sp.S == 1) {
-            GemmArgs g2 = g;
-            g2.qw1 = w1->qweight;
-            g2.sc1 = w1->scales;
-            g2.qz1 = w1->qzeros;
-            g2.C1 = w1->c;
-            return run(g2, cb2, sp2);
-        }
+    const GemmPlan pl = plan_gemm(ctx, false, M, K, N, need);
+    // Both weights' tiles in one grid when one weight's alone does not split
+    // K (the partials are laid out for one C, and a split changes the order
+    // of the f32 sums, so the results would no longer be those of
+    // st_gptq_i4_gemm); otherwise two launches on A.
+    if (w1 && pl.sp.S == 1) {
+        const GemmPlan pl2 = plan_gemm(ctx, false, M, K, 2 * N, need, false);
+        GemmArgs g2 = g;
+        g2.qw1 = w1->qweight;
+        g2.sc1 = w1->scales;
+        g2.qz1 = w1->qzeros;
+        g2.C1 = w1->c;
+        return run(g2, pl2.tile, pl2.sp);
     }
-    if (int rc = run(g, cb, sp)) return rc;
+    if (int rc = run(g, pl.tile, pl.sp)) return rc;
     if (!w1) return ST_OK;
     GemmArgs g1 = g;
     g1.qw = w1->qweight;
     g1.sc = w1->scales;
     g1.qz = w1->qzeros;
     g1.C = w1->c;
-    return run(g1, cb, sp);
+    return run(g1, pl.tile, pl.sp);
 }
 
 }  // namespace
@@ -882,7 +914,6 @@ extern "C" int st_int8_gemm(st_context *ctx, const uint16_t *a, const int8_t *w,
         return st::fail(ST_ERR_SHAPE, "%s: a or w above 2 GiB (M=%d K=%d N=%d); split M or N", fn, M, K, N);
     const GemmArgs g{reinterpret_cast<const _Float16 *>(a), reinterpret_cast<const uint32_t *>(w), nullptr, nullptr, 0,
                      nullptr, scale, c, c_dtype == ST_F16, M, K, N};
-    const int cb = pick_cb(ctx, M, N, true);
-    const Split sp = plan_split(ctx, M, K, N, cb, 0);
-    return tiled ? launch_gs<128, true, true>(ctx, g, cb, sp) : launch_gs<128, false, true>(ctx, g, cb, sp);
+    const GemmPlan pl = plan_gemm(ctx, true, M, K, N, 0);
+    return tiled ? launch_gs<128, true, true>(ctx, g, pl.tile, pl.sp) : launch_gs<128, false, true>(ctx, g, pl.tile, pl.sp);
 }
