@@ -88,10 +88,16 @@ constexpr int kF16ShortK = 2048;
 // of f16): i4mm.hip, except for one source of at least 3 tiles per CU (8
 // tokens of f32 x, i4mm / i4xs: 2560 x 10240 7.5 / 8.4 us, gate/up 2560 x
 // 9728 9.8 / 11.8, gate/up 4096 x 11008 13.6 / 14.5; 4096 x 14336 12.9 / 11.3,
-// 2560 x 151936 53.8 / 43.3). Above 16 rows i4xs took every shape measured.
+// 2560 x 151936 53.8 / 43.3), and of at most 2 in groups of 64 with f32 x,
+// where i4mm's 8-byte weight loads hold too little in flight (6 tokens: 1024 x
+// 6144 5.5 / 5.2, 4096 x 4160 11.7 / 8.9, 4096 x 8000 12.0 / 10.2, 8192 x 6144
+// 19.8 / 12.4, 4096 x 6144 with zeros and act-order 14.8 / 12.4; at 2.5 tiles
+// per CU 4096 x 10240 10.5 / 11.6; f16 x, 4096 x 6144, 11.4 / 15.0; group 128,
+// 4096 x 6144, 8.0 / 9.2). Above 16 rows i4xs took every shape measured.
 bool use_i4mm(const st_context *ctx, const QmvParams &p, int ntiles, int nsrc, int xm) {
-    return xm != XM_SILU && ntiles > ctx->num_cus && p.M <= (xm == XM_F32 ? 8 : 16) &&
-           (nsrc == 2 || ntiles < 3 * ctx->num_cus);
+    if (xm == XM_SILU || ntiles <= ctx->num_cus || p.M > (xm == XM_F32 ? 8 : 16)) return false;
+    if (nsrc == 2) return true;
+    return ntiles < 3 * ctx->num_cus && !(xm == XM_F32 && p.gs == 64 && ntiles <= 2 * ctx->num_cus);
 }
 
 // -1: not taken.

@@ -45,6 +45,8 @@ def _ref(orc, c, x, K, N, gs, act):
     (3, 3072, 1032, 128, True, True, False),     # act-order: fewest tokens
     (24, 4096, 4104, 64, True, True, False),     # act-order, group 64, 257 tiles
     (7, 2560, 13000, 128, False, False, False),  # one source of more than 3 tiles per CU
+    (8, 1024, 8192, 64, True, True, False),      # group 64, two tiles per CU: the last of its rule
+    (5, 3072, 8200, 64, False, False, False),    # one tile more
     (20, 1024, 4112, 128, True, False, True),    # f16 x, one token block
     (32, 6144, 776, 64, True, True, True),       # f16 x gathered
 ])
