@@ -19,7 +19,7 @@ LIB = os.path.join(HERE, "libshady_hip.so")
 SOURCES = [
     "runtime.hip", "qmv.hip", "qmv_i4_p0.hip", "qmv_i4_p1.hip", "qmv_i4t_p0.hip", "qmv_i4t_p1.hip", "qmv_i8.hip", "qmv_i8t.hip",
     "i8mm.hip", "i4mm.hip", "i4xs.hip", "i4xs_f32.hip", "i4xs_f32d.hip", "i4xs_f32s.hip", "i4xs_f16.hip", "i4xs_f16d.hip",
-    "i4xs_f16s.hip", "i4xs_f16g.hip", "dequant.hip", "gemm.hip", "bf16mv.hip",
+    "i4xs_f16g.hip", "dequant.hip", "gemm.hip", "bf16mv.hip",
 ]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

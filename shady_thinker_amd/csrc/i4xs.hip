@@ -1,19 +1,19 @@
 // Host side of the skinny GPTQ kernel (i4xs.hpp): how a call is split over
-// workgroups, the act-order gather and the reduction of K slices.
+// workgroups, the pre-passes (act-order gather, f16 silu(a) * b) and the
+// reduction of K slices.
 #include "i4xs.hpp"
 
 #include <algorithm>
 
 namespace st {
 namespace xs {
-// instantiated in i4xs_{f32,f32d,f32s,f16,f16d,f16s,f16g}.hip
+// instantiated in i4xs_{f32,f32d,f32s,f16,f16d,f16g}.hip
 extern template int launch<X_F32, 1>(st_context *, const Args &, int, int, bool);
 extern template int launch<X_F32, 2>(st_context *, const Args &, int, int, bool);
 extern template int launch<X_F32_SILU, 1>(st_context *, const Args &, int, int, bool);
 extern template int launch<X_F16, 1>(st_context *, const Args &, int, int, bool);
 extern template int launch<X_F16, 2>(st_context *, const Args &, int, int, bool);
 extern template int launch<X_F16G, 1>(st_context *, const Args &, int, int, bool);
-extern template int launch<X_F16_SILU, 1>(st_context *, const Args &, int, int, bool);
 }  // namespace xs
 }  // namespace st
 
@@ -25,7 +25,7 @@ using namespace st::xs;
 // order (deterministic), the epilogue silu(gate) * up for two sources.
 template <int NSRC, bool F16OUT>
 __global__ __launch_bounds__(256) void i4xs_reduce_kernel(const float *__restrict__ part, void *__restrict__ y, int MN,
-                                                          int ks) {
+                                                          int ks, const float *__restrict__ rsc, int N) {
     const int idx = blockIdx.x * 256 + threadIdx.x;
     if (idx >= MN) return;
     float t[kMaxSplit][NSRC];  // every slice's load issued before the first add
@@ -41,7 +41,7 @@ __global__ __launch_bounds__(256) void i4xs_reduce_kernel(const float *__restric
         for (int s = 0; s < kMaxSplit; ++s)
             if (s < ks) v[sr] += t[s][sr];
     }
-    const float r = NSRC == 2 ? silu_f(v[0]) * v[NSRC - 1] : v[0];
+    const float r = NSRC == 2 ? silu_f(v[0]) * v[NSRC - 1] : rsc ? v[0] * rsc[idx / N] : v[0];
     if (F16OUT)
         static_cast<_Float16 *>(y)[idx] = (_Float16)r;
     else
@@ -70,6 +70,70 @@ __global__ __launch_bounds__(256) void i4xs_gather_kernel(const T *__restrict__ 
     __builtin_memcpy(xg + i, v, sizeof v);
 }
 
+// f16 silu(a) * b of a short prompt, once for all workgroups: row t's products
+// (of k = perm[.] under act-order) times 2^-e rounded to f16, 2^e just above
+// 2^-15 of the largest finite one, rsc[t] = 2^e. In the skinny kernel itself,
+// which formed them before, every workgroup did so again for its K slice, and
+// two inputs held its waves to two units (more slices). us per call, before /
+// now: 77 tokens 9728 x 2560 29.1 / 26.4, 4096 x 2560 22.6 / 15.3; 160 tokens
+// 11008 x 4096 51.9 / 43.6; with act-order (the GEMM before) 33 tokens 9728 x
+// 2560 31.9 / 25.0. All of a row's loads are in flight at once: a block of 256
+// threads in several passes took 8.0 us at 77 tokens, this 5.8.
+constexpr int kSiluThreads = 1024;
+__global__ __launch_bounds__(kSiluThreads) void i4xs_silu_kernel(const _Float16 *__restrict__ a, const _Float16 *__restrict__ b,
+                                                                 const int32_t *__restrict__ perm, _Float16 *__restrict__ out,
+                                                                 float *__restrict__ rsc, int K) {
+    constexpr int P = 4;  // chunks of 8 k per thread: K <= 32768
+    __shared__ float wmax[kSiluThreads / 64];
+    const size_t base = (size_t)blockIdx.x * K;
+    half8 g[P], u[P];
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        const int k = (p * kSiluThreads + (int)threadIdx.x) * 8;
+        g[p] = u[p] = half8{};
+        if (k >= K) continue;
+        if (perm) {
+            const int4 p0 = *reinterpret_cast<const int4 *>(perm + k), p1 = *reinterpret_cast<const int4 *>(perm + k + 4);
+            const int pk[8] = {p0.x, p0.y, p0.z, p0.w, p1.x, p1.y, p1.z, p1.w};
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                g[p][e] = a[base + pk[e]];
+                u[p][e] = b[base + pk[e]];
+            }
+        } else {
+            g[p] = *reinterpret_cast<const half8 *>(a + base + k);
+            u[p] = *reinterpret_cast<const half8 *>(b + base + k);
+        }
+    }
+    float m = 0.f, h[P][8];
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        if (p * kSiluThreads * 8 >= K) break;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            h[p][e] = silu_f((float)g[p][e]) * (float)u[p][e];
+            m = fabsf(h[p][e]) <= 3.402823466e38f ? fmaxf(m, fabsf(h[p][e])) : m;
+        }
+    }
+    for (int d = 32; d; d >>= 1) m = fmaxf(m, __shfl_xor(m, d));
+    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kSiluThreads / 64; ++w) m = fmaxf(m, wmax[w]);
+    const int ex = max(__builtin_amdgcn_frexp_expf(m), -100) - 15;
+    const float up = __builtin_amdgcn_ldexpf(1.0f, -ex);
+    if (threadIdx.x == 0) rsc[blockIdx.x] = __builtin_amdgcn_ldexpf(1.0f, ex);
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+        const int k = (p * kSiluThreads + (int)threadIdx.x) * 8;
+        if (k >= K) break;
+        half8 o;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = (_Float16)(h[p][e] * up);
+        *reinterpret_cast<half8 *>(out + base + k) = o;
+    }
+}
+
 struct Split {
     int ks = 0, groups = 0;  // ks = 0: no split fits
 };
@@ -82,7 +146,7 @@ struct Split {
 Split plan(const st_context *ctx, int xm, int M, int K, int N, int nsrc, size_t ws) {
     const int units = K / 128, ntiles = (N + kTileN - 1) / kTileN;
     const int tb = (M + block_tokens(xm) - 1) / block_tokens(xm);
-    const bool half = is_half(xm), silu = xm == X_F32_SILU || xm == X_F16_SILU;
+    const bool half = is_half(xm), silu = xm == X_F32_SILU;
     const int umax = silu ? 2 : kMaxUnits;
     const double x_us = half ? 0.4 : 0.8, tile_us = half ? 0.25 : 0.22;
     Split best;
@@ -111,24 +175,31 @@ namespace st {
 
 int int4_xs(st_context *ctx, const XsCall &c) {
     const bool half = c.x_f16, silu = c.xb != nullptr;
-    int xm = half ? (silu ? X_F16_SILU : c.round_w ? X_F16G : X_F16) : (silu ? X_F32_SILU : X_F32);
-    // act-order: x (or silu(x) * xb, f32 only) gathered into the workspace first
-    size_t off = 0;
-    if (c.perm) {
-        if (half && silu) return -1;
-        off = ((size_t)c.M * c.K * (half ? 2 : 4) + 255) & ~size_t(255);
+    // (f16 silu(a) * b: exact weights, so that only the product is rounded)
+    int xm = half ? (c.round_w && !silu ? X_F16G : X_F16) : (silu ? X_F32_SILU : X_F32);
+    // act-order, and f16 silu(x) * xb: x (or the product) goes to the workspace first
+    const bool pre = c.perm || (half && silu);
+    size_t off = 0, rsc_off = 0;
+    if (pre) {
+        rsc_off = off = ((size_t)c.M * c.K * (half ? 2 : 4) + 255) & ~size_t(255);
+        if (half && silu) off = (off + (size_t)c.M * sizeof(float) + 255) & ~size_t(255);
         if (!ctx->ws || off > ctx->ws_bytes) return -1;
-        if (silu) xm = X_F32;
+        if (silu && !half) xm = X_F32;
     }
     const Split sp = plan(ctx, xm, c.M, c.K, c.N, c.nsrc, ctx->ws ? ctx->ws_bytes - off : 0);
     if (!sp.ks) return -1;
     Args a{};
     a.x = c.x;
     a.xb = c.xb;
-    if (c.perm) {
+    if (pre) {
         void *xg = ctx->ws;
         const dim3 g((unsigned)(((size_t)c.M * c.K / 4 + 255) / 256)), b(256);
-        if (half)
+        if (half && silu) {
+            float *const rsc = reinterpret_cast<float *>(reinterpret_cast<char *>(ctx->ws) + rsc_off);
+            st::launch(ctx, i4xs_silu_kernel, dim3(c.M), dim3(kSiluThreads), 0, static_cast<const _Float16 *>(c.x),
+                       static_cast<const _Float16 *>(c.xb), c.perm, static_cast<_Float16 *>(xg), rsc, c.K);
+            a.rsc = rsc;
+        } else if (half)
             st::launch(ctx, i4xs_gather_kernel<uint16_t, false>, g, b, 0, static_cast<const uint16_t *>(c.x),
                        static_cast<const uint16_t *>(nullptr), c.perm, static_cast<uint16_t *>(xg), c.M, c.K);
         else if (silu)
@@ -137,7 +208,7 @@ int int4_xs(st_context *ctx, const XsCall &c) {
         else
             st::launch(ctx, i4xs_gather_kernel<float, false>, g, b, 0, static_cast<const float *>(c.x),
                        static_cast<const float *>(nullptr), c.perm, static_cast<float *>(xg), c.M, c.K);
-        if (int rc = launch_check("i4xs_gather_kernel")) return rc;
+        if (int rc = launch_check("i4xs pre-pass")) return rc;
         a.x = xg;
         a.xb = nullptr;
     }
@@ -167,18 +238,17 @@ int int4_xs(st_context *ctx, const XsCall &c) {
         case X_F32: rc = c.nsrc == 2 ? xs::launch<X_F32, 2>(ctx, a, c.gs, sp.groups, hz) : xs::launch<X_F32, 1>(ctx, a, c.gs, sp.groups, hz); break;
         case X_F16: rc = c.nsrc == 2 ? xs::launch<X_F16, 2>(ctx, a, c.gs, sp.groups, hz) : xs::launch<X_F16, 1>(ctx, a, c.gs, sp.groups, hz); break;
         case X_F16G: rc = xs::launch<X_F16G, 1>(ctx, a, c.gs, sp.groups, hz); break;
-        case X_F32_SILU: rc = xs::launch<X_F32_SILU, 1>(ctx, a, c.gs, sp.groups, hz); break;
-        default: rc = xs::launch<X_F16_SILU, 1>(ctx, a, c.gs, sp.groups, hz); break;
+        default: rc = xs::launch<X_F32_SILU, 1>(ctx, a, c.gs, sp.groups, hz); break;
     }
     if (rc || sp.ks == 1) return rc;
     const int mn = c.M * c.N;
     const dim3 g((mn + 255) / 256), b(256);
     if (c.nsrc == 2)
-        c.y_f16 ? st::launch(ctx, i4xs_reduce_kernel<2, true>, g, b, 0, a.part, a.y, mn, sp.ks)
-                : st::launch(ctx, i4xs_reduce_kernel<2, false>, g, b, 0, a.part, a.y, mn, sp.ks);
+        c.y_f16 ? st::launch(ctx, i4xs_reduce_kernel<2, true>, g, b, 0, a.part, a.y, mn, sp.ks, a.rsc, c.N)
+                : st::launch(ctx, i4xs_reduce_kernel<2, false>, g, b, 0, a.part, a.y, mn, sp.ks, a.rsc, c.N);
     else
-        c.y_f16 ? st::launch(ctx, i4xs_reduce_kernel<1, true>, g, b, 0, a.part, a.y, mn, sp.ks)
-                : st::launch(ctx, i4xs_reduce_kernel<1, false>, g, b, 0, a.part, a.y, mn, sp.ks);
+        c.y_f16 ? st::launch(ctx, i4xs_reduce_kernel<1, true>, g, b, 0, a.part, a.y, mn, sp.ks, a.rsc, c.N)
+                : st::launch(ctx, i4xs_reduce_kernel<1, false>, g, b, 0, a.part, a.y, mn, sp.ks, a.rsc, c.N);
     return launch_check("i4xs_reduce_kernel");
 }
 

@@ -1,7 +1,8 @@
 // Skinny GPTQ int4 GEMM with x held in registers (gfx950): a few to a few
 // dozen tokens against tiled weights (st_gptq_i4_repack),
 //   y[m, n]  = sum_g s[g, n] * sum_{k in g} (q[k, n] - z[g, n]) * x[m, k]
-// or silu(gate) * up of two such sums, x as f32, f16 or silu(a) * b of either
+// or silu(gate) * up of two such sums, x as f32, f16 or f32 silu(a) * b (f16:
+// a pre-pass)
 // (semantics of gptq_matvec.wgsl:51-58, fused_gate_up_silu_4t.wgsl:24-90 and
 // fused_silu_gptq_4t.wgsl:26-81; the reference runs one token at a time).
 //
@@ -44,9 +45,9 @@ constexpr unsigned kNoLoad = 0x80000000u;  // buffer offset past every resource:
 
 // X_F16G: f16 x against (q - z) s rounded once to f16 (the prefill GEMM's
 // weights) instead of exact (q - z), s applied to the sums.
-enum { X_F16 = 0, X_F32 = 1, X_F32_SILU = 2, X_F16_SILU = 3, X_F16G = 4 };
+enum { X_F16 = 0, X_F32 = 1, X_F32_SILU = 2, X_F16G = 3 };
 
-constexpr bool is_half(int xm) { return xm == X_F16 || xm == X_F16G || xm == X_F16_SILU; }  // one f16 value per x
+constexpr bool is_half(int xm) { return xm == X_F16 || xm == X_F16G; }  // one f16 value per x
 
 constexpr int kWaves = 8;                   // waves per workgroup
 constexpr int kMaxUnits = 4;                // 128-k units per wave
@@ -59,6 +60,7 @@ struct Args {
     const uint32_t *qz[2];
     void *y;
     float *part;  // K slices' partial sums (ks > 1)
+    const float *rsc;  // or nullptr: factor of each token's y (one source)
     int zoff, M, K, N, tq, trem, uq, urem, ks, tblocks, f16out;  // tq, trem: tiles / runs; uq, urem: 128-k units / K slices
 };
 
@@ -137,8 +139,8 @@ template <int XM, int NSRC, int GS, int U, int R, bool HZ>
 __global__ __launch_bounds__(64 * kWaves) void i4xs_kernel(Args a) {
     constexpr bool HALF = is_half(XM);  // one f16 value per x, two 16-row blocks
     constexpr bool ROUND = XM == X_F16G;
-    constexpr bool SILU = XM == X_F32_SILU || XM == X_F16_SILU;
-    constexpr bool SCALED = !HALF || SILU;  // x scaled by 2^(15 - ex) per token and wave
+    constexpr bool SILU = XM == X_F32_SILU;
+    constexpr bool SCALED = !HALF;  // x scaled by 2^(15 - ex) per token and wave
     constexpr int MB = HALF ? 2 : 1;      // 16-row blocks
     constexpr int TPB = 16 * MB;          // tokens per workgroup
     constexpr int NG = GS == 64 ? 2 : 1;  // groups per 128-k unit
@@ -289,30 +291,18 @@ __global__ __launch_bounds__(64 * kWaves) void i4xs_kernel(Args a) {
             float m = 0.f;
 #pragma unroll
             for (int u = 0; u < U; ++u) {
-                if constexpr (SILU) {  // the product replaces x's own registers (f32; f16 x: below)
+                if constexpr (SILU) {  // the product replaces x's own registers
 #pragma unroll
                     for (int h = 0; h < XL; ++h) {
-                        if constexpr (!HALF) {
-                            f32x4 c = __builtin_bit_cast(f32x4, xr[u][j][h]);
-                            const f32x4 d = __builtin_bit_cast(f32x4, xbr[u][j][h]);
+                        f32x4 c = __builtin_bit_cast(f32x4, xr[u][j][h]);
+                        const f32x4 d = __builtin_bit_cast(f32x4, xbr[u][j][h]);
 #pragma unroll
-                            for (int e = 0; e < 4; ++e) c[e] = silu_f(c[e]) * d[e];
-                            xr[u][j][h] = __builtin_bit_cast(u32x4, c);
-                        } else {
-                            const half8 g8 = __builtin_bit_cast(half8, xr[u][j][h]), u8 = __builtin_bit_cast(half8, xbr[u][j][h]);
-                            f32x4 c, d;
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) {
-                                c[e] = silu_f((float)g8[e]) * (float)u8[e];
-                                d[e] = silu_f((float)g8[e + 4]) * (float)u8[e + 4];
-                            }
-                            xr[u][j][h] = __builtin_bit_cast(u32x4, c);
-                            xbr[u][j][h] = __builtin_bit_cast(u32x4, d);
-                        }
+                        for (int e = 0; e < 4; ++e) c[e] = silu_f(c[e]) * d[e];
+                        xr[u][j][h] = __builtin_bit_cast(u32x4, c);
                     }
                 }
                 const f32x4 c0 = __builtin_bit_cast(f32x4, xr[u][j][0]);
-                const f32x4 c1 = __builtin_bit_cast(f32x4, HALF ? xbr[u % (SILU ? U : 1)][j][0] : xr[u][j][XL - 1]);
+                const f32x4 c1 = __builtin_bit_cast(f32x4, xr[u][j][XL - 1]);
                 asm("v_max3_f32 %0, |%1|, |%2|, %0\n\tv_max3_f32 %0, |%3|, |%4|, %0"
                     : "+v"(m) : "v"(c0[0]), "v"(c0[1]), "v"(c0[2]), "v"(c0[3]));
                 asm("v_max3_f32 %0, |%1|, |%2|, %0\n\tv_max3_f32 %0, |%3|, |%4|, %0"
@@ -342,15 +332,15 @@ __global__ __launch_bounds__(64 * kWaves) void i4xs_kernel(Args a) {
                 *reinterpret_cast<u32x4 *>(dst) = to_b_order(u < nu ? xr[u][j][0] : u32x4{0, 0, 0, 0});
             } else {
                 const f32x4 c0 = __builtin_bit_cast(f32x4, xr[u][j][0]);
-                const f32x4 c1 = __builtin_bit_cast(f32x4, HALF ? xbr[u % (SILU ? U : 1)][j][0] : xr[u][j][XL - 1]);
+                const f32x4 c1 = __builtin_bit_cast(f32x4, xr[u][j][XL - 1]);
                 u32x4 H, L;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     H[e] = mix_hi(c0[e], c1[e], up[j]);
-                    if constexpr (!HALF) L[e] = mix_lo(c0[e], c1[e], up[j], H[e]);
+                    L[e] = mix_lo(c0[e], c1[e], up[j], H[e]);
                 }
                 *reinterpret_cast<u32x4 *>(dst) = H;
-                if constexpr (!HALF) *reinterpret_cast<u32x4 *>(dst + 4096) = L;
+                *reinterpret_cast<u32x4 *>(dst + 4096) = L;
             }
         }
 #pragma unroll
@@ -476,7 +466,7 @@ __global__ __launch_bounds__(64 * kWaves) void i4xs_kernel(Args a) {
                 for (int sr = 0; sr < NSRC; ++sr) a.part[((size_t)(ksl * NSRC + sr) * a.M + m) * N + nc] = y[sr];
                 continue;
             }
-            const float yv = NSRC == 2 ? silu_f(y[0]) * y[NSRC - 1] : y[0];
+            const float yv = NSRC == 2 ? silu_f(y[0]) * y[NSRC - 1] : a.rsc ? y[0] * a.rsc[m] : y[0];
             if (a.f16out)
                 static_cast<_Float16 *>(a.y)[(size_t)m * N + nc] = (_Float16)yv;
             else
@@ -497,7 +487,7 @@ int launch_gs(st_context *ctx, const Args &a, int groups, bool hz) {
     } while (0)
     const int U = (a.uq + (a.urem > 0) + kWaves - 1) / kWaves;
     // (silu(a) * b: both inputs of a unit in flight, at most two units)
-    constexpr bool SILU = XM == X_F32_SILU || XM == X_F16_SILU;
+    constexpr bool SILU = XM == X_F32_SILU;
     if (U == 1)
         ST_XS(1, 4);
     else if (U == 2)

@@ -108,6 +108,9 @@ def test_skinny_gate_up(gpu, orc, Mr, K, N, gs, zeros, act, f16):
     (1, 2048, 136, 128, True, False, False, torch.float32),
     (77, 4096, 520, 128, True, False, True, torch.float32),
     (40, 1152, 1032, 64, False, False, True, torch.float16),
+    (100, 9728, 520, 64, True, True, True, torch.float16),  # act-order: the product is gathered
+    (33, 32768, 24, 256, False, False, True, torch.float32),  # the longest row of the product's pre-pass
+    (35, 8320, 264, 128, True, True, True, torch.float32),  # 8 k past a pass of its threads
 ])
 def test_skinny_gemm(gpu, orc, Mr, K, N, gs, zeros, act, silu, out):
     c = _case(orc, 1000 + Mr, K, N, gs, zeros, act, Mr, True)
@@ -126,6 +129,29 @@ def test_skinny_gemm(gpu, orc, Mr, K, N, gs, zeros, act, silu, out):
     # weights (silu: the product) rounded once to f16, then C
     tol = TOL_F16 * (2**0.5 if out == torch.float16 else 1)
     assert orc.rel_l2(y.float().cpu().numpy(), _ref(orc, c, xin, K, N, gs, act)) < tol
+
+
+def test_skinny_gemm_silu_scales(gpu, orc):
+    """f16 silu(a) * b of very different size by token: past f16's range, below
+    its normals, zero, and one that is not finite, each row by itself."""
+    Mr, K, N = 36, 2176, 264
+    c = _case(orc, 81, K, N, 128, False, False, Mr, True)
+    w = _up(gpu, c, 128)
+    rng = np.random.default_rng(81)
+    a, b = (rng.standard_normal((Mr, K)) for _ in range(2))
+    size = 2.0 ** np.linspace(-12, 11, Mr)
+    a, b = (a * size[:, None]).astype(np.float16), (b * size[:, None]).astype(np.float16)
+    a[5], b[7, 3] = 0, np.inf
+    y = torch.full((Mr, N), float("nan"), device="cuda")
+    M.fused_silu_gptq_gemm(gpu, torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda(), w.qweight, w.scales, y, K, N, 128,
+                           w.qzeros, w.perm, w.flags)
+    torch.cuda.synchronize()
+    y = y.cpu().numpy().astype(np.float64)
+    assert not y[5].any() and not np.isfinite(y[7]).any()
+    keep = [i for i in range(Mr) if i not in (5, 7)]
+    ref = _ref(orc, c, orc.silu_gate_f64(a[keep], b[keep]), K, N, 128, False)
+    for i, r in zip(keep, ref):
+        assert orc.rel_l2(y[i] / np.abs(r).max(), r / np.abs(r).max()) < TOL_F16, i
 
 
 @pytest.mark.parametrize("bad", [float("nan"), float("inf")])
