@@ -143,11 +143,15 @@ struct Split {
 // projections of 2560- and 4096-wide layers at 6-128 tokens): a wave's x
 // costs x_us per unit, a tile tile_us per unit, and K slices a second launch
 // plus their partial sums' way to memory and back.
-Split plan(const st_context *ctx, int xm, int M, int K, int N, int nsrc, size_t ws) {
+Split plan(const st_context *ctx, int xm, int gs, bool hz, int M, int K, int N, int nsrc, size_t ws) {
     const int units = K / 128, ntiles = (N + kTileN - 1) / kTileN;
     const int tb = (M + block_tokens(xm) - 1) / block_tokens(xm);
     const bool half = is_half(xm), silu = xm == X_F32_SILU;
-    const int umax = silu ? 2 : kMaxUnits;
+    // Groups of 64 with zero points: four units' scales, zeros and fragments
+    // spill (20-28 registers), so three. 4096 x 14336, four / three: 16 tokens
+    // of f16 x 23.1 / 16.6 us, 32 of f32 26.1 / 23.5, gate/up 4096 x 14336 16 of f32
+    // 40.0 / 24.9, 32 58.1 / 37.2. (X_F16G, 4 registers: 100 tokens 38.0 / 46.0, so four.)
+    const int umax = silu ? 2 : gs == 64 && hz && xm != X_F16G ? 3 : kMaxUnits;
     const double x_us = half ? 0.4 : 0.8, tile_us = half ? 0.25 : 0.22;
     Split best;
     double least = 1e30;
@@ -186,7 +190,7 @@ int int4_xs(st_context *ctx, const XsCall &c) {
         if (!ctx->ws || off > ctx->ws_bytes) return -1;
         if (silu && !half) xm = X_F32;
     }
-    const Split sp = plan(ctx, xm, c.M, c.K, c.N, c.nsrc, ctx->ws ? ctx->ws_bytes - off : 0);
+    const Split sp = plan(ctx, xm, c.gs, c.qz[0] != nullptr, c.M, c.K, c.N, c.nsrc, ctx->ws ? ctx->ws_bytes - off : 0);
     if (!sp.ks) return -1;
     Args a{};
     a.x = c.x;

@@ -1,9 +1,8 @@
 // Skinny GPTQ int4 GEMM with x held in registers (gfx950): a few to a few
 // dozen tokens against tiled weights (st_gptq_i4_repack),
 //   y[m, n]  = sum_g s[g, n] * sum_{k in g} (q[k, n] - z[g, n]) * x[m, k]
-// or silu(gate) * up of two such sums, x as f32, f16 or f32 silu(a) * b (f16:
-// a pre-pass)
-// (semantics of gptq_matvec.wgsl:51-58, fused_gate_up_silu_4t.wgsl:24-90 and
+// or silu(gate) * up of two such sums, x as f32, f16 or f32 silu(a) * b (f16: a
+// pre-pass) (semantics of gptq_matvec.wgsl:51-58, fused_gate_up_silu_4t.wgsl:24-90 and
 // fused_silu_gptq_4t.wgsl:26-81; the reference runs one token at a time).
 //
 //  * Exact products: (q - z) is an integer in [-16, 15], exact in f16 (the
@@ -496,7 +495,10 @@ int launch_gs(st_context *ctx, const Args &a, int groups, bool hz) {
         return st::fail(ST_ERR_UNSUPPORTED, "i4xs: %d units per wave", U);
     else if (U == 3)
         ST_XS(3, 4);
-    else
+    else if constexpr (GS == 64 && XM != X_F16G) {  // (with zero points: at most three units, see plan)
+        if (hz) return st::fail(ST_ERR_UNSUPPORTED, "i4xs: %d units per wave", U);
+        st::launch(ctx, (i4xs_kernel<XM, NSRC, GS, 4, 2, false>), grid, block, 0, a);
+    } else
         ST_XS(4, 2);
 #undef ST_XS
     return st::launch_check("i4xs_kernel");

@@ -83,6 +83,7 @@ def test_skinny_silu_matvec(gpu, orc, Mr, K, N, gs, zeros, act):
     (9, 1536, 4120, 128, True, False, False),
     (32, 4096, 1032, 64, False, False, False),
     (17, 5120, 776, 256, True, True, True),
+    (12, 3328, 1032, 64, True, False, False),  # group 64 with zero points: three units a wave at most
 ])
 def test_skinny_gate_up(gpu, orc, Mr, K, N, gs, zeros, act, f16):
     c = _case(orc, 900 + Mr, K, N, gs, zeros, act, Mr, f16)
