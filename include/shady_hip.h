@@ -69,6 +69,12 @@ typedef enum { ST_F32 = 0, ST_F16 = 1, ST_BF16 = 2 } st_dtype;
 /* Message of the last failed call on this thread ("" if none). */
 const char *st_last_error(void);
 
+/* The kernels that this thread's calls have launched since its last call of
+ * st_launches (the newest 64 at most), oldest first: writes up to `max` names
+ * (static strings) and returns how many. Several kernels stand behind one
+ * entry point; this says which a call took. */
+int st_launches(const char **names, int max);
+
 /* Version string of the built library (kernels + ABI revision). */
 const char *st_version(void);
 

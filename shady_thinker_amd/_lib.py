@@ -60,6 +60,7 @@ _SIGNATURES = {
     "st_context_get_tune": (_I, [_P, _I, ctypes.POINTER(_I)]),
     "st_context_set_timing_events": (_I, [_P, _P, _P]),
     "st_context_pin_workspace": (_I, [_P, _I]),
+    "st_launches": (_I, [ctypes.POINTER(ctypes.c_char_p), _I]),
     "st_alloc": (_I, [_P, _SZ, ctypes.POINTER(_P)]),
     "st_free": (_I, [_P, _P]),
     "st_upload": (_I, [_P, _P, _P, _SZ]),
@@ -112,6 +113,13 @@ def lib() -> ctypes.CDLL:
 def check(fn: str, code: int) -> None:
     if code != ST_OK:
         raise ShadyHipError(fn, code, lib().st_last_error().decode())
+
+
+def launches() -> list[str]:
+    """Names of the kernels this thread has launched since the last call of
+    launches() (the newest 64), oldest first: which kernels a call took."""
+    names = (ctypes.c_char_p * 64)()
+    return [names[i].decode() for i in range(lib().st_launches(names, 64))]
 
 
 _bound: dict = {}  # entry points by name, bound once

@@ -74,11 +74,22 @@ inline int hip_fail(hipError_t e, const char *what) {
 
 inline bool aligned16(const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
+// The names of the calling thread's last launches (st_launches): the dispatch
+// rules choose among several kernels for one entry point, and a test of one of
+// them has to know that it ran.
+struct LaunchLog {
+    static constexpr int kNames = 64;
+    const char *name[kNames];  // string literals; launch i at i % kNames
+    unsigned count = 0, taken = 0;
+};
+extern thread_local LaunchLog g_launches;
+
 // Launch-error check after a kernel launch (launch failures only; faults
 // surface at the next synchronising call).
 inline int launch_check(const char *what) {
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(e, what);
+    g_launches.name[g_launches.count++ % LaunchLog::kNames] = what;
     return ST_OK;
 }
 

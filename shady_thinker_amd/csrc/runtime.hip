@@ -4,6 +4,7 @@
 // pointers.
 #include "common.hpp"
 
+#include <algorithm>
 #include <cstdlib>
 #include <cstring>
 #include <mutex>
@@ -22,6 +23,8 @@ void set_error(const char *fmt, ...) {
 }
 
 void clear_error() { g_last_error.clear(); }
+
+thread_local LaunchLog g_launches;
 
 }  // namespace st
 
@@ -53,6 +56,15 @@ static int scratch_for(int device, void **out) {
 extern "C" {
 
 const char *st_last_error(void) { return st::g_last_error.c_str(); }
+
+int st_launches(const char **names, int max) {
+    st::LaunchLog &g = st::g_launches;
+    const unsigned kept = std::min<unsigned>(g.count - g.taken, st::LaunchLog::kNames);
+    const int n = names && max > 0 ? std::min<int>((int)kept, max) : 0;
+    for (int i = 0; i < n; ++i) names[i] = g.name[(g.count - n + i) % st::LaunchLog::kNames];
+    g.taken = g.count;
+    return n;
+}
 
 const char *st_version(void) { return "shady_hip 0.1 gfx950 abi-1"; }
 

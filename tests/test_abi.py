@@ -39,6 +39,12 @@ def test_version_and_error_string():
     assert isinstance(L.st_last_error(), bytes)
 
 
+def test_launches_is_empty_without_launches():
+    _lib.launches()
+    assert _lib.launches() == []
+    assert sta.lib().st_launches(None, 0) == 0
+
+
 def test_null_arguments_are_rejected():
     L = sta.lib()
     assert L.st_context_create(0, None) == 1  # ST_ERR_INVALID
