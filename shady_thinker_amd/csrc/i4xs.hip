@@ -22,25 +22,20 @@ namespace {
 using namespace st::xs;
 
 // y = epilogue(sum over slices s < ks of part[s][src]), the slices added in
-// order (deterministic), the epilogue silu(gate) * up for two sources.
+// pairs (a fixed order), the epilogue silu(gate) * up for two sources.
 template <int NSRC, bool F16OUT>
 __global__ __launch_bounds__(256) void i4xs_reduce_kernel(const float *__restrict__ part, void *__restrict__ y, int MN,
                                                           int ks, const float *__restrict__ rsc, int N) {
     const int idx = blockIdx.x * 256 + threadIdx.x;
     if (idx >= MN) return;
-    float t[kMaxSplit][NSRC];  // every slice's load issued before the first add
+    float t[NSRC][kMaxSplit];  // every slice's load issued before the first add
 #pragma unroll
     for (int s = 0; s < kMaxSplit; ++s)
 #pragma unroll
-        for (int sr = 0; sr < NSRC; ++sr) t[s][sr] = s < ks ? part[(size_t)(s * NSRC + sr) * MN + idx] : 0.f;
+        for (int sr = 0; sr < NSRC; ++sr) t[sr][s] = s < ks ? part[(size_t)(s * NSRC + sr) * MN + idx] : 0.f;
     float v[NSRC];
 #pragma unroll
-    for (int sr = 0; sr < NSRC; ++sr) {
-        v[sr] = 0.f;
-#pragma unroll
-        for (int s = 0; s < kMaxSplit; ++s)
-            if (s < ks) v[sr] += t[s][sr];
-    }
+    for (int sr = 0; sr < NSRC; ++sr) v[sr] = pair_sum(t[sr]);
     const float r = NSRC == 2 ? silu_f(v[0]) * v[NSRC - 1] : rsc ? v[0] * rsc[idx / N] : v[0];
     if (F16OUT)
         static_cast<_Float16 *>(y)[idx] = (_Float16)r;
@@ -146,12 +141,8 @@ struct Split {
 Split plan(const st_context *ctx, int xm, int gs, bool hz, int M, int K, int N, int nsrc, size_t ws) {
     const int units = K / 128, ntiles = (N + kTileN - 1) / kTileN;
     const int tb = (M + block_tokens(xm) - 1) / block_tokens(xm);
-    const bool half = is_half(xm), silu = xm == X_F32_SILU;
-    // Groups of 64 with zero points: four units' scales, zeros and fragments
-    // spill (20-28 registers), so three. 4096 x 14336, four / three: 16 tokens
-    // of f16 x 23.1 / 16.6 us, 32 of f32 26.1 / 23.5, gate/up 4096 x 14336 16 of f32
-    // 40.0 / 24.9, 32 58.1 / 37.2. (X_F16G, 4 registers: 100 tokens 38.0 / 46.0, so four.)
-    const int umax = silu ? 2 : gs == 64 && hz && xm != X_F16G ? 3 : kMaxUnits;
+    const bool half = is_half(xm);
+    const int umax = max_units(xm, nsrc, gs, hz);
     const double x_us = half ? 0.4 : 0.8, tile_us = half ? 0.25 : 0.22;
     Split best;
     double least = 1e30;

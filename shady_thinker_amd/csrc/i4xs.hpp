@@ -9,17 +9,17 @@
 //    f16 1024 bias: 1024 + q, minus 1024 + z). f16 x is used as is. f32 x
 //    (and silu(a) * b) is scaled per token and wave by a power of two into
 //    f16's range and split into hi + lo, two f16 values (about 22
-//    significant bits): two MFMAs into one accumulator. Each 64 or 128 k
-//    sum into a fresh f32 accumulator that is then scaled by s in f32.
+//    significant bits): two MFMAs, into two accumulators. Each 64 or 128 k
+//    sum into fresh f32 accumulators that are then added and scaled by s in f32.
 //  * Work split. A workgroup owns a run of 16-column tiles, a K slice and a
 //    block of tokens (16 f32 or 32 f16). Its waves split the slice's 128-k
 //    units, U consecutive units each, and keep the MFMA A fragments of their
 //    own units in registers (32 VGPRs per unit) for all the workgroup's
-//    tiles: x is read, scaled and split once per workgroup, nothing of it
-//    goes through LDS, and no wave waits for another while weights stream.
+//    tiles: x is read, scaled and split once per workgroup, none of it is
+//    shared through LDS, and no wave waits for another while weights stream.
 //    Per tile each wave leaves its 16-column partial sums in LDS; after every
-//    R / NSRC tiles the workgroup meets once and adds them in wave order
-//    (deterministic).
+//    R / NSRC tiles the workgroup meets once and adds them in pairs (a fixed
+//    order).
 //  * Weights stream through a register ring of R tiles x U units per wave
 //    (48-64 KiB in flight per CU); loads past the end use an out-of-range
 //    buffer offset (no access), so every path issues the same loads.
@@ -27,7 +27,7 @@
 //    run side by side on one XCD, so the weights come from HBM once and from
 //    that XCD's L2 after.
 //  * Few tiles, or K beyond what the waves hold: K slices across workgroups,
-//    f32 partials in the workspace, added in slice order by a reduce launch.
+//    f32 partials in the workspace, added in a fixed order by a reduce launch.
 #pragma once
 #include "common.hpp"
 
@@ -49,7 +49,18 @@ enum { X_F16 = 0, X_F32 = 1, X_F32_SILU = 2, X_F16G = 3 };
 constexpr bool is_half(int xm) { return xm == X_F16 || xm == X_F16G; }  // one f16 value per x
 
 constexpr int kWaves = 8;                   // waves per workgroup
-constexpr int kMaxUnits = 4;                // 128-k units per wave
+// 128-k units per wave at most: their weights, fragments and sums are in
+// registers, two f32 inputs of silu(a) * b at first too, and where they spill
+// one unit less is faster or the same. us at 4 / 3 units (128), 3 / 2 (64):
+// gate/up with zero points 4096 x 14336, 32 tokens, f32 x, group 128 36.8 /
+// 31.8, group 256 38.5 / 33.4, f16 x 26.9 / 24.9 and 29.0 / 25.8; 5632 x 9728
+// group 64 f32 x 51.5 / 37.8, f16 x 31.6 / 26.7. One source with zero points:
+// 4 in groups 128 and 256 (6-8 registers spilled; from 5% slower than 3 units,
+// 3328 x 4096, to 5% faster, 4096 x 14336), 3 in groups of 64 (20-28 spilled at
+// 4: 4096 x 14336, f16 x, 23.1 / 16.6).
+constexpr int max_units(int xm, int nsrc, int gs, bool hz) {
+    return xm == X_F32_SILU ? 2 : xm == X_F16G || !hz ? 4 : 4 - (nsrc == 2) - (gs == 64);
+}
 constexpr int block_tokens(int xm) { return is_half(xm) ? 32 : 16; }
 
 struct Args {
@@ -109,6 +120,18 @@ __device__ __forceinline__ u32x4 to_b_order(u32x4 a) {
 __device__ __forceinline__ float silu_f(float v) { return __fdividef(v, 1.0f + __expf(-v)); }
 
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
+// The sum of p in pairs of pairs: a fixed order, each value rounded log2(n)
+// times (in a row n - 1 times, at growing sums).
+template <int n>
+__device__ __forceinline__ float pair_sum(float (&p)[n]) {
+    static_assert((n & (n - 1)) == 0, "a power of two");
+#pragma unroll
+    for (int d = 1; d < n; d *= 2)
+#pragma unroll
+        for (int i = 0; i < n; i += 2 * d) p[i] += p[i + d];
+    return p[0];
+}
 
 template <int CTRL>
 __device__ __forceinline__ float dpp_f(float v) {
@@ -378,14 +401,15 @@ __global__ __launch_bounds__(64 * kWaves) void i4xs_kernel(Args a) {
                 zhi[u][j] = __builtin_bit_cast(half2_t, zh | (zh << 16));
             }
         constexpr int NA = ROUND ? (NU < 2 ? NU : 2) : NU;  // (ROUND: units may share accumulators)
-        f32x4 acc[NA][MB];
+        // [0..1]: the two row blocks, or (f32 x) the hi and the lo parts, whose
+        // sums meet once per group: in one chain hi's sum, nearly exact by
+        // itself, was rounded to lo's steps at every MFMA.
+        f32x4 acc[NA][2];
 #pragma unroll
         for (int j = 0; j < NG; ++j) {
             if (!ROUND || j == 0)
 #pragma unroll
-                for (int u = 0; u < NA; ++u)
-#pragma unroll
-                    for (int mb = 0; mb < MB; ++mb) acc[u][mb] = f32x4{0.f, 0.f, 0.f, 0.f};
+                for (int u = 0; u < NA; ++u) acc[u][0] = acc[u][1] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int e = 0; e < EK; ++e) {
                 const int step = EK * j + e;
@@ -400,7 +424,7 @@ __global__ __launch_bounds__(64 * kWaves) void i4xs_kernel(Args a) {
                     acc[u % NA][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[u][step][0], b[u], acc[u % NA][0], 0, 0, 0);
 #pragma unroll
                 for (int u = 0; u < NU; ++u)
-                    acc[u % NA][MB - 1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[u][step][1], b[u], acc[u % NA][MB - 1], 0, 0, 0);
+                    acc[u % NA][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[u][step][1], b[u], acc[u % NA][1], 0, 0, 0);
             }
             if constexpr (!ROUND)
 #pragma unroll
@@ -408,7 +432,8 @@ __global__ __launch_bounds__(64 * kWaves) void i4xs_kernel(Args a) {
 #pragma unroll
                     for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-                        for (int i = 0; i < 4; ++i) ys[mb][i] = __builtin_fmaf(sf[u][j], acc[u][mb][i], ys[mb][i]);
+                        for (int i = 0; i < 4; ++i)
+                            ys[mb][i] = __builtin_fmaf(sf[u][j], SCALED ? acc[u][0][i] + acc[u][1][i] : acc[u][mb][i], ys[mb][i]);
         }
         if constexpr (ROUND)
 #pragma unroll
@@ -454,9 +479,10 @@ __global__ __launch_bounds__(64 * kWaves) void i4xs_kernel(Args a) {
             float y[NSRC];
 #pragma unroll
             for (int sr = 0; sr < NSRC; ++sr) {
-                y[sr] = 0.f;
+                float p[kWaves];
 #pragma unroll
-                for (int w = 0; w < kWaves; ++w) y[sr] += red[w * (WB / 4) + (((rt * NSRC + sr) * MB + mb) * 4 + i) * 64 + l];
+                for (int w = 0; w < kWaves; ++w) p[w] = red[w * (WB / 4) + (((rt * NSRC + sr) * MB + mb) * 4 + i) * 64 + l];
+                y[sr] = pair_sum(p);
             }
             const int m = tok0 + 16 * mb + 4 * (l >> 4) + i, nc = kTileN * (t0 + t + rt) + (l & 15);
             if (t + rt >= nt || m >= a.M || nc >= N) continue;
@@ -477,31 +503,22 @@ __global__ __launch_bounds__(64 * kWaves) void i4xs_kernel(Args a) {
 template <int XM, int NSRC, int GS>
 int launch_gs(st_context *ctx, const Args &a, int groups, bool hz) {
     const dim3 grid(groups * a.ks * a.tblocks), block(64 * kWaves);
-#define ST_XS(U_, R_)                                                                                          \
-    do {                                                                                                       \
-        if (hz)                                                                                                \
-            st::launch(ctx, (i4xs_kernel<XM, NSRC, GS, U_, R_, true>), grid, block, 0, a);                \
-        else                                                                                                   \
-            st::launch(ctx, (i4xs_kernel<XM, NSRC, GS, U_, R_, false>), grid, block, 0, a);               \
-    } while (0)
-    const int U = (a.uq + (a.urem > 0) + kWaves - 1) / kWaves;
-    // (silu(a) * b: both inputs of a unit in flight, at most two units)
-    constexpr bool SILU = XM == X_F32_SILU;
-    if (U == 1)
-        ST_XS(1, 4);
-    else if (U == 2)
-        ST_XS(2, 4);
-    else if constexpr (SILU)
-        return st::fail(ST_ERR_UNSUPPORTED, "i4xs: %d units per wave", U);
-    else if (U == 3)
-        ST_XS(3, 4);
-    else if constexpr (GS == 64 && XM != X_F16G) {  // (with zero points: at most three units, see plan)
-        if (hz) return st::fail(ST_ERR_UNSUPPORTED, "i4xs: %d units per wave", U);
-        st::launch(ctx, (i4xs_kernel<XM, NSRC, GS, 4, 2, false>), grid, block, 0, a);
-    } else
-        ST_XS(4, 2);
-#undef ST_XS
-    return st::launch_check("i4xs_kernel");
+    auto units = [&](auto UC, auto HZC) {
+        constexpr int U = decltype(UC)::value;
+        constexpr bool HZ = decltype(HZC)::value;
+        if constexpr (U <= max_units(XM, NSRC, GS, HZ)) {
+            st::launch(ctx, (i4xs_kernel<XM, NSRC, GS, U, U == 4 ? 2 : 4, HZ>), grid, block, 0, a);
+            return st::launch_check("i4xs_kernel");
+        } else
+            return st::fail(ST_ERR_UNSUPPORTED, "i4xs: %d units per wave", U);
+    };
+    auto zeros = [&](auto UC) { return hz ? units(UC, std::true_type{}) : units(UC, std::false_type{}); };
+    switch ((a.uq + (a.urem > 0) + kWaves - 1) / kWaves) {
+        case 1: return zeros(std::integral_constant<int, 1>{});
+        case 2: return zeros(std::integral_constant<int, 2>{});
+        case 3: return zeros(std::integral_constant<int, 3>{});
+        default: return zeros(std::integral_constant<int, 4>{});
+    }
 }
 
 template <int XM, int NSRC>

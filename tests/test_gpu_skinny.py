@@ -9,6 +9,7 @@ import torch
 
 import shady_thinker_amd as sta
 from shady_thinker_amd import model as M
+from shady_thinker_amd._lib import launches
 
 pytestmark = pytest.mark.gpu
 
@@ -58,6 +59,31 @@ def test_skinny_matvec(gpu, orc, Mr, K, N, gs, zeros, act, f16):
     M.gptq_matvec(gpu, "t", x, w.qweight, w.scales, y, K, N, gs, w.qzeros, w.perm, w.flags)
     torch.cuda.synchronize()
     assert orc.rel_l2(y.cpu().numpy(), _ref(orc, c, c["x"], K, N, gs, act)) < TOL
+
+
+@pytest.mark.parametrize("Mr,K,N,gs,zeros,act", [
+    (22, 11008, 1416, 128, False, True),
+    (10, 10240, 2488, 128, True, False),
+    (26, 9472, 624, 256, False, False),
+])
+def test_skinny_f32_sums(gpu, orc, Mr, K, N, gs, zeros, act):
+    """f32 x keeps f32 sums: the hi parts' products (nearly exact in f32) and the
+    lo parts' are summed apart within a group, and the groups in few roundings.
+
+    Bound: x is held to half a unit of its 22nd bit or better, 2^-23 / sqrt(3)
+    = 6.9e-8 rms at the worst mantissa and 4.6e-8 over a binade. After it a sum
+    is rounded at most 4 times within a wave, 3 over the waves and 4 over the
+    slices, each 2^-24 / sqrt(3) = 3.4e-8 of the sum so far (sqrt(j / n) of the
+    whole one after j of n equal parts): sqrt(2.5 + 1.75 + 1.9) 3.4e-8 = 8.5e-8
+    in all, 9.7e-8 with x's part. (In one chain of hi and lo: 1.34e-7.)"""
+    c = _case(orc, 1100 + Mr, K, N, gs, zeros, act, Mr, False)
+    w = _up(gpu, c, gs)
+    y = torch.full((Mr, N), float("nan"), device="cuda")
+    launches()
+    M.gptq_matvec(gpu, "t", torch.from_numpy(c["x"]).cuda(), w.qweight, w.scales, y, K, N, gs, w.qzeros, w.perm, w.flags)
+    assert "i4xs_kernel" in launches()
+    torch.cuda.synchronize()
+    assert orc.rel_l2(y.cpu().numpy(), _ref(orc, c, c["x"], K, N, gs, act)) < 1.1e-7
 
 
 @pytest.mark.parametrize("Mr,K,N,gs,zeros,act", [
