@@ -25,11 +25,13 @@
 //    buffer offset (no access), so every path issues the same loads.
 //  * More tokens than a block: workgroups of the same tiles and other tokens
 //    run side by side on one XCD, so the weights come from HBM once and from
-//    that XCD's L2 after.
+//    that XCD's L2 after (on any XCDs, in grids that are no multiple of 8: 3
+//    blocks 6% slower over 307 drawn prompts, up to 13%, 5 blocks 8%).
 //  * Few tiles, or K beyond what the waves hold: K slices across workgroups,
 //    f32 partials in the workspace, added in a fixed order by a reduce launch.
 #pragma once
 #include "common.hpp"
+#include "xcd.hpp"
 
 #include <type_traits>
 
@@ -39,7 +41,7 @@ namespace xs {
 constexpr int kTileN = 16;
 constexpr int kMaxSplit = 16;              // K slices
 constexpr int kRsrcWord3 = 0x00020000;     // raw 32-bit buffer data (gfx9-class)
-constexpr int kNt = 2;                       // non-temporal loads: weights are read once
+constexpr int kNt = 2;                       // non-temporal loads: a workgroup reads its weights once
 constexpr unsigned kNoLoad = 0x80000000u;  // buffer offset past every resource: reads 0, touches no memory
 
 // X_F16G: f16 x against (q - z) s rounded once to f16 (the prefill GEMM's
@@ -179,10 +181,10 @@ __global__ __launch_bounds__(64 * kWaves) void i4xs_kernel(Args a) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int q = lane >> 4, r16 = lane & 15;
 
-    // XCD-major order: workgroups go to XCDs round-robin, so consecutive ids
-    // (first the token blocks of one tile run, then its K slices) share an XCD.
-    const int nb = gridDim.x;
-    int id = nb % 8 == 0 ? (blockIdx.x % 8) * (nb / 8) + blockIdx.x / 8 : blockIdx.x;
+    // XCD-major order: consecutive ids (first the token blocks of one tile
+    // run, then its K slices) share an XCD, but for the 7 places where one
+    // XCD's workgroups end.
+    int id = xcd_order(blockIdx.x, gridDim.x);
     const int tok0 = (id % a.tblocks) * TPB;
     id /= a.tblocks;
     const int ksl = id % a.ks, grp = id / a.ks;
