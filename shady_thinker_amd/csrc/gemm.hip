@@ -834,6 +834,7 @@ int gemm_impl(const char *fn, st_context *ctx, const uint16_t *a, const uint16_t
             x.sc[0] = w1->scales;
             x.qz[0] = w1->qzeros;
             x.y = w1->c;
+            x.gathered = perm != nullptr;
             rc = st::int4_xs(ctx, x);
         }
         if (rc != -1) return rc;

@@ -187,14 +187,18 @@ int int4_xs(st_context *ctx, const XsCall &c) {
     a.x = c.x;
     a.xb = c.xb;
     if (pre) {
+        a.x = ctx->ws;
+        a.xb = nullptr;
+        if (half && silu) a.rsc = reinterpret_cast<float *>(reinterpret_cast<char *>(ctx->ws) + rsc_off);
+    }
+    if (pre && !c.gathered) {
         void *xg = ctx->ws;
         const dim3 g((unsigned)(((size_t)c.M * c.K / 4 + 255) / 256)), b(256);
-        if (half && silu) {
-            float *const rsc = reinterpret_cast<float *>(reinterpret_cast<char *>(ctx->ws) + rsc_off);
+        if (half && silu)
             st::launch(ctx, i4xs_silu_kernel, dim3(c.M), dim3(kSiluThreads), 0, static_cast<const _Float16 *>(c.x),
-                       static_cast<const _Float16 *>(c.xb), c.perm, static_cast<_Float16 *>(xg), rsc, c.K);
-            a.rsc = rsc;
-        } else if (half)
+                       static_cast<const _Float16 *>(c.xb), c.perm, static_cast<_Float16 *>(xg),
+                       reinterpret_cast<float *>(reinterpret_cast<char *>(ctx->ws) + rsc_off), c.K);
+        else if (half)
             st::launch(ctx, i4xs_gather_kernel<uint16_t, false>, g, b, 0, static_cast<const uint16_t *>(c.x),
                        static_cast<const uint16_t *>(nullptr), c.perm, static_cast<uint16_t *>(xg), c.M, c.K);
         else if (silu)
@@ -203,9 +207,7 @@ int int4_xs(st_context *ctx, const XsCall &c) {
         else
             st::launch(ctx, i4xs_gather_kernel<float, false>, g, b, 0, static_cast<const float *>(c.x),
                        static_cast<const float *>(nullptr), c.perm, static_cast<float *>(xg), c.M, c.K);
-        if (int rc = launch_check("i4xs pre-pass")) return rc;
-        a.x = xg;
-        a.xb = nullptr;
+        if (int rc = launch_check(half && silu ? "i4xs_silu_kernel" : "i4xs_gather_kernel")) return rc;
     }
     for (int i = 0; i < 2; ++i) {
         const int j = i < c.nsrc ? i : 0;

@@ -158,6 +158,28 @@ def test_skinny_gemm(gpu, orc, Mr, K, N, gs, zeros, act, silu, out):
     assert orc.rel_l2(y.float().cpu().numpy(), _ref(orc, c, xin, K, N, gs, act)) < tol
 
 
+@pytest.mark.parametrize("Mr,K,N,gs,act", [(77, 4096, 520, 128, True), (40, 9728, 264, 64, True), (64, 2048, 264, 128, False)])
+def test_skinny_gate_up_gemm(gpu, orc, Mr, K, N, gs, act):
+    """Gate and up of a short prompt: x gathered once for both weights, results
+    those of two single calls."""
+    c = _case(orc, 1150, K, N, gs, False, act, Mr, True)
+    c2 = _case(orc, 1151, K, N, gs, False, act, Mr, True)
+    c2["g_idx"] = c["g_idx"]
+    ws = [_up(gpu, v, gs) for v in (c, c2)]
+    x = torch.from_numpy(c["x"]).cuda()
+    y = [torch.full((Mr, N), float("nan"), device="cuda") for _ in range(4)]
+    launches()
+    M.gate_up_gemm(gpu, x, ws[0].qweight, ws[0].scales, ws[1].qweight, ws[1].scales, y[0], y[1], K, N, gs, perm=ws[0].perm,
+                   flags=ws[0].flags)
+    ran = launches()
+    assert ran.count("i4xs_kernel") == 2 and ran.count("i4xs_gather_kernel") == int(act)
+    for w, o in zip(ws, y[2:]):
+        M.gptq_gemm(gpu, x, w.qweight, w.scales, o, K, N, gs, None, w.perm, w.flags)
+    torch.cuda.synchronize()
+    assert torch.equal(y[0], y[2]) and torch.equal(y[1], y[3])
+    assert orc.rel_l2(y[1].cpu().numpy(), _ref(orc, c2, c["x"], K, N, gs, act)) < TOL_F16
+
+
 def test_skinny_gemm_silu_scales(gpu, orc):
     """f16 silu(a) * b of very different size by token: past f16's range, below
     its normals, zero, and one that is not finite, each row by itself."""
