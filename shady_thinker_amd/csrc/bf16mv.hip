@@ -135,10 +135,13 @@ __global__ __launch_bounds__(kThreads) void bf16mv_kernel(const void *__restrict
 //    loads (six bytes per x would not fit the LDS for every K taken here).
 //  * Each wave keeps the next US segments of its row groups in flight while
 //    it computes US.
-//  * A sum that is not finite is done again in plain f32 (inf - inf or inf * 0
-//    among the parts of an infinite x or weight would make a NaN of an
-//    infinity), and so is one so small that the last parts of its x may have
-//    been lost below bf16's range (2^-133).
+//  * x is staged times 2^24 and the sums are taken times 2^-24: the last part
+//    of the smallest f32 subnormal is then a normal bf16 value (2^-125), so
+//    that no part of any x is lost, whatever the weights.
+//  * A sum that is not finite (inf - inf or inf * 0 among the parts of an
+//    infinite x or weight would make a NaN of an infinity; the scale overflows
+//    from |x| = 2^104) is done again in plain f32, by the whole wave: a token
+//    with a NaN or an infinity in it does so for every row.
 // Bound by HBM. us with 2 / 4 / 5 / 8 tokens, the former kernel (a row's 8
 // lanes reading every token's x, f32 FMAs; bound by those reads) and this one:
 //   2560 x 151936  191 / 187 / 366 / 371   143-155 (5.0-5.4 TB/s)
@@ -153,6 +156,7 @@ constexpr int US = 4;                      // segments (KiB of weights) per batc
 constexpr int kRsrcWord3 = 0x00020000;     // raw 32-bit buffer data (gfx9-class)
 constexpr unsigned kNoLoad = 0x80000000u;  // buffer offset past every resource: reads 0, touches no memory
 constexpr int kNt = 2;                     // non-temporal loads: weights are read once
+constexpr float kUp = 16777216.0f, kDown = 1.0f / kUp;  // x is staged times 2^24
 
 __device__ __forceinline__ int x_swizzle(int m) { return (m & 1) | ((m & 2) << 2); }
 
@@ -191,26 +195,31 @@ __global__ __launch_bounds__(64 * kMmWaves) void bf16mm_kernel(const void *__res
             wv[u] = __builtin_amdgcn_raw_buffer_load_b128(r, o, 0, kNt);
         }
     };
+    const __amdgpu_buffer_rsrc_t rx =
+        __builtin_amdgcn_make_buffer_rsrc((void *)xp, (short)0, M * K * (F16X ? 2 : 4), kRsrcWord3);
+    // token m's x of k .. k + 3; past M or K zeros, by offset and not by a
+    // branch: with one around each load and its store the loads of eight
+    // tokens came one after the other (5120 x 264, 8 tokens of f16 x: 41 us)
+    auto load_x = [&](int m, int k) __attribute__((always_inline)) {
+        const unsigned o = m < M && k < K ? (unsigned)(m * K + k) * (F16X ? 2u : 4u) : kNoLoad;
+        if constexpr (F16X) {
+            const half4 s = __builtin_bit_cast(half4, __builtin_amdgcn_raw_buffer_load_b64(rx, o, 0, 0));
+            return f32x4{(float)s[0], (float)s[1], (float)s[2], (float)s[3]};
+        } else {
+            return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, o, 0, 0));
+        }
+    };
     u32x4 wa[US], wb[US];
     load(wa, wid, 0);
 
     for (int c = tid; c < Kp / 4; c += blockDim.x) {
         f32x4 v[8];  // chunk c of every token, all loads in flight at once
 #pragma unroll
-        for (int m = 0; m < 8; ++m) {
-            v[m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-            if (m >= M || 4 * c >= K) continue;  // (K % 8 == 0)
-            const size_t at = (size_t)m * K + 4 * c;
-            if constexpr (F16X) {
-                const half4 s = *reinterpret_cast<const half4 *>(static_cast<const _Float16 *>(xp) + at);
-                v[m] = f32x4{(float)s[0], (float)s[1], (float)s[2], (float)s[3]};
-            } else {
-                v[m] = *reinterpret_cast<const f32x4 *>(static_cast<const float *>(xp) + at);
-            }
-        }
+        for (int m = 0; m < 8; ++m) v[m] = load_x(m, 4 * c);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int m = 0; m < 8; ++m)
-            if (m < M) *reinterpret_cast<f32x4 *>(&xs[m * Kp + 4 * (c ^ x_swizzle(m))]) = v[m];
+            if (m < M) *reinterpret_cast<f32x4 *>(&xs[m * Kp + 4 * (c ^ x_swizzle(m))]) = v[m] * kUp;
     }
     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
 
@@ -248,6 +257,26 @@ __global__ __launch_bounds__(64 * kMmWaves) void bf16mm_kernel(const void *__res
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[i] = low[i] = 0.0f;
     };
+    // Row n's sum for token m in plain f32, by all lanes.
+    auto row_sum = [&](int n, int m) __attribute__((always_inline)) {
+        const uint16_t *const wr = w + (size_t)n * K;
+        float t = 0.0f;
+#pragma unroll 1
+        for (int k = 8 * lane; k < K; k += 512) {  // K % 8 == 0
+            const u32x4 wv = *reinterpret_cast<const u32x4 *>(wr + k);
+            f32x4 x2[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) x2[i] = load_x(m, k + 4 * i);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const unsigned we = wv[e >> 1];
+                t = fmaf(__uint_as_float(e & 1 ? we & 0xFFFF0000u : we << 16), x2[e >> 2][e & 3], t);
+            }
+        }
+#pragma unroll
+        for (int d = 1; d < 64; d *= 2) t += __shfl_xor(t, d);
+        return t;
+    };
     auto store = [&](int g) __attribute__((always_inline)) {
         acc += low;
         // Lane: column l % 32 = (token, h), A rows 8 (i / 4) + 4 q + i % 4 =
@@ -261,24 +290,15 @@ __global__ __launch_bounds__(64 * kMmWaves) void bf16mm_kernel(const void *__res
             out = h == i ? t : out;
         }
         const int n = 8 * g + 2 * h + q;
-        if (n >= N || mid >= M) return;
-        const float mag = fabsf(out);
-        if (!(mag <= 3.402823466e38f) || (mag < 1e-25f && mag > 0.0f)) {
-            // in the one-token kernel's order
-            const uint16_t *wr = w + (size_t)n * K;
-            float t[8];
-#pragma unroll
-            for (int c = 0; c < 8; ++c) {
-                t[c] = 0.0f;
-                for (int k0 = 8 * c; k0 < K; k0 += 64)
-                    for (int k = k0; k < k0 + 8; ++k) {
-                        const unsigned wk = (unsigned)wr[k] << 16;
-                        t[c] = fmaf(__uint_as_float(wk), xrow[4 * ((k >> 2) ^ sw) + (k & 3)], t[c]);
-                    }
-            }
-            out = ((t[0] + t[1]) + (t[2] + t[3])) + ((t[4] + t[5]) + (t[6] + t[7]));
+        const bool mine = n < N && mid < M;
+        const bool bad = mine && !(fabsf(out) <= 3.402823466e38f);
+        out *= kDown;
+        for (unsigned long long todo = __ballot(bad); todo; todo &= todo - 1) {
+            const int l = __builtin_ctzll(todo);
+            const float t = row_sum(8 * g + 2 * (l & 3) + (l >> 5), (l >> 2) & 7);  // lane l's row and token
+            out = lane == l ? t : out;
         }
-        y[(size_t)mid * N + n] = out;
+        if (mine) y[(size_t)mid * N + n] = out;
     };
     clear();
     int g = wid, b = 0;  // the batch in hand

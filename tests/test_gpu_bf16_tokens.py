@@ -72,3 +72,36 @@ def test_bf16_tokens_scales_of_x(gpu):
     assert not y[7].any()
     for r in range(7):
         assert ((y[r] - ref[r]).norm() / ref[r].norm()).item() < TOL, r
+
+
+@pytest.mark.parametrize("xs,ws", [
+    (2.0**-120, 2.0**50),   # x's third part below 2^-133
+    (2.0**-140, 2.0**60),   # x below f32's normals
+    (2.0**60, 2.0**-130),   # weights below bf16's normals
+    (2.0**-20, 2.0**-110),  # sums below f32's normals
+    (2.0**110, 2.0**-20),   # x past the staging scale's range
+])
+def test_bf16_tokens_far_scales(gpu, xs, ws):
+    """Small x against large weights and the other way: no part of x is lost
+    whatever the size of the sum."""
+    K, N, Mr = 1000, 264, 5
+    x, w = _case(7, K, N, Mr)
+    x, w = x * xs, (w.float() * ws).to(torch.bfloat16)
+    y = _run(gpu, x.cuda(), w.cuda()).double()
+    ref = x.double() @ w.double().t()
+    tiny = ref.abs().max() < 2.0**-120  # f32's steps below its normals
+    assert ((y - ref).norm() / ref.norm()).item() < (2.0**-149 * (K * N * Mr) ** 0.5 / ref.norm().item() + TOL if tiny else TOL)
+
+
+def test_bf16_tokens_one_bad_token(gpu):
+    """A NaN and an infinity in two tokens of a call over many rows: theirs are
+    what f32 sums give, the other tokens' are bit for bit what they are without."""
+    K, N, Mr = 520, 20001, 8
+    x, w = _case(8, K, N, Mr)
+    good = _run(gpu, x.cuda(), w.cuda())
+    x[2, 7], x[6, 500] = float("nan"), float("inf")
+    y = _run(gpu, x.cuda(), w.cuda())
+    keep = [0, 1, 3, 4, 5, 7]
+    assert torch.equal(y[keep], good[keep]) and torch.isnan(y[2]).all()
+    ref = x[6] @ w.float().t()
+    assert torch.equal(torch.isnan(y[6]), torch.isnan(ref)) and torch.equal(y[6][torch.isinf(ref)], ref[torch.isinf(ref)])
