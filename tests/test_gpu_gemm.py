@@ -14,6 +14,7 @@ import torch
 
 import shady_thinker_amd as sta
 from shady_thinker_amd import model as M
+from shady_thinker_amd._lib import launches
 
 pytestmark = pytest.mark.gpu
 
@@ -31,6 +32,19 @@ def run_gemm(gpu, w, a_np, out_dtype=torch.float32):
     M.gptq_gemm(gpu, a, w.qweight, w.scales, c, w.K, w.N, w.group_size, w.qzeros, w.perm, w.flags)
     torch.cuda.synchronize()
     return c.float().cpu().numpy()
+
+
+# Short prompts on tiled weights go to the skinny kernel (i4xs.hpp). Tests of
+# the GEMM at such sizes run twice: as dispatched, and with GEMM_CB set, which
+# keeps the skinny kernel out (0: the GEMM's tile stays its own choice).
+@pytest.fixture(params=["skinny", "gemm"])
+def route(request, tune):
+    if request.param == "gemm":
+        tune(GEMM_CB=0)
+    launches()
+    yield request.param
+    ran = set(launches())
+    assert ("gemm_kernel" in ran, "i4xs_kernel" in ran) == (request.param == "gemm", request.param == "skinny")
 
 
 @pytest.mark.parametrize("tiled", [True, False])
@@ -141,7 +155,7 @@ def test_gemm_full_config_vs_oracle(gpu, orc, Mr):
     assert e16 < 1e-5
 
 
-def test_gemm_graph_replay_matches_eager(gpu, orc):
+def test_gemm_graph_replay_matches_eager(gpu, orc, route):
     Mr, K, N, gs = 160, 1024, 392, 128
     c = orc.gptq_case(8, K, N, gs, act_order=True, M=Mr, x_dtype=np.float16)
     w = up(gpu, c)
@@ -176,9 +190,13 @@ def test_gemm_split_k_matches_unsplit(gpu, orc, gs, tune):
     Mr, K, N = 64, 4096, 264
     c = orc.gptq_case(60 + gs, K, N, gs, zeros=True, act_order=True, M=Mr, x_dtype=np.float16)
     w = up(gpu, c)
+    tune(GEMM_CB=0)  # (else the skinny kernel takes so few rows)
+    launches()
     y_split = run_gemm(gpu, w, c["x"])
+    assert "splitk_reduce_kernel" in launches()
     tune(GEMM_NO_SPLIT=1)
     y_one = run_gemm(gpu, w, c["x"])
+    assert launches()[-1] == "gemm_kernel"
     ref = orc.gptq_matvec_f64(c["x"], c["qweight"], c["scales"], K, N, gs, qzeros=c["qzeros"], g_idx=c["g_idx"])
     e_s, e_o, e_so = orc.rel_l2(y_split, ref), orc.rel_l2(y_one, ref), orc.rel_l2(y_split, y_one)
     print(f"split-K gs={gs}: split {e_s:.3e}, one {e_o:.3e}, split vs one {e_so:.3e}")
@@ -206,7 +224,7 @@ def test_gemm_tile_widths_agree(gpu, orc, Mr, K, N, gs, zeros, act, tune):
     assert orc.rel_l2(ys["1"], ref) < 5e-4
 
 
-def test_gemm_long_k(gpu, orc):
+def test_gemm_long_k(gpu, orc, route):
     Mr, K, N, gs = 80, 32768, 264, 128
     c = orc.gptq_case(120, K, N, gs, zeros=True, act_order=True, M=Mr, x_dtype=np.float16)
     w = up(gpu, c)
@@ -216,11 +234,12 @@ def test_gemm_long_k(gpu, orc):
 
 
 @pytest.mark.parametrize("out_dtype", [torch.float32, torch.float16])
-def test_gemm_unaligned_c_matches_aligned(gpu, orc, out_dtype):
-    """C one element past a 16-byte boundary takes the per-element epilogue,
-    an aligned C the epilogue staged through LDS (16-byte row chunks): the
-    same values bit for bit."""
-    Mr, K, N, gs = 130, 1024, 264, 128
+def test_gemm_unaligned_c_matches_aligned(gpu, orc, out_dtype, route):
+    """C one element past a 16-byte boundary takes the GEMM's per-element
+    epilogue, an aligned C the one staged through LDS (16-byte row chunks; K
+    too short to be split, whose partials are aligned): the same values bit
+    for bit. The skinny kernel writes elements either way."""
+    Mr, K, N, gs = 130, 512, 264, 128
     c = orc.gptq_case(77, K, N, gs, zeros=True, M=Mr, x_dtype=np.float16)
     w = up(gpu, c)
     a = torch.from_numpy(c["x"]).to(gpu.device)
@@ -251,14 +270,15 @@ def run_gate_up(gpu, wg, wu, a_np, out_dtype=torch.float32):
     (300, 1536, 776, 64, True, True, False, torch.float32),     # act-order, zeros, row-major qweight
     (257, 2048, 520, 256, True, False, True, torch.float16),    # group 256, ragged M
     (64, 4096, 264, 128, False, False, True, torch.float32),    # few tiles: split-K, two launches on one A
+    (300, 4096, 264, 128, False, False, True, torch.float32),   # the same beyond the skinny kernel's rows
     (33, 1024, 1032, 128, "up", False, True, torch.float32),    # zero points on up only
-    (128, 2560, 9728, 128, False, False, True, torch.float16),  # combined grid would not split K, one weight alone would
+    (128, 2560, 9728, 128, False, False, True, torch.float16),  # a short prompt: the skinny kernel, one launch per weight
 ])
 def test_gate_up_gemm_equals_two_gemms(gpu, orc, Mr, K, N, gs, zeros, act, tiled, out):
     """st_gptq_i4_gate_up_gemm: each output bit for bit what st_gptq_i4_gemm
     gives for that weight (one grid over both weights' tiles, or two
-    launches on the shared pre-processed A when K is split), and within the
-    GEMM bar of the f64 oracle."""
+    launches on the shared pre-processed A when K is split, or the skinny
+    kernel once per weight), and within the GEMM bar of the f64 oracle."""
     cg = orc.gptq_case(600 + Mr, K, N, gs, zeros=zeros is True, act_order=act, M=Mr, x_dtype=np.float16)
     cu = orc.gptq_case(700 + Mr, K, N, gs, zeros=bool(zeros), act_order=act)
     cu["g_idx"] = cg["g_idx"]
@@ -275,7 +295,7 @@ def test_gate_up_gemm_equals_two_gemms(gpu, orc, Mr, K, N, gs, zeros, act, tiled
         assert e < TOL
 
 
-def test_gate_up_gemm_graph_replay(gpu, orc):
+def test_gate_up_gemm_graph_replay(gpu, orc, route):
     """Captured once, replayed three times with eager work between: both
     outputs equal the eager call's bit for bit every time."""
     Mr, K, N, gs = 256, 1024, 2048, 128

@@ -14,6 +14,7 @@ import torch
 
 import shady_thinker_amd as sta
 from shady_thinker_amd import model as M
+from shady_thinker_amd._lib import launches
 
 pytestmark = pytest.mark.gpu
 
@@ -807,9 +808,22 @@ def test_int8_mm_f16_graph_replay(gpu, orc):
         assert torch.equal(y, eager)
 
 
-def _force_i4mm(tune):
+# Two f16-MFMA kernels take several tokens (the rules are in qmv.hip): i4mm
+# where the tokens fill 16 MFMA rows or less (8 of f32 x, 16 of f16) and N has
+# more 16-column tiles than the GPU CUs (256 here), for one source only on some
+# numbers of tiles per CU; i4xs the rest. Each test says which of them its rows
+# mean.
+def _force_f16(tune):
+    """An f16-MFMA kernel (not the integer-limb ones) from 2 tokens on."""
     tune(I4MM_MIN_M=2)
     tune(I4MM_MIN_TILES=1)
+
+
+def _ran(kernel):
+    """The one of the two that ran since the last look, and no other."""
+    ran = set(launches())
+    assert (kernel in ran) and not {"i4mm_kernel", "i4xs_kernel", "qmv_kernel"} - {kernel} & ran, ran
+    return ran
 
 
 def _gate_up(gpu, wg, wu, x, dtype=torch.float32):
@@ -823,24 +837,32 @@ def _gate_up(gpu, wg, wu, x, dtype=torch.float32):
     return y.cpu().numpy()
 
 
-@pytest.mark.parametrize("Mr,K,N,gs,zeros,f16,dual", [
-    (2, 128, 64, 128, False, False, False),     # one unit, one tile
-    (5, 384, 72, 64, True, False, False),       # group 64, ragged last tile
-    (16, 2560, 6144, 128, False, False, False),  # configs[4] q|k|v at batch 16
-    (16, 9728, 2560, 128, False, False, False),  # configs[4] down: 160 tiles, 76 units
-    (9, 4096, 520, 256, True, False, False),    # group 256, two 16-row blocks
-    (12, 1024, 1000, 128, True, True, False),   # f16 x
-    (3, 256, 36880, 128, False, False, False),  # 2305 tiles: more workgroups than CUs
-    (16, 2560, 9728, 128, False, False, True),  # configs[4] gate/up at batch 16
-    (6, 1536, 776, 64, True, True, True),       # gate/up, f16 x, zeros, group 64
+@pytest.mark.parametrize("Mr,K,N,gs,zeros,f16,dual,kernel", [
+    (2, 128, 64, 128, False, False, False, "i4xs"),     # one unit, one tile
+    (5, 384, 72, 64, True, False, False, "i4xs"),       # group 64, ragged last tile
+    (16, 2560, 6144, 128, False, False, False, "i4xs"),  # a 2560-wide layer's q|k|v at batch 16
+    (16, 9728, 2560, 128, False, False, False, "i4xs"),  # its down: 160 tiles, 76 units
+    (9, 4096, 520, 256, True, False, False, "i4xs"),    # group 256
+    (12, 1024, 1000, 128, True, True, False, "i4xs"),   # f16 x
+    (3, 256, 36880, 128, False, False, False, "i4xs"),  # 2305 tiles: more than the CUs take at once
+    (16, 2560, 9728, 128, False, False, True, "i4xs"),  # gate/up at batch 16
+    (6, 1536, 776, 64, True, True, True, "i4xs"),       # gate/up, f16 x, zeros, group 64
+    (2, 128, 4112, 128, False, False, False, "i4mm"),   # one unit, 257 tiles: one or two per workgroup
+    (5, 384, 8264, 64, True, False, False, "i4mm"),     # group 64, 517 tiles, ragged last tile
+    (8, 2560, 6144, 128, False, False, False, "i4mm"),  # q|k|v at batch 8: 16 MFMA rows
+    (7, 4096, 4168, 256, True, False, False, "i4mm"),   # group 256, ragged last tile
+    (16, 1024, 5000, 128, True, True, False, "i4mm"),   # f16 x: 16 rows
+    (3, 256, 12264, 128, False, False, False, "i4mm"),  # 767 tiles: three per workgroup
+    (8, 2560, 9728, 128, False, False, True, "i4mm"),   # gate/up at batch 8
+    (6, 1536, 4232, 64, True, True, True, "i4mm"),      # gate/up, f16 x, zeros, group 64, ragged
+    (4, 256, 16408, 128, True, False, True, "i4mm"),    # gate/up, 1026 tile pairs: more workgroups than CUs
 ])
-def test_int4_mm_f16(gpu, orc, Mr, K, N, gs, zeros, f16, dual, tune):
-    """2..16 tokens on tiled GPTQ weights: the f16-MFMA kernel ((q - z)
-    exact in f16, f32 x as two f16 rows per 128-k block scaled by a power of
-    two, exact products, f32 sums and per-group scaling) against the f64
-    oracle, and against the integer-limb kernels. (The entry points choose
-    it for 12+ tokens and more tiles than CUs; forced here.)"""
-    _force_i4mm(tune)
+def test_int4_mm_f16(gpu, orc, Mr, K, N, gs, zeros, f16, dual, kernel, tune):
+    """2..16 tokens on tiled GPTQ weights: the f16-MFMA kernels ((q - z) exact
+    in f16, f32 x as two f16 values scaled by a power of two, exact products,
+    f32 sums and per-group scaling) against the f64 oracle, and the
+    integer-limb kernels on the same call."""
+    _force_f16(tune)
     xd = np.float16 if f16 else np.float32
     c = orc.gptq_case(150 + Mr, K, N, gs, zeros=zeros, M=Mr, x_dtype=xd)
     w = up(gpu, c)
@@ -854,22 +876,25 @@ def test_int4_mm_f16(gpu, orc, Mr, K, N, gs, zeros, f16, dual, tune):
         run = lambda: _gate_up(gpu, w, w2, c["x"], dt)
     else:
         run = lambda: run_matvec(gpu, w, c["x"], dt)
+    launches()
     y = run()
+    _ran(kernel + "_kernel")
     e = orc.rel_l2(y, ref)
     print(f"int4 f16-MFMA M={Mr} K={K} N={N} gs={gs} dual={dual} rel-L2 {e:.3e}")
     assert np.isfinite(y).all() and e < 1e-5
     tune(I4MM_MIN_M=99)
     assert orc.rel_l2(run(), ref) < TOL
+    assert not {"i4mm_kernel", "i4xs_kernel"} & set(launches())
 
 
 @pytest.mark.parametrize("Mr,K,N,gs,zeros,dual", [
-    (2, 128, 64, 128, False, False),       # one unit, one tile
-    (5, 384, 72, 64, True, False),         # group 64, ragged last tile
-    (16, 2560, 6144, 128, False, False),   # configs[4] q|k|v at batch 16
-    (9, 4096, 520, 256, True, False),      # group 256, two 16-row blocks
-    (3, 256, 36880, 128, False, False),    # more workgroups than CUs
-    (16, 2560, 9728, 128, False, True),    # configs[4] gate/up at batch 16
-    (6, 1536, 776, 64, True, True),        # gate/up, zeros, group 64
+    (2, 128, 4112, 128, False, False),     # one unit, 257 tiles
+    (5, 384, 8264, 64, True, False),       # group 64, ragged last tile
+    (8, 2560, 6144, 128, False, False),    # q|k|v of a 2560-wide layer at batch 8: 16 MFMA rows
+    (7, 4096, 4168, 256, True, False),     # group 256
+    (3, 256, 12264, 128, False, False),    # 767 tiles: three per workgroup
+    (8, 2560, 9728, 128, False, True),     # gate/up at batch 8
+    (6, 1536, 4232, 64, True, True),       # gate/up, zeros, group 64
 ])
 def test_int4_mm_f16_split_in_kernel(gpu, orc, Mr, K, N, gs, zeros, dual, tune):
     """f32 x on the f16-MFMA kernel is split into its hi / lo f16 rows and
@@ -877,7 +902,7 @@ def test_int4_mm_f16_split_in_kernel(gpu, orc, Mr, K, N, gs, zeros, dual, tune):
     pre-pass launch): the same arithmetic as the pre-pass, so y equals the
     pre-pass path (I4MM_PREPASS=1) bit for bit, and the f64 oracle within
     1e-5. x spans large and tiny magnitudes (per-unit exponents differ)."""
-    _force_i4mm(tune)
+    _force_f16(tune)
     c = orc.gptq_case(330 + Mr, K, N, gs, zeros=zeros, M=Mr)
     x = c["x"].copy()
     x[:, : K // 2] *= np.float32(3e4)
@@ -892,9 +917,12 @@ def test_int4_mm_f16_split_in_kernel(gpu, orc, Mr, K, N, gs, zeros, dual, tune):
         run = lambda: _gate_up(gpu, w, w2, x)
     else:
         run = lambda: run_matvec(gpu, w, x, torch.float32)
+    launches()
     y_in = run()
+    assert "i4mm_prep_kernel" not in _ran("i4mm_kernel")
     tune(I4MM_PREPASS=1)
     y_pre = run()
+    assert "i4mm_prep_kernel" in _ran("i4mm_kernel")
     np.testing.assert_array_equal(y_in, y_pre)
     e = orc.rel_l2(y_in, ref)
     print(f"int4 f16-MFMA in-kernel split M={Mr} K={K} N={N} gs={gs} dual={dual} rel-L2 {e:.3e}")
@@ -902,10 +930,10 @@ def test_int4_mm_f16_split_in_kernel(gpu, orc, Mr, K, N, gs, zeros, dual, tune):
 
 
 @pytest.mark.parametrize("Mr,K,N,gs,zeros,f16,dual", [
-    (16, 2560, 9728, 128, False, False, True),   # configs[4] gate/up: 608 tile pairs, 3 per workgroup
+    (8, 2560, 9728, 128, False, False, True),    # gate/up, 608 tile pairs, 3 per workgroup
     (9, 1024, 11008, 128, True, True, True),     # Llama-7B gate/up width, f16 x, zeros
-    (12, 1024, 12288, 128, False, False, False),  # one source, 768 tiles: 3 per workgroup, 4 waves each
-    (16, 1024, 20480, 64, True, False, False),   # one source, 1280 tiles: 5 per workgroup, group 64
+    (7, 1024, 12272, 128, False, False, False),  # one source, 767 tiles: 3 per workgroup, 4 waves each
+    (6, 1024, 12264, 64, True, False, False),    # the same in groups of 64, ragged
     (11, 2048, 9728, 256, True, True, True),     # gate/up, group 256, f16 x, zeros
 ])
 def test_int4_mm_f16_12_waves(gpu, orc, Mr, K, N, gs, zeros, f16, dual, tune):
@@ -916,7 +944,7 @@ def test_int4_mm_f16_12_waves(gpu, orc, Mr, K, N, gs, zeros, f16, dual, tune):
     a wave both sources of its tile (I4MM_PAIR): 4-way instead of 2-way K
     slices, so its sums round differently; it is held to the f64 oracle
     (1e-5), like the one-source forms."""
-    _force_i4mm(tune)
+    _force_f16(tune)
     xd = np.float16 if f16 else np.float32
     c = orc.gptq_case(190 + Mr, K, N, gs, zeros=zeros, M=Mr, x_dtype=xd)
     w = up(gpu, c)
@@ -930,11 +958,13 @@ def test_int4_mm_f16_12_waves(gpu, orc, Mr, K, N, gs, zeros, f16, dual, tune):
         run = lambda: _gate_up(gpu, w, w2, c["x"], dt)
     else:
         run = lambda: run_matvec(gpu, w, c["x"], dt)
+    launches()
     yd = run()
     tune(I4MM_PAIR=0)
     y12 = run()
     tune(I4MM_WAVES=16)
     y16 = run()
+    _ran("i4mm_kernel")
     for name, y in (("default", yd), ("one source per wave", y12)):
         e = orc.rel_l2(y, ref)
         print(f"int4 f16-MFMA 12 waves ({name}) M={Mr} K={K} N={N} gs={gs} dual={dual} rel-L2 {e:.3e}")
@@ -943,16 +973,17 @@ def test_int4_mm_f16_12_waves(gpu, orc, Mr, K, N, gs, zeros, f16, dual, tune):
 
 
 @pytest.mark.parametrize("Mr,K,N,gs,zeros,f16,dual", [
-    (16, 2560, 6144, 128, False, False, False),  # configs[4] q|k|v shape, f32 x (gathered in the pre-pass)
+    (8, 2560, 6144, 128, False, False, False),   # a 2560-wide layer's q|k|v, f32 x (gathered in the pre-pass)
     (12, 1024, 4112, 64, True, True, False),     # f16 x (gather pass), zeros, group 64, 257 tiles
-    (16, 2560, 9728, 128, True, False, True),    # gate/up, f32 x
+    (8, 2560, 9728, 128, True, False, True),     # gate/up, f32 x
+    (6, 1024, 4240, 64, True, False, True),      # gate/up, f32 x, zeros, group 64
     (13, 1536, 5200, 256, False, True, True),    # gate/up, f16 x, group 256
 ])
 def test_int4_mm_f16_act_order(gpu, orc, Mr, K, N, gs, zeros, f16, dual, tune):
-    """Act-order checkpoints on the f16-MFMA kernel (9-16 tokens): x read
-    through the upload's permutation (rows sorted by group), against the f64
-    oracle with scale[g_idx[k]], and against the integer-limb kernels."""
-    _force_i4mm(tune)
+    """Act-order checkpoints on i4mm: x read through the upload's permutation
+    (rows sorted by group) by the pre-pass or the gather, against the f64
+    oracle with scale[g_idx[k]], and the integer-limb kernels on the same call."""
+    _force_f16(tune)
     xd = np.float16 if f16 else np.float32
     c = orc.gptq_case(170 + Mr, K, N, gs, zeros=zeros, act_order=True, M=Mr, x_dtype=xd)
     w = up(gpu, c)
@@ -969,7 +1000,9 @@ def test_int4_mm_f16_act_order(gpu, orc, Mr, K, N, gs, zeros, f16, dual, tune):
         run = lambda: _gate_up(gpu, w, w2, c["x"], dt)
     else:
         run = lambda: run_matvec(gpu, w, c["x"], dt)
+    launches()
     y = run()
+    assert ("i4mm_gather_kernel" if f16 else "i4mm_prep_kernel") in _ran("i4mm_kernel")
     e = orc.rel_l2(y, ref)
     print(f"int4 f16-MFMA act-order M={Mr} K={K} N={N} gs={gs} dual={dual} rel-L2 {e:.3e}")
     assert np.isfinite(y).all() and e < 1e-5
@@ -977,64 +1010,78 @@ def test_int4_mm_f16_act_order(gpu, orc, Mr, K, N, gs, zeros, f16, dual, tune):
     assert orc.rel_l2(run(), ref) < TOL
 
 
-@pytest.mark.parametrize("Mr,N,dual,want", [
-    (5, 4112, False, True),     # 257 tiles, 5 tokens: the f16-MFMA kernel
-    (11, 4112, True, True),     # gate/up at 11 tokens
-    (6, 4112, True, True),      # gate/up at 6 tokens
-    (4, 4112, False, False),    # 4 tokens: the limb (or streaming) kernels
-    (10, 4096, False, True),    # 256 tiles, not more than the CUs: groups of 8 tiles, K split across workgroups
-    (8, 4096, False, False),    # 8 tokens on 256 tiles: the limb kernels
+@pytest.mark.parametrize("Mr,K,N,gs,act,dual,f16,kernel", [
+    (5, 1024, 4112, 128, False, False, False, "i4mm"),   # 257 tiles, 5 tokens
+    (4, 1024, 4112, 128, False, False, False, "qmv"),    # 4 tokens: the integer-limb (or streaming) kernels
+    (9, 1024, 4112, 128, False, False, False, "i4xs"),   # more than 8 tokens of f32 x
+    (16, 1024, 4112, 128, False, False, True, "i4mm"),   # 16 of f16
+    (17, 1024, 4112, 128, False, False, True, "i4xs"),
+    (8, 1024, 12272, 128, False, False, False, "i4mm"),  # 767 tiles: below 3 per CU
+    (8, 1024, 12280, 128, False, False, False, "i4xs"),  # 768 (the last one ragged)
+    (8, 1024, 8192, 64, False, False, False, "i4xs"),    # groups of 64 with f32 x: i4mm only above 2 per CU
+    (8, 1024, 8200, 64, False, False, False, "i4mm"),
+    (8, 1024, 8192, 64, False, False, True, "i4mm"),
+    (11, 1024, 4112, 128, False, True, False, "i4xs"),   # gate/up
+    (6, 1024, 4112, 128, False, True, False, "i4mm"),
+    (4, 1024, 4112, 128, False, True, False, "qmv"),
+    (10, 1024, 4096, 128, False, False, False, "i4xs"),  # 256 tiles: not more than the CUs
+    (8, 1024, 4096, 128, False, False, False, "qmv"),    # K below 2048: the limb kernels to 8 tokens
+    (5, 2048, 4096, 128, False, False, False, "i4xs"),   # else to 4
+    (4, 2048, 4096, 128, False, False, False, "qmv"),
+    (3, 2048, 4096, 128, True, False, False, "i4xs"),    # act-order: to 2
+    (2, 2048, 4096, 128, True, False, False, "qmv"),
 ])
-def test_int4_mm_f16_default_routing(gpu, orc, Mr, N, dual, want, tune):
+def test_int4_mm_f16_default_routing(gpu, orc, Mr, K, N, gs, act, dual, f16, kernel, tune):
     """Which kernel the GPTQ entry points pick by default on an MI355X (256
-    CUs): the f16-MFMA kernel from 5 tokens on linears with more 16-column
-    tiles than CUs and from 9 tokens on the others (with K split across
-    workgroups), the integer-limb kernels below. The default call's y
-    must equal, bit for bit, the call with that kernel forced; both are
-    checked against the f64 oracle."""
+    CUs), on both sides of every line of the rule; the result against the f64
+    oracle."""
     ncu = torch.cuda.get_device_properties(gpu.device).multi_processor_count
     if ncu != 256:
         pytest.skip(f"routing thresholds are stated for 256 CUs, this GPU has {ncu}")
-    K, gs = 1024, 128
-    c = orc.gptq_case(190 + Mr, K, N, gs, zeros=True, M=Mr)
+    c = orc.gptq_case(190 + Mr, K, N, gs, zeros=True, act_order=act, M=Mr, x_dtype=np.float16 if f16 else np.float32)
     w = up(gpu, c)
-    ref = orc.gptq_matvec_f64(c["x"], c["qweight"], c["scales"], K, N, gs, qzeros=c["qzeros"])
+    dt = torch.float16 if f16 else torch.float32
+    ref = orc.gptq_matvec_f64(c["x"], c["qweight"], c["scales"], K, N, gs, qzeros=c["qzeros"],
+                              g_idx=c["g_idx"] if act else None)
+    launches()
     if dual:
         c2 = orc.gptq_case(290 + Mr, K, N, gs, zeros=True)
         w2 = up(gpu, c2)
+        launches()
         ref = orc.silu_gate_f64(ref, orc.gptq_matvec_f64(c["x"], c2["qweight"], c2["scales"], K, N, gs,
                                                          qzeros=c2["qzeros"]))
-        run = lambda: _gate_up(gpu, w, w2, c["x"])
+        y = _gate_up(gpu, w, w2, c["x"], dt)
     else:
-        run = lambda: run_matvec(gpu, w, c["x"], torch.float32)
-    y = run()
-    if want:
-        _force_i4mm(tune)
+        y = run_matvec(gpu, w, c["x"], dt)
+    ran = set(launches())
+    if kernel == "qmv":
+        assert not {"i4mm_kernel", "i4xs_kernel"} & ran and {"qmv_kernel", "qmv_stream_kernel"} & ran, ran
     else:
-        tune(I4MM_MIN_M=99)
-    y_forced = run()
+        assert kernel + "_kernel" in ran and not {"i4mm_kernel", "i4xs_kernel"} - {kernel + "_kernel"} & ran, ran
     assert orc.rel_l2(y, ref) < TOL
-    np.testing.assert_array_equal(y, y_forced)
 
 
-@pytest.mark.parametrize("Mr,K,N,gs,zeros,f16,dual,act", [
-    (16, 4096, 2560, 128, False, False, False, False),  # configs[4] o: 160 tiles, 20 groups of 8, 12 K slices
-    (16, 9728, 2560, 128, False, False, False, False),  # configs[4] down: 76 units
-    (9, 11008, 4096, 128, True, False, False, False),   # Llama-7B down at 9 tokens, zeros
-    (12, 4096, 4096, 128, False, True, False, False),   # f16 x, 256 tiles
-    (10, 2048, 520, 64, True, False, False, False),     # group 64, ragged last tile
-    (13, 3072, 776, 256, False, False, False, False),   # group 256
-    (16, 2560, 1024, 128, False, False, True, False),   # gate/up on 64 tile pairs
-    (11, 1536, 776, 128, True, True, True, False),      # gate/up, f16 x, zeros
-    (16, 4096, 2560, 128, True, False, False, True),    # act-order, f32 x: pre-pass rows, then the partials
-    (14, 2048, 1040, 128, False, True, True, True),     # act-order, f16 x gathered, gate/up
+@pytest.mark.parametrize("Mr,K,N,gs,zeros,f16,dual,act,split", [
+    (16, 4096, 2560, 128, False, False, False, False, True),  # o of a 2560-wide layer: 160 tiles
+    (16, 9728, 2560, 128, False, False, False, False, True),  # its down: 76 units
+    (9, 11008, 4096, 128, True, False, False, False, True),   # Llama-7B down at 9 tokens, zeros
+    (12, 4096, 4096, 128, False, True, False, False, False),  # f16 x, 256 tiles: one K slice
+    (12, 8192, 4096, 128, False, True, False, False, True),   # two
+    (10, 2048, 520, 64, True, False, False, False, False),    # group 64, ragged last tile
+    (10, 8448, 520, 64, True, False, False, False, True),
+    (13, 3072, 776, 256, False, False, False, False, True),   # group 256
+    (16, 2560, 1024, 128, False, False, True, False, True),   # gate/up on 64 tile pairs
+    (11, 1536, 776, 128, True, True, True, False, False),     # gate/up, f16 x, zeros
+    (16, 4096, 2560, 128, True, False, False, True, True),    # act-order, f32 x: the gathered x, then the partials
+    (14, 2048, 1040, 128, False, True, True, True, False),    # act-order, f16 x gathered, gate/up
+    (14, 6144, 1040, 128, False, True, True, True, True),
 ])
-def test_int4_mm_f16_k_split(gpu, orc, Mr, K, N, gs, zeros, f16, dual, act, tune):
-    """9-16 tokens on no more 16-column tiles than CUs: the f16-MFMA kernel
-    takes groups of 8 tiles with K split across workgroups (whole chunks per
-    slice), f32 partial sums in the workspace (after the pre-pass rows when
-    there are any) added in slice order by a reduce launch. Against the f64
-    oracle (1e-5), against the integer-limb kernels, and deterministic."""
+def test_int4_mm_f16_k_split(gpu, orc, Mr, K, N, gs, zeros, f16, dual, act, split, tune):
+    """9-16 tokens on no more 16-column tiles than CUs: i4xs takes runs of tiles,
+    K split across workgroups where its estimate says so, f32 partial sums in the workspace (after
+    the gathered x when there is one) added in a fixed order by a reduce launch.
+    Against the f64 oracle (1e-5), deterministic, and the integer-limb kernels
+    on the same call."""
     xd = np.float16 if f16 else np.float32
     c = orc.gptq_case(400 + Mr, K, N, gs, zeros=zeros, act_order=act, M=Mr, x_dtype=xd)
     w = up(gpu, c)
@@ -1052,30 +1099,33 @@ def test_int4_mm_f16_k_split(gpu, orc, Mr, K, N, gs, zeros, f16, dual, act, tune
     else:
         run = lambda: run_matvec(gpu, w, c["x"], dt)
     tune(I4MM_MIN_M=2)
+    launches()
     y = run()
+    assert split == ("i4xs_reduce_kernel" in _ran("i4xs_kernel"))
     e = orc.rel_l2(y, ref)
     print(f"int4 f16-MFMA K split M={Mr} K={K} N={N} gs={gs} dual={dual} act={act} rel-L2 {e:.3e}")
     assert np.isfinite(y).all() and e < 1e-5
     np.testing.assert_array_equal(run(), y)
     tune(I4MM_SPLIT_TILES=0)
+    launches()
     assert orc.rel_l2(run(), ref) < TOL
+    assert not {"i4mm_kernel", "i4xs_kernel"} & set(launches())
 
 
 @pytest.mark.parametrize("Mr,K,N,gs,zeros,f16,act,dual", [
-    (32, 2560, 10240, 128, False, False, False, False),  # configs[4] q|k|v at 32 tokens: 64 MFMA rows
+    (32, 2560, 10240, 128, False, False, False, False),  # a 2560-wide layer's q|k|v at 32 tokens: two token blocks
     (17, 2048, 6160, 256, True, False, False, False),    # 17 tokens, group 256, ragged last tile
     (24, 9728, 2560, 128, True, False, False, False),    # few tiles: K split across workgroups
-    (32, 1024, 8200, 128, False, True, False, False),    # f16 x: two 16-row blocks
-    (20, 2048, 4160, 128, True, False, True, False),     # act-order: the pre-pass splits 20 tokens
-    (32, 1024, 4160, 64, False, False, False, False),    # group 64 with f32 x: 16-token blocks
-    (32, 2560, 9728, 128, False, False, False, True),    # configs[4] gate/up at 32 tokens, one source per wave
+    (32, 1024, 8200, 128, False, True, False, False),    # f16 x: two 16-row blocks of one token block
+    (20, 2048, 4160, 128, True, False, True, False),     # act-order: x gathered first
+    (32, 1024, 4160, 64, False, False, False, False),    # group 64 with f32 x
+    (32, 2560, 9728, 128, False, False, False, True),    # its gate/up at 32 tokens
     (19, 1024, 2064, 256, True, True, True, True),       # gate/up, f16 x, act-order, zeros
 ])
 def test_int4_mm_f16_32_tokens(gpu, orc, Mr, K, N, gs, zeros, f16, act, dual, tune):
-    """17-32 tokens in one f16-MFMA launch (the weights read once; f32 x as
-    64 hi/lo rows, 2-unit chunks; gate/up with one source per wave), against
-    the f64 oracle (1e-5), equal to the same call in 16-token pieces on the
-    integer-limb kernels within the bar, and deterministic."""
+    """17-32 tokens in one i4xs launch (two token blocks of f32 x, one of f16),
+    against the f64 oracle (1e-5), deterministic, and the same call in 16-token
+    pieces on the integer-limb kernels within the bar."""
     xd = np.float16 if f16 else np.float32
     c = orc.gptq_case(430 + Mr, K, N, gs, zeros=zeros, act_order=act, M=Mr, x_dtype=xd)
     w = up(gpu, c)
@@ -1092,7 +1142,9 @@ def test_int4_mm_f16_32_tokens(gpu, orc, Mr, K, N, gs, zeros, f16, act, dual, tu
         run = lambda: _gate_up(gpu, w, w2, c["x"], dt)
     else:
         run = lambda: run_matvec(gpu, w, c["x"], dt)
+    launches()
     y = run()
+    assert act == ("i4xs_gather_kernel" in _ran("i4xs_kernel"))
     e = orc.rel_l2(y, ref)
     print(f"int4 f16-MFMA {Mr} tokens K={K} N={N} gs={gs} act={act} dual={dual} rel-L2 {e:.3e}")
     assert np.isfinite(y).all() and e < 1e-5
@@ -1101,18 +1153,21 @@ def test_int4_mm_f16_32_tokens(gpu, orc, Mr, K, N, gs, zeros, f16, act, dual, tu
     assert orc.rel_l2(run(), ref) < TOL
 
 
-def test_int4_mm_f16_integer_exact(gpu, orc, tune):
+@pytest.mark.parametrize("Mr,N,kernel", [(11, 136, "i4xs"), (7, 4136, "i4mm")])
+def test_int4_mm_f16_integer_exact(gpu, orc, Mr, N, kernel, tune):
     """Integer x, unit scales, zeros: every product and partial sum is an
     integer below 2^24, so y equals the exact integer result bit for bit
     (pins the nibble order, the zero nibble and the row/column mapping)."""
-    _force_i4mm(tune)
-    Mr, K, N, gs = 11, 1152, 136, 128
+    _force_f16(tune)
+    K, gs = 1152, 128
     c = orc.gptq_case(170, K, N, gs, zeros=True)
     rng = np.random.default_rng(3)
     x = rng.integers(-3, 4, size=(Mr, K)).astype(np.float32)
     c["scales"] = np.ones_like(c["scales"])
     w = up(gpu, c)
+    launches()
     y = run_matvec(gpu, w, x)
+    _ran(kernel + "_kernel")
     qw, qz = c["qweight"], c["qzeros"]
     q = np.stack([(qw >> (4 * j)) & 0xF for j in range(8)], axis=1).reshape(K, N).astype(np.int64)
     z = np.stack([(qz >> (4 * j)) & 0xF for j in range(8)], axis=2).reshape(K // gs, N).astype(np.int64)
@@ -1120,25 +1175,29 @@ def test_int4_mm_f16_integer_exact(gpu, orc, tune):
     assert np.array_equal(y, (x.astype(np.int64) @ Wd).astype(np.float32))
 
 
-def test_int4_mm_f16_wide_range_x(gpu, orc, tune):
+@pytest.mark.parametrize("N,kernel", [(264, "i4xs"), (4136, "i4mm")])
+def test_int4_mm_f16_wide_range_x(gpu, orc, N, kernel, tune):
     """f32 x spanning 1e-30 .. 1e30 across 128-k blocks (outside f16's
-    range): the per-block power-of-two split keeps the bar."""
-    _force_i4mm(tune)
-    Mr, K, N = 7, 2048, 264
+    range): the split after a scaling by powers of two keeps the bar."""
+    _force_f16(tune)
+    Mr, K = 7, 2048
     c = orc.gptq_case(171, K, N, 128, M=Mr)
     blk = np.repeat(10.0 ** np.linspace(-30, 30, K // 128), 128).astype(np.float32)
     x = (c["x"] * blk).astype(np.float32)
     w = up(gpu, c)
+    launches()
     y = run_matvec(gpu, w, x)
+    _ran(kernel + "_kernel")
     ref = orc.gptq_matvec_f64(x, c["qweight"], c["scales"], K, N, 128)
     assert np.isfinite(y).all() and orc.rel_l2(y, ref) < 1e-5
 
 
-def test_int4_mm_f16_graph_replay(gpu, orc, tune):
-    """Gate/up and matvec on the f16-MFMA kernel under graph capture: every
+@pytest.mark.parametrize("Mr,N,kernel", [(16, 1040, "i4xs"), (8, 4160, "i4mm")])
+def test_int4_mm_f16_graph_replay(gpu, orc, Mr, N, kernel, tune):
+    """Gate/up and matvec on the f16-MFMA kernels under graph capture: every
     replay equals the eager result bit for bit."""
-    _force_i4mm(tune)
-    Mr, K, N = 16, 2560, 1040
+    _force_f16(tune)
+    K = 2560
     c = orc.gptq_case(172, K, N, 128, M=Mr)
     c2 = orc.gptq_case(173, K, N, 128)
     w, w2 = up(gpu, c), up(gpu, c2)
@@ -1150,7 +1209,9 @@ def test_int4_mm_f16_graph_replay(gpu, orc, tune):
         M.gptq_matvec(gpu, "t", x, w.qweight, w.scales, y, K, N, 128, None, None, w.flags)
         M.fused_gate_up_silu(gpu, x, w.qweight, w.scales, w2.qweight, w2.scales, h, K, N, 128, flags=w.flags)
 
+    launches()
     calls()
+    _ran(kernel + "_kernel")
     torch.cuda.synchronize()
     ye, he = y.clone(), h.clone()
     s = torch.cuda.Stream()
@@ -1167,15 +1228,19 @@ def test_int4_mm_f16_graph_replay(gpu, orc, tune):
         assert torch.equal(y, ye) and torch.equal(h, he)
 
 
-def test_int4_mm_f16_zeros_plus_one(gpu, orc, tune):
+@pytest.mark.parametrize("Mr,N,kernel", [(14, 392, "i4xs"), (6, 4232, "i4mm")])
+def test_int4_mm_f16_zeros_plus_one(gpu, orc, Mr, N, kernel, tune):
     """AutoGPTQ-v1 zero points (stored z - 1, ST_FLAG_ZEROS_PLUS_ONE) on the
-    f16-MFMA kernel, matvec and gate/up, against the f64 oracle."""
-    _force_i4mm(tune)
-    Mr, K, N, gs = 14, 1280, 392, 128
+    f16-MFMA kernels, matvec and gate/up, against the f64 oracle."""
+    _force_f16(tune)
+    K, gs = 1280, 128
     c = orc.gptq_case(180, K, N, gs, zeros=True, M=Mr)
     c2 = orc.gptq_case(181, K, N, gs, zeros=True)
     w, w2 = up(gpu, c, zeros_plus_one=True), up(gpu, c2, zeros_plus_one=True)
     g = orc.gptq_matvec_f64(c["x"], c["qweight"], c["scales"], K, N, gs, qzeros=c["qzeros"], zero_offset=1)
     u = orc.gptq_matvec_f64(c["x"], c2["qweight"], c2["scales"], K, N, gs, qzeros=c2["qzeros"], zero_offset=1)
+    launches()
     assert orc.rel_l2(run_matvec(gpu, w, c["x"]), g) < 1e-5
+    _ran(kernel + "_kernel")
     assert orc.rel_l2(_gate_up(gpu, w, w2, c["x"]), orc.silu_gate_f64(g, u)) < 1e-5
+    _ran(kernel + "_kernel")
