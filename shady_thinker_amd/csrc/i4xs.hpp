@@ -57,9 +57,10 @@ constexpr int kWaves = 8;                   // waves per workgroup
 // gate/up with zero points 4096 x 14336, 32 tokens, f32 x, group 128 36.8 /
 // 31.8, group 256 38.5 / 33.4, f16 x 26.9 / 24.9 and 29.0 / 25.8; 5632 x 9728
 // group 64 f32 x 51.5 / 37.8, f16 x 31.6 / 26.7. One source with zero points:
-// 4 in groups 128 and 256 (6-8 registers spilled; from 5% slower than 3 units,
-// 3328 x 4096, to 5% faster, 4096 x 14336), 3 in groups of 64 (20-28 spilled at
-// 4: 4096 x 14336, f16 x, 23.1 / 16.6).
+// 4 in groups 128 and 256 (f16 x: 8 registers spilled; f32 x, two units at a
+// time, none; from 5% slower than 3 units, 3328 x 4096, to 5% faster, 4096 x
+// 14336), 3 in groups of 64 (20-28 spilled at 4: 4096 x 14336, f16 x, 23.1 /
+// 16.6).
 constexpr int max_units(int xm, int nsrc, int gs, bool hz) {
     return xm == X_F32_SILU ? 2 : xm == X_F16G || !hz ? 4 : 4 - (nsrc == 2) - (gs == 64);
 }
@@ -402,41 +403,46 @@ __global__ __launch_bounds__(64 * kWaves) void i4xs_kernel(Args a) {
                 zlo[u][j] = __builtin_bit_cast(half2_t, zl | (zl << 16));
                 zhi[u][j] = __builtin_bit_cast(half2_t, zh | (zh << 16));
             }
-        constexpr int NA = ROUND ? (NU < 2 ? NU : 2) : NU;  // (ROUND: units may share accumulators)
         // [0..1]: the two row blocks, or (f32 x) the hi and the lo parts, whose
         // sums meet once per group: in one chain hi's sum, nearly exact by
-        // itself, was rounded to lo's steps at every MFMA.
+        // itself, was rounded to lo's steps at every MFMA. Four units of them go
+        // two by two: with all eight sums and zero points live six registers
+        // spilled (3840 x 75936, 12 tokens, 45.6 / 40.0 us).
+        constexpr int PU = SCALED && NU == 4 ? 2 : NU;  // units at a time
+        constexpr int NA = ROUND ? (NU < 2 ? NU : 2) : PU;  // (ROUND: units may share accumulators)
         f32x4 acc[NA][2];
 #pragma unroll
-        for (int j = 0; j < NG; ++j) {
-            if (!ROUND || j == 0)
+        for (int p = 0; p < NU; p += PU)
 #pragma unroll
-                for (int u = 0; u < NA; ++u) acc[u][0] = acc[u][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int j = 0; j < NG; ++j) {
+                if (!ROUND || j == 0)
 #pragma unroll
-            for (int e = 0; e < EK; ++e) {
-                const int step = EK * j + e;
-                half8 b[NU];
+                    for (int u = 0; u < NA; ++u) acc[u][0] = acc[u][1] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-                for (int u = 0; u < NU; ++u) {
-                    b[u] = word_to_b(ring[rr][u][step], zlo[u][j], zhi[u][j]);
-                    if constexpr (ROUND) b[u] *= (_Float16)sf[u][j];  // (sf: an f16 value)
+                for (int e = 0; e < EK; ++e) {
+                    const int step = EK * j + e;
+                    half8 b[PU];
+#pragma unroll
+                    for (int u = 0; u < PU; ++u) {
+                        b[u] = word_to_b(ring[rr][p + u][step], zlo[p + u][j], zhi[p + u][j]);
+                        if constexpr (ROUND) b[u] *= (_Float16)sf[p + u][j];  // (sf: an f16 value)
+                    }
+#pragma unroll
+                    for (int u = 0; u < PU; ++u)
+                        acc[u % NA][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[p + u][step][0], b[u], acc[u % NA][0], 0, 0, 0);
+#pragma unroll
+                    for (int u = 0; u < PU; ++u)
+                        acc[u % NA][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[p + u][step][1], b[u], acc[u % NA][1], 0, 0, 0);
                 }
+                if constexpr (!ROUND)
 #pragma unroll
-                for (int u = 0; u < NU; ++u)
-                    acc[u % NA][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[u][step][0], b[u], acc[u % NA][0], 0, 0, 0);
+                    for (int u = 0; u < PU; ++u)
 #pragma unroll
-                for (int u = 0; u < NU; ++u)
-                    acc[u % NA][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[u][step][1], b[u], acc[u % NA][1], 0, 0, 0);
+                        for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+                            for (int i = 0; i < 4; ++i)
+                                ys[mb][i] = __builtin_fmaf(sf[p + u][j], SCALED ? acc[u][0][i] + acc[u][1][i] : acc[u][mb][i], ys[mb][i]);
             }
-            if constexpr (!ROUND)
-#pragma unroll
-                for (int u = 0; u < NU; ++u)
-#pragma unroll
-                    for (int mb = 0; mb < MB; ++mb)
-#pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            ys[mb][i] = __builtin_fmaf(sf[u][j], SCALED ? acc[u][0][i] + acc[u][1][i] : acc[u][mb][i], ys[mb][i]);
-        }
         if constexpr (ROUND)
 #pragma unroll
             for (int u = 0; u < NA; ++u)
