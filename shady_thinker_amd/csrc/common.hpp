@@ -142,5 +142,9 @@ struct XsCall {
     bool gathered = false;  // the workspace holds the act-order gather of this x, by the call before
 };
 int int4_xs(st_context *ctx, const XsCall &c);
+// Its estimated time (us) for f16 x and one source, and *pre_us that of its
+// pre-pass, by which the prefill entry points choose (1e30: not taken). Both
+// depend on sizes and options only, without xb not on whether there are zeros.
+double int4_xs_us(const st_context *ctx, const XsCall &c, double *pre_us);
 
 }  // namespace st

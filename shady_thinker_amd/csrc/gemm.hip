@@ -159,6 +159,7 @@ __global__ __launch_bounds__(64 * WN, 2) void gemm_kernel(const _Float16 *__rest
         sc = sc1;
         qz = qz1;
         C = C1;
+        if (part) part += (size_t)(gridDim.x / T) * M * N;  // (its partials follow the first weight's)
     }
     const int m0 = mt * BM, n0 = nt * BN;
     const int nw = n0 + 32 * CB * wave;  // this wave's columns
@@ -602,10 +603,15 @@ __global__ __launch_bounds__(256) void prep_a_kernel(const _Float16 *__restrict_
 
 constexpr int kMaxSplit = 8;  // K splits of a small GEMM grid (plan_gemm)
 
-// C[m, n] = sum over s < S of part[s, m, n] (fixed order: deterministic).
+// C[m, n] = sum over s < S of part[s, m, n] (fixed order: deterministic);
+// blockIdx.y 1: C1, from the partials after the first weight's.
 template <bool F16OUT>
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float *__restrict__ part, void *__restrict__ C,
-                                                            size_t MN, int S) {
+                                                            void *__restrict__ C1, size_t MN, int S) {
+    if (blockIdx.y) {
+        part += S * MN;
+        C = C1;
+    }
     const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
     if (i >= MN) return;  // MN % 4 == 0 (N % 8 == 0)
     // All slices' loads first (S <= kMaxSplit), then the adds in slice order:
@@ -651,7 +657,7 @@ struct GemmArgs {
     void *C;
     bool f16out;
     int M, K, N;
-    // optional second weight on the same A (C1 != NULL; no split-K)
+    // optional second weight on the same A (C1 != NULL)
     const uint32_t *qw1 = nullptr;
     const uint16_t *sc1 = nullptr;
     const uint32_t *qz1 = nullptr;
@@ -696,11 +702,11 @@ int launch_gs(st_context *ctx, const GemmArgs &g, int tile, const Split &sp) {
     void *C = g.C;
     if (sp.S > 1) {
         const size_t MN = (size_t)M * N;
-        const dim3 rg((unsigned)((MN / 4 + 255) / 256));
+        const dim3 rg((unsigned)((MN / 4 + 255) / 256), g.C1 ? 2 : 1);
         if (f16out)
-            st::launch(ctx, splitk_reduce_kernel<true>, rg, dim3(256), 0, sp.part, C, MN, sp.S);
+            st::launch(ctx, splitk_reduce_kernel<true>, rg, dim3(256), 0, sp.part, C, g.C1, MN, sp.S);
         else
-            st::launch(ctx, splitk_reduce_kernel<false>, rg, dim3(256), 0, sp.part, C, MN, sp.S);
+            st::launch(ctx, splitk_reduce_kernel<false>, rg, dim3(256), 0, sp.part, C, g.C1, MN, sp.S);
         return st::launch_check("splitk_reduce_kernel");
     }
     return ST_OK;
@@ -715,63 +721,93 @@ int launch_tiled(st_context *ctx, const GemmArgs &g, int gs, int tile, const Spl
     }
 }
 
-// Time (us) of one 128-k step of n workgroup tiles that run at once, from
-// sweeps of 200-2048 rows on weights of 2048 x 2560 to 2560 x 19456 (MI355X).
-// Up to a tile per CU its own pipeline bounds it (more CUs at work lower the
-// clock a little); beyond, two share a CU, and from about 1.1 PFLOP/s on the
-// chip as a whole does.
-double step_us(bool i8, int tile, int n, int ncu) {
-    switch (tile) {
-        case kTile128:
-            if (n <= ncu) return i8 ? 0.8 + 0.0012 * n : 0.85 + 0.0017 * n;
-            return std::max(1.85, (i8 ? 0.0037 : 0.0039) * n);
-        case kTile256:
-            if (n <= ncu) return i8 ? 1.15 + 0.0025 * n : 1.5 + 0.0024 * n;
-            return std::max(i8 ? 3.2 : 3.25, (i8 ? 0.0075 : 0.008) * n);
-        default: return std::max(i8 ? 2.2 : 2.35, (i8 ? 0.0139 : 0.0152) * n);
-    }
+// Time (us) of one 128-k step of n workgroup tiles that run at once, a1 + b1 n
+// on at most one per CU, else (two share a CU) a2 + b2 n, and what a tile's
+// start and end take beyond a 128-column one's. Fitted to 1900 drawn calls of
+// 33-2048 rows, one weight and two, each with every tile (MI355X, cold weights:
+// within 5% rms). Groups of 64 take twice the scale loads and conversions of a
+// step, the more per wave the wider the tile.
+struct StepCost {
+    double start, a1, b1, a2, b2, round;  // round: a further round's start and end, less what overlaps
+};
+enum Family { kGroups = 0, kGroups64 = 1, kInt8 = 2 };
+constexpr StepCost kStep[3][3] = {
+    {{0.0, 0.865, 0.0008, 1.14, 0.0015, 0.0}, {2.4, 1.43, 0.0020, 2.13, 0.0024, -3.6}, {3.0, 2.09, 0.0037, 0, 0, 3.9}},
+    {{0.0, 0.966, 0.0006, 1.15, 0.0016, -2.5}, {2.6, 1.83, 0.0011, 2.42, 0.0022, -7.0}, {3.3, 2.56, 0.0027, 0, 0, 1.6}},
+    {{0.0, 0.81, 0.0010, 1.05, 0.0017, -0.3}, {2.8, 1.15, 0.0016, 2.2, 0.0020, -2.0}, {3.1, 1.95, 0.0025, 0, 0, 3.5}},
+};
+
+// n tiles of kps steps in rounds of as many as fit the chip (two 128- or
+// 256-column workgroups per CU, one of 512), the last one smaller. !vec: C
+// written element by element (13 us a round of 256 or 512 columns).
+double tiles_us(Family fam, int tile, long long n, int kps, int ncu, bool vec) {
+    const StepCost &c = kStep[fam][tile];
+    const int slots = tile == kTile512 ? ncu : 2 * ncu, rest = (int)(n % slots);
+    auto step = [&](int t) { return t <= ncu ? c.a1 + c.b1 * t : c.a2 + c.b2 * t; };
+    const int rounds = (int)(n / slots) + (rest > 0);
+    double us = c.start + kps * ((n / slots) * step(slots) + (rest ? step(rest) : 0.0)) + (rounds - 1) * c.round;
+    if (!vec) us += rounds * (tile == kTile128 ? 6.5 : 13.0);
+    return us;
 }
+
+// A split's reduction: its launch, S f32 partials of C written and read, less
+// C's own way.
+double split_us(Family fam, int S, double MN) { return S > 1 ? (fam == kInt8 ? 2.3 : 3.1) + 1e-6 * (2 * S - 1) * MN : 0.0; }
 
 struct GemmPlan {
     int tile;
     Split sp;
+    double us;  // tiles and reduction
 };
 
-// The workgroup tile and the K splits with the least estimated time: rounds of
-// as many tiles as fit the chip (two 128- or 256-column workgroups per CU, one
-// of 512), the last one smaller; a split adds its reduction, S f32 partials
-// of C written and read. At most kMaxSplit splits of an even number of at
-// least 4 K tiles, within the workspace left after A'. GEMM_CB forces the tile
-// (1, 2, 3), GEMM_NO_SPLIT = 1 no split.
-// Before (128 columns up to a 256-column tile per CU, then 256; splits
-// whenever tiles filled half the CUs or less) and now, us with the pre-pass:
-// 512 rows 2560 x 19456 72 -> 60, 768 rows 83 -> 77, 1024 rows 4096 x 14336
-// 122 -> 114, 2048 rows 237 -> 225, 512 rows 2048 x 2560 25 -> 20.
-GemmPlan plan_gemm(st_context *ctx, bool i8, int M, int K, int N, size_t ws_used, bool split = true) {
-    const int ncu = ctx->num_cus, ntiles = K / KT;
+// The tile with the least estimated time for `weights` of K x N in one grid, K
+// in S splits of kps steps.
+GemmPlan best_tile(const st_context *ctx, Family fam, int M, int N, int weights, int S, int kps, bool vec) {
     const int force = st::tune(ctx, ST_TUNE_GEMM_CB, 0);
-    const int smax = !split || st::tune(ctx, ST_TUNE_GEMM_NO_SPLIT, 0) == 1 ? 1 : std::min(kMaxSplit, ntiles / 4);
-    const size_t off = (ws_used + 255) & ~size_t(255);
-    GemmPlan best{kTile128, {1, ntiles, nullptr}};
-    double least = 1e30;
+    GemmPlan best{kTile128, {S, kps, nullptr}, 1e30};
     for (int tile = kTile128; tile <= kTile512; ++tile) {
         if (force >= 1 && force <= 3 && tile != force - 1) continue;
-        const int T = tile_count(M, N, tile), slots = tile == kTile512 ? ncu : 2 * ncu;
-        for (int s = 1; s <= std::max(1, smax); ++s) {
-            if (s > 1 && off + (size_t)s * M * N * sizeof(float) > ctx->ws_bytes) break;
-            int kps = (ntiles + s - 1) / s;
-            if (s > 1) kps += kps & 1;
-            const int S = (ntiles + kps - 1) / kps;
-            if (S != s) continue;
-            const long long n = (long long)T * S;
-            double us = kps * ((n / slots) * step_us(i8, tile, slots, ncu) + (n % slots ? step_us(i8, tile, (int)(n % slots), ncu) : 0.0));
-            if (S > 1) us += 3.0 + 2e-6 * S * M * N;
-            if (us < least) {
-                least = us;
-                best.tile = tile;
-                best.sp = Split{S, kps, S > 1 ? reinterpret_cast<float *>(reinterpret_cast<char *>(ctx->ws) + off) : nullptr};
-            }
+        const double us = tiles_us(fam, tile, (long long)weights * tile_count(M, N, tile) * S, kps, ctx->num_cus, vec || S > 1) +
+                          split_us(fam, S, (double)weights * M * N);
+        if (us < best.us) {
+            best.us = us;
+            best.tile = tile;
         }
+    }
+    return best;
+}
+
+constexpr double kPreUs = 8.0;  // a GEMM call's launches
+
+// The workgroup tile and the K splits of one weight's call with the least
+// estimated time: at most kMaxSplit splits of an even number of at least 4 K
+// tiles, their partials within `ws` bytes of workspace. GEMM_CB forces the tile
+// (1, 2, 3), GEMM_NO_SPLIT = 1 no split. Nothing depends on addresses.
+// pairs: a gate/up call of such weights has the results of two single calls and
+// so their splits, but twice the tiles to fill the chip with. Neither is split
+// where a single call loses less than three tenths of what the gate/up call gains
+// by it (of weights that widen, N >= K, as an MLP's gate and up do).
+// Against 128 columns up to a 256-column tile per CU, then 256, and splits
+// whenever tiles filled half the CUs or less (drawn calls, cold weights): one
+// weight, 257-2048 rows, 0.94 of the time (300 calls, at most 1 of them above
+// 1.05), silu(a) b 0.92, gate/up 0.91 (600, at most 2), INT8 33-1024 rows 0.97.
+GemmPlan plan_gemm(const st_context *ctx, Family fam, int M, int K, int N, bool f16out, bool pairs, size_t ws) {
+    const int ntiles = K / KT;
+    const int smax = st::tune(ctx, ST_TUNE_GEMM_NO_SPLIT, 0) == 1 ? 1 : std::min(kMaxSplit, ntiles / 4);
+    const bool vec = N % (f16out ? 8 : 4) == 0;
+    const GemmPlan whole = best_tile(ctx, fam, M, N, 1, 1, ntiles, vec);
+    GemmPlan best = whole;
+    for (int s = 2; s <= smax && (size_t)s * M * N * sizeof(float) <= ws; ++s) {
+        int kps = (ntiles + s - 1) / s;
+        kps += kps & 1;
+        if ((ntiles + kps - 1) / kps != s) continue;
+        const GemmPlan p = best_tile(ctx, fam, M, N, 1, s, kps, vec);
+        if (p.us < best.us) best = p;
+    }
+    if (pairs && N >= K && best.sp.S > 1) {
+        const double two = best_tile(ctx, fam, M, N, 2, 1, ntiles, vec).us;
+        const double two_split = best_tile(ctx, fam, M, N, 2, best.sp.S, best.sp.kps, vec).us;
+        if ((kPreUs + whole.us) / (kPreUs + best.us) - 1 < 0.3 * ((kPreUs + two_split) / (kPreUs + two) - 1)) return whole;
     }
     return best;
 }
@@ -789,15 +825,32 @@ struct GptqOperand {
 };
 
 // Calls that the skinny kernel takes (i4xs.hpp, tiled weights): up to 160
-// tokens, and up to 256 on weights of at most 2^24 values, whose GEMM is mostly
-// its launches (pre-pass, tiles, split-K reduction). GEMM / skinny, us in a
-// graph with cold weights (MI355X): 33 tokens 4096 x 4096 16.5 / 8.5, 4096 x
-// 14336 27.8 / 17.1, 11008 x 4096 26.5 / 17.4; 128 tokens 24.8 / 11.2, 33.7 /
-// 27.5, 30.8 / 27.4; 160 tokens 25.6 / 16.7, 46.3 / 38.6, 41.6 / 38.3; 256
-// tokens 30.9 / 18.5, 47.0 / 46.4, 44.2 / 53.4.
-bool use_skinny(const st_context *ctx, int M, int K, int N, uint32_t flags) {
-    return (flags & ST_FLAG_TILED) && (M <= 160 || (M <= 256 && (long long)K * N <= (1 << 24))) &&
-           st::tune(ctx, ST_TUNE_GEMM_CB, -1) < 0 && st::tune(ctx, ST_TUNE_GEMM_NO_SPLIT, -1) < 0;
+// tokens, and up to 256 on weights of at most 2^24 values, from 65 on where its
+// estimate (int4_xs_us) is below the GEMM's with its pre-pass. A gate/up call has
+// the results of two single calls, so the rule is one for both: the GEMM also
+// takes weights that widen (N >= K, as an MLP's gate and up do) where it is
+// estimated to be faster for two of them, whose tiles fill the chip better, and
+// to lose less than three tenths of that for one.
+// us by the bounds alone / now / on the GEMM before the skinny kernel, gate/up:
+// 124 tokens 4864 x 11248 90 / 51 / 64, 139 tokens 4608 x 11968 115 / 72 / 74,
+// 160 tokens 2560 x 9728 45 / 40 / 42. In each of four draws of 600 gate/up calls
+// of 33-420 tokens 10-15 are left that run 5-50% longer than on that GEMM (131
+// tokens 1792 x 10856 54 / 47 / 33, 217 tokens 1024 x 12464 42 / 39 / 26): 130-256
+// tokens against short and very wide weights, whose single calls are far faster
+// on the skinny kernel. Of 600 single calls 1-3.
+bool use_skinny(const st_context *ctx, const st::XsCall &x, uint32_t flags, const GemmPlan &pl, Family fam) {
+    if (!(flags & ST_FLAG_TILED) || x.M > 256 || (x.M > 160 && (long long)x.K * x.N > (1 << 24)) ||
+        st::tune(ctx, ST_TUNE_GEMM_CB, -1) >= 0 || st::tune(ctx, ST_TUNE_GEMM_NO_SPLIT, -1) >= 0)
+        return false;
+    if (x.M <= 64) return true;
+    const double MK = (double)x.M * x.K, MN = (double)x.M * x.N, pre = kPreUs + 0.9e-6 * MK;
+    double pre_xs;
+    const double xs = st::int4_xs_us(ctx, x, &pre_xs), g = pre + pl.us + 0.6e-6 * MN;
+    if (x.xb) return pre_xs + xs < g + 6.7 + 1.2e-6 * MK;
+    if (g < pre_xs + xs) return false;
+    if (x.N < x.K) return true;
+    const double pair = pre + best_tile(ctx, fam, x.M, x.N, 2, pl.sp.S, pl.sp.kps, true).us + 1.2e-6 * MN;
+    return g / (pre_xs + xs) - 1 >= 0.3 * ((pre_xs + 2 * xs) / pair - 1);
 }
 
 // The prefill GEMM behind the entry points: u == NULL for a . dequant(W),
@@ -828,9 +881,12 @@ int gemm_impl(const char *fn, st_context *ctx, const uint16_t *a, const uint16_t
         return st::fail(ST_ERR_WORKSPACE, "%s: needs %zu B of workspace for A (st_context_reserve_workspace)", fn,
                         need);
     if (perm && !st::aligned16(perm)) return st::fail(ST_ERR_ALIGN, "%s: perm must be 16-byte aligned", fn);
-    if (use_skinny(ctx, M, K, N, flags)) {
-        st::XsCall x{a, u, true, perm, {qweight, nullptr}, {scales, nullptr}, {qzeros, nullptr},
-                     (flags & ST_FLAG_ZEROS_PLUS_ONE) ? 1 : 0, c, c_dtype == ST_F16, M, K, N, group_size, 1, true};
+    const Family fam = group_size == 64 ? kGroups64 : kGroups;
+    const size_t off = (need + 255) & ~size_t(255), left = off < ctx->ws_bytes ? ctx->ws_bytes - off : 0;  // (for partials)
+    GemmPlan pl = plan_gemm(ctx, fam, M, K, N, c_dtype == ST_F16, !u, left);
+    st::XsCall x{a, u, true, perm, {qweight, nullptr}, {scales, nullptr}, {qzeros, nullptr},
+                 (flags & ST_FLAG_ZEROS_PLUS_ONE) ? 1 : 0, c, c_dtype == ST_F16, M, K, N, group_size, 1, true};
+    if (use_skinny(ctx, x, flags, pl, fam)) {
         int rc = st::int4_xs(ctx, x);
         if (rc == ST_OK && w1) {
             x.qw[0] = w1->qweight;
@@ -853,19 +909,16 @@ int gemm_impl(const char *fn, st_context *ctx, const uint16_t *a, const uint16_t
         return (flags & ST_FLAG_TILED) ? launch_tiled<true>(ctx, ga, group_size, tile, sp)
                                        : launch_tiled<false>(ctx, ga, group_size, tile, sp);
     };
-    const GemmPlan pl = plan_gemm(ctx, false, M, K, N, need);
-    // Both weights' tiles in one grid when one weight's alone does not split
-    // K (the partials are laid out for one C, and a split changes the order
-    // of the f32 sums, so the results would no longer be those of
-    // st_gptq_i4_gemm); otherwise two launches on A.
-    if (w1 && pl.sp.S == 1) {
-        const GemmPlan pl2 = plan_gemm(ctx, false, M, K, 2 * N, need, false);
+    if (pl.sp.S > 1) pl.sp.part = reinterpret_cast<float *>(reinterpret_cast<char *>(ctx->ws) + off);
+    // Both weights' tiles in one grid, if their partials fit; else two launches
+    // on A.
+    if (w1 && (pl.sp.S == 1 || (size_t)2 * pl.sp.S * M * N * sizeof(float) <= left)) {
         GemmArgs g2 = g;
         g2.qw1 = w1->qweight;
         g2.sc1 = w1->scales;
         g2.qz1 = w1->qzeros;
         g2.C1 = w1->c;
-        return run(g2, pl2.tile, pl2.sp);
+        return run(g2, best_tile(ctx, fam, M, N, 2, pl.sp.S, pl.sp.kps, true).tile, pl.sp);
     }
     if (int rc = run(g, pl.tile, pl.sp)) return rc;
     if (!w1) return ST_OK;
@@ -918,6 +971,7 @@ extern "C" int st_int8_gemm(st_context *ctx, const uint16_t *a, const int8_t *w,
         return st::fail(ST_ERR_SHAPE, "%s: a or w above 2 GiB (M=%d K=%d N=%d); split M or N", fn, M, K, N);
     const GemmArgs g{reinterpret_cast<const _Float16 *>(a), reinterpret_cast<const uint32_t *>(w), nullptr, nullptr, 0,
                      nullptr, scale, c, c_dtype == ST_F16, M, K, N};
-    const GemmPlan pl = plan_gemm(ctx, true, M, K, N, 0);
+    GemmPlan pl = plan_gemm(ctx, kInt8, M, K, N, g.f16out, false, ctx->ws_bytes);
+    if (pl.sp.S > 1) pl.sp.part = ctx->ws;
     return tiled ? launch_gs<128, true, true>(ctx, g, pl.tile, pl.sp) : launch_gs<128, false, true>(ctx, g, pl.tile, pl.sp);
 }

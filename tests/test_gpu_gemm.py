@@ -326,3 +326,52 @@ def test_gate_up_gemm_graph_replay(gpu, orc, route):
         assert torch.equal(og, eg) and torch.equal(ou, eu), f"replay {i}"
         call(eg, eu)  # eager work between
         torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("Mr,K,N,gs,act,pair", [
+    (64, 1024, 9000, 128, False, "i4xs_kernel"),     # up to 64 tokens: the skinny kernel
+    (77, 2560, 9728, 128, False, "i4xs_kernel"),
+    (124, 4864, 11248, 256, False, "gemm_kernel"),   # the GEMM's grid of both weights is the faster one
+    (139, 4608, 11968, 128, True, "gemm_kernel"),
+    (150, 4608, 1048, 64, True, "i4xs_kernel"),      # weights that narrow: by one alone
+    (256, 1024, 1032, 128, False, "i4xs_kernel"),
+    (161, 5120, 5952, 128, False, "gemm_kernel"),    # above 160 tokens and 2^24 values
+    (257, 1024, 1032, 128, False, "gemm_kernel"),
+])
+def test_gate_up_takes_the_kernel_of_single_calls(gpu, Mr, K, N, gs, act, pair):
+    """One rule for both kinds of call, on both sides of its lines: a gate/up
+    call takes the kernel of a single call, and gives its bits."""
+    g = torch.Generator(device="cuda").manual_seed(Mr)
+    qw = [torch.randint(-2**31, 2**31, (sta.lib().st_gptq_i4_tiled_words(K, N, gs),), dtype=torch.int32, device="cuda", generator=g)
+          for _ in range(2)]
+    sc = [(torch.rand(K // gs, N, device="cuda", generator=g) * 0.01).half() for _ in range(2)]
+    qz = torch.randint(-2**31, 2**31, (K // gs, N // 8), dtype=torch.int32, device="cuda", generator=g)  # (up's: gate has none)
+    perm = torch.randperm(K, device="cuda", generator=g).int() if act else None
+    a = torch.randn(Mr, K, device="cuda", generator=g).half()
+    y = [torch.full((Mr, N), float("nan"), device="cuda") for _ in range(4)]
+    launches()
+    M.gate_up_gemm(gpu, a, qw[0], sc[0], qw[1], sc[1], y[0], y[1], K, N, gs, up_qz=qz, perm=perm, flags=2)
+    ran = launches()
+    for i in range(2):
+        M.gptq_gemm(gpu, a, qw[i], sc[i], y[2 + i], K, N, gs, (None, qz)[i], perm, 2)
+    torch.cuda.synchronize()
+    assert {"gemm_kernel", "i4xs_kernel"} & set(ran) == {pair} == {"gemm_kernel", "i4xs_kernel"} & set(launches())
+    assert torch.equal(y[0], y[2]) and torch.equal(y[1], y[3])
+
+
+@pytest.mark.parametrize("out", [torch.float32, torch.float16])
+@pytest.mark.parametrize("Mr,K,N,gs", [(300, 4096, 264, 128), (129, 8192, 1032, 64), (700, 2048, 136, 256)])
+def test_gate_up_gemm_splits_in_one_grid(gpu, orc, Mr, K, N, gs, out, tune):
+    """Where a single call splits K, both weights' splits are one grid and one
+    reduction, of which either weight's half is a single call's."""
+    tune(GEMM_CB=0)
+    cg = orc.gptq_case(800 + Mr, K, N, gs, zeros=True, M=Mr, x_dtype=np.float16)
+    cu = orc.gptq_case(900 + Mr, K, N, gs)
+    wg, wu = up(gpu, cg), up(gpu, cu)
+    launches()
+    yg, yu = run_gate_up(gpu, wg, wu, cg["x"], out)
+    assert launches() == ["prep_a_kernel", "gemm_kernel", "splitk_reduce_kernel"]
+    np.testing.assert_array_equal(yg, run_gemm(gpu, wg, cg["x"], out))
+    np.testing.assert_array_equal(yu, run_gemm(gpu, wu, cg["x"], out))
+    assert "splitk_reduce_kernel" in launches()
+    assert orc.rel_l2(yu, orc.gptq_matvec_f64(cg["x"], cu["qweight"], cu["scales"], K, N, gs)) < 5e-4

@@ -13,6 +13,7 @@ import torch
 
 import shady_thinker_amd as sta
 from shady_thinker_amd import model as M
+from shady_thinker_amd._lib import launches
 
 pytestmark = pytest.mark.gpu
 
@@ -152,3 +153,16 @@ def test_int8_gemm_split_k_matches_unsplit(gpu, orc, tune):
     ref = orc.int8_matvec_f64(c["x"], c["w"], c["scale"], K, N)
     assert orc.rel_l2(y_split, ref) < TIGHT and orc.rel_l2(y_one, ref) < TIGHT
     assert orc.rel_l2(y_split, y_one) < 1e-6
+
+
+@pytest.mark.parametrize("Mr,N,split", [(170, 2188, True), (170, 2184, False), (773, 804, True)])
+def test_int8_gemm_unaligned_rows_split(gpu, orc, Mr, N, split):
+    """f16 C with N no multiple of 8: written element by element a tile costs
+    more than a split's reduction, whose partials' rows are aligned."""
+    K = 1152
+    c = orc.int8_case(60 + N, K, N, M=Mr)
+    w = sta.Int8Weight.upload(gpu, c["w"], c["scale"])
+    launches()
+    y = run(gpu, w, c["x"], torch.float16)
+    assert split == ("splitk_reduce_kernel" in launches())
+    assert orc.rel_l2(y, orc.int8_matvec_f64(c["x"], c["w"], c["scale"], K, N)) < 2.0**-11
