@@ -74,37 +74,49 @@ __global__ __launch_bounds__(256) void repack8_kernel(const int8_t *__restrict__
 //     11008 x 4096                   10.6 / 11.6             13.6 / 12.1
 //     silu(a) b, 4096 x 4096          8.4 /  9.3              9.9 /  9.6
 //     act-order 4096 x 4096          14.4 /  9.7             13.1 /  9.9
-//     act-order 4096 x 4096 2 tokens  7.9 /  9.5
 //   wide: 2560 x 151936     4 tokens 39   / 42     5 tokens 77   / 42
-// so from 5 tokens on, with act-order on narrow linears from 3 (the limb
-// kernels gather x in every workgroup); narrow linears with K below 2048 keep
-// the limb kernels to 8 tokens.
+// so from 5 tokens on; narrow linears with K below 2048 keep the limb kernels to
+// 8 tokens. Under act-order the limb kernels gather x in every workgroup, which
+// 3 and 4 tokens of a long x make dearer than the skinny kernel's gather launch
+// (narrow linears drawn, limb / skinny: 3 tokens, K 1024-2600 0.86, to 4200 0.91,
+// above 1.17; 4 tokens 0.92, 1.05, 1.31): there from M K = 3 x 4096, silu(a) b
+// from 3 tokens (1.1-4.1).
 constexpr int kF16MinM = 5;
 constexpr int kF16MinMActOrder = 3;
+constexpr int kF16MinMKActOrder = 3 * 4096;
 constexpr int kF16MinMShortK = 9;
 constexpr int kF16ShortK = 2048;
 
-// Wide linears whose tokens fill 16 MFMA rows or less (8 tokens of f32 x, 16
-// of f16): i4mm.hip, except for one source of at least 3 tiles per CU (8
-// tokens of f32 x, i4mm / i4xs: 2560 x 10240 7.5 / 8.4 us, gate/up 2560 x
-// 9728 9.8 / 11.8, gate/up 4096 x 11008 13.6 / 14.5; 4096 x 14336 12.9 / 11.3,
-// 2560 x 151936 53.8 / 43.3), and of at most 2 in groups of 64 with f32 x,
-// where i4mm's 8-byte weight loads hold too little in flight (6 tokens: 1024 x
-// 6144 5.5 / 5.2, 4096 x 4160 11.7 / 8.9, 4096 x 8000 12.0 / 10.2, 8192 x 6144
-// 19.8 / 12.4, 4096 x 6144 with zeros and act-order 14.8 / 12.4; at 2.5 tiles
-// per CU 4096 x 10240 10.5 / 11.6; f16 x, 4096 x 6144, 11.4 / 15.0; group 128,
-// 4096 x 6144, 8.0 / 9.2). Above 16 rows i4xs took every shape measured.
+// Wide linears whose tokens fill 16 MFMA rows or less (8 tokens of f32 x, 16 of
+// f16): i4mm.hip for gate/up (8 tokens of f32 x, i4mm / i4xs: 2560 x 9728 9.8 /
+// 11.8 us, 4096 x 11008 13.6 / 14.5) and for one source by its tiles per CU (i4mm
+// time over i4xs's, 400 drawn calls of 5-16 tokens, f32 x / f16 x):
+//   below 3    2560 x 10240 7.5 / 8.4 us; but in groups of 64 with f32 x and at
+//              most 2, where i4mm's 8-byte weight loads hold too little in
+//              flight, i4xs (6 tokens: 4096 x 8000 12.0 / 10.2, 8192 x 6144
+//              19.8 / 12.4; 4096 x 10240, 2.5 per CU, 10.5 / 11.6)
+//   3 to 4     1.06 / 1.04 (in groups of 256 0.94 / 0.97): i4xs
+//   4 to 6     0.93 / 0.87
+//   6 to 8     0.98 / 0.88
+//   above      1.30 / 1.15: more tiles than i4mm's workgroups take at once
+// From 9 tokens of f32 x and 17 of f16 on i4xs is the faster one of the two in
+// most shapes, not in all (f16 x of 17-32 tokens on 2-8 tiles per CU: 40 of 226
+// drawn calls ran 4-30% faster on a two-row-block i4mm, which is gone).
 bool use_i4mm(const st_context *ctx, const QmvParams &p, int ntiles, int nsrc, int xm) {
-    if (xm == XM_SILU || ntiles <= ctx->num_cus || p.M > (xm == XM_F32 ? 8 : 16)) return false;
+    const int ncu = ctx->num_cus;
+    if (xm == XM_SILU || ntiles <= ncu || p.M > (xm == XM_F32 ? 8 : 16)) return false;
     if (nsrc == 2) return true;
-    return ntiles < 3 * ctx->num_cus && !(xm == XM_F32 && p.gs == 64 && ntiles <= 2 * ctx->num_cus);
+    if (ntiles < 3 * ncu) return !(xm == XM_F32 && p.gs == 64 && ntiles <= 2 * ncu);
+    return ntiles > 4 * ncu && ntiles <= (xm == XM_F32 ? 6 : 8) * ncu;
 }
 
 // -1: not taken.
 int launch_f16(st_context *ctx, const QmvParams &p, bool tiled, int nsrc, int xm) {
     const int ntiles = (p.N + kTileN - 1) / kTileN;
     const bool few = ntiles <= ctx->num_cus;
-    const int dflt = !few ? kF16MinM : p.perm ? kF16MinMActOrder : p.K < kF16ShortK ? kF16MinMShortK : kF16MinM;
+    int dflt = kF16MinM;
+    if (few && !p.perm && p.K < kF16ShortK) dflt = kF16MinMShortK;
+    if (few && p.perm && (xm == XM_SILU || (long long)p.M * p.K >= kF16MinMKActOrder)) dflt = kF16MinMActOrder;
     const int min_m = std::max(2, st::tune(ctx, ST_TUNE_I4MM_MIN_M, dflt));
     const int min_tiles = st::tune(ctx, ST_TUNE_I4MM_MIN_TILES, ctx->num_cus + 1);
     const bool split = few && st::tune(ctx, ST_TUNE_I4MM_SPLIT_TILES, 1) > 0;
@@ -129,12 +141,11 @@ int launch_i4(st_context *ctx, QmvParams &p, bool tiled, int nsrc, int xm) {
     return p.perm ? dispatch<FMT_I4, true>(ctx, p, nsrc, xm) : dispatch<FMT_I4, false>(ctx, p, nsrc, xm);
 }
 
-// Calls with more than kTokenBlock tokens run as blocks of kTokenBlock: the
-// per-wave staging of the multi-token kernels grows with M * K per wave, and
-// at 32 tokens two blocks of 16 (or eight of 4) measured several times
-// faster than one launch, even though every block streams the weights again.
-// (A skinny-GEMM kernel that reuses the weights across blocks is the better
-// design for M > 4.)
+// Calls with more than kTokenBlock tokens that no f16-MFMA kernel takes run as
+// blocks of kTokenBlock: the per-wave staging of the limb kernels grows with
+// M * K per wave, and at 32 tokens two blocks of 16 (or eight of 4) measured
+// several times faster than one launch, even though every block streams the
+// weights again.
 constexpr int kTokenBlock = 16;
 
 // Fewest tokens for which st_int8_matvec takes the f16-MFMA kernel (f16 x, tiled weights).
@@ -209,10 +220,11 @@ int st_gptq_i4_matvec_noalloc(st_context *ctx, const void *x, int x_dtype, const
                               int K, int N, int group_size, uint32_t flags) {
     if (!ctx) return st::fail(ST_ERR_INVALID, "st_gptq_i4_matvec_noalloc: ctx is NULL");
     if (!ctx->scratch) return st::fail(ST_ERR_WORKSPACE, "st_gptq_i4_matvec_noalloc: no scratch on this device");
-    // The most any path of the call keeps: the f16-MFMA kernel's split of up
-    // to 32 tokens of f32 x (one launch; 2 f16 rows per token and a factor per 128 k)
-    // or, for f16 x under act-order, its gathered rows; split-K partials
-    // shrink (or go unsplit) to fit what is there.
+    // The most any path of the call keeps: i4mm's pre-pass rows of f32 x (2 f16
+    // rows per token and a factor per 128 k; the skinny kernel's gathered f32 x
+    // is smaller) or, for f16 x under act-order, the gathered rows. f32 x without
+    // act-order keeps none of it unless I4MM_PREPASS is set, but is held to the
+    // same limit. Split-K partials shrink (or go unsplit) to fit what is there.
     if (M > 0 && K > 0 && (x_dtype == ST_F32 || perm)) {
         // (f16 x under act-order: the gathered rows, mb K halves)
         const size_t mb = (size_t)std::min(M, 2 * kTokenBlock);

@@ -853,6 +853,8 @@ def _gate_up(gpu, wg, wu, x, dtype=torch.float32):
     (7, 4096, 4168, 256, True, False, False, "i4mm"),   # group 256, ragged last tile
     (16, 1024, 5000, 128, True, True, False, "i4mm"),   # f16 x: 16 rows
     (3, 256, 12264, 128, False, False, False, "i4mm"),  # 767 tiles: three per workgroup
+    (6, 384, 24568, 128, True, False, False, "i4mm"),   # 1536 tiles: six per workgroup, ragged
+    (11, 384, 32760, 64, True, True, False, "i4mm"),    # f16 x, 2048 tiles: eight per workgroup, ragged
     (8, 2560, 9728, 128, False, False, True, "i4mm"),   # gate/up at batch 8
     (6, 1536, 4232, 64, True, True, True, "i4mm"),      # gate/up, f16 x, zeros, group 64, ragged
     (4, 256, 16408, 128, True, False, True, "i4mm"),    # gate/up, 1026 tile pairs: more workgroups than CUs
@@ -1018,6 +1020,12 @@ def test_int4_mm_f16_act_order(gpu, orc, Mr, K, N, gs, zeros, f16, dual, tune):
     (17, 1024, 4112, 128, False, False, True, "i4xs"),
     (8, 1024, 12272, 128, False, False, False, "i4mm"),  # 767 tiles: below 3 per CU
     (8, 1024, 12280, 128, False, False, False, "i4xs"),  # 768 (the last one ragged)
+    (8, 512, 16384, 128, False, False, False, "i4xs"),   # 1024: 4 per CU
+    (8, 512, 16392, 128, False, False, False, "i4mm"),   # 1025
+    (8, 256, 24576, 128, False, False, False, "i4mm"),   # 1536: 6 per CU
+    (8, 256, 24584, 128, False, False, False, "i4xs"),
+    (16, 256, 32768, 128, False, False, True, "i4mm"),   # f16 x: 8 per CU
+    (16, 256, 32776, 128, False, False, True, "i4xs"),
     (8, 1024, 8192, 64, False, False, False, "i4xs"),    # groups of 64 with f32 x: i4mm only above 2 per CU
     (8, 1024, 8200, 64, False, False, False, "i4mm"),
     (8, 1024, 8192, 64, False, False, True, "i4mm"),
@@ -1028,8 +1036,12 @@ def test_int4_mm_f16_act_order(gpu, orc, Mr, K, N, gs, zeros, f16, dual, tune):
     (8, 1024, 4096, 128, False, False, False, "qmv"),    # K below 2048: the limb kernels to 8 tokens
     (5, 2048, 4096, 128, False, False, False, "i4xs"),   # else to 4
     (4, 2048, 4096, 128, False, False, False, "qmv"),
-    (3, 2048, 4096, 128, True, False, False, "i4xs"),    # act-order: to 2
-    (2, 2048, 4096, 128, True, False, False, "qmv"),
+    (3, 4096, 1024, 128, True, False, False, "i4xs"),    # act-order: from 3 with M K >= 12288
+    (3, 3968, 1024, 128, True, False, False, "qmv"),
+    (4, 3072, 1024, 128, True, False, False, "i4xs"),
+    (4, 2944, 1024, 128, True, False, False, "qmv"),
+    (2, 8192, 1024, 128, True, False, False, "qmv"),
+    (5, 1024, 1024, 128, True, False, False, "i4xs"),
 ])
 def test_int4_mm_f16_default_routing(gpu, orc, Mr, K, N, gs, act, dual, f16, kernel, tune):
     """Which kernel the GPTQ entry points pick by default on an MI355X (256
