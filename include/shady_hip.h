@@ -111,7 +111,7 @@ typedef enum {
     ST_TUNE_NO_KSPLIT,         /* 1: no split-K of several-token decode on few tiles */
     ST_TUNE_SPLIT_TILES_CU,    /* several-token decode: split K up to this many tiles per CU */
     ST_TUNE_TOKEN_BLOCK,       /* decode: tokens per launch (1..16) */
-    ST_TUNE_I4MM_MIN_M,        /* GPTQ decode: fewest tokens for the f16-MFMA kernels (default 5; on at most one tile per CU 3 with act-order, 9 with K below 2048) */
+    ST_TUNE_I4MM_MIN_M,        /* GPTQ decode: fewest tokens for the f16-MFMA kernels (default 5; on at most one tile per CU 9 with K below 2048, 3 under act-order with M K of 12288 or silu(a) b) */
     ST_TUNE_I4MM_MIN_TILES,    /* GPTQ decode: fewest 16-column tiles for the f16-MFMA kernels */
     ST_TUNE_I8MM_MIN_M,        /* INT8 decode: fewest tokens for the f16-MFMA kernel */
     ST_TUNE_GEMM_CB,           /* prefill GEMM: workgroup tile of 128 (1), 256 (2) or 512 (3) columns; set, the skinny kernel takes no GEMM call */
@@ -183,14 +183,16 @@ int st_flush(st_context *ctx);
  * Requires K % group_size == 0, group_size in {64, 128, 256}, N % 8 == 0,
  * 1 <= M <= 32, 16-byte aligned qweight and x. Accumulation: exact integer
  * products of the nibbles with a 3 x 8-bit split of x scaled by a power of
- * two per group, f32 across groups (rel-L2 vs f64 ~1e-7). From 5 tokens on
- * tiled weights (with at most one 16-column tile per CU from 3 under perm and
- * from 9 with K below 2048; then K may be split across workgroups, partial sums in the
- * context workspace): f16 MFMA on exact (q - z) and x (f16 x as is; f32 x
- * scaled by a power of two and split into two f16 parts; with perm x is
- * gathered into the context workspace first), f32
- * sums, rel-L2 vs f64 ~1e-7, the weights read once for up to 32 tokens. The
- * same rule applies to st_gptq_i4_gate_up_silu. */
+ * two per group, f32 across groups (rel-L2 vs f64 ~3e-7). From 5 tokens on
+ * tiled weights (with at most one 16-column tile per CU from 9 with K below
+ * 2048, and from 3 under perm with M K of 12288 at least): f16 MFMA on exact
+ * (q - z) and x (f16 x as is; f32 x scaled by a power of two per token and at
+ * most 512 k and split into two f16 parts, together 22 bits, whose products are
+ * summed apart within a group), f32 sums; rel-L2 vs f64 of f32 x 0.8e-7 to
+ * 1.7e-7, the weights read once for up to 32 tokens. K may be split across
+ * workgroups, with partial sums in the context workspace, where x gathered under
+ * perm comes first. The same rule applies to st_gptq_i4_gate_up_silu, and but for
+ * the last condition to st_gptq_i4_silu_matvec (from 3 tokens under perm). */
 int st_gptq_i4_matvec(st_context *ctx, const void *x, int x_dtype,
                       const uint32_t *qweight, const uint16_t *scales,
                       const uint32_t *qzeros, const int32_t *perm, float *y,
@@ -199,16 +201,16 @@ int st_gptq_i4_matvec(st_context *ctx, const void *x, int x_dtype,
 /* No counterpart in the reference: for callers that cannot allocate device
  * memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc). st_gptq_i4_matvec with everything its kernels keep
- * beyond the inputs and outputs (the f16-MFMA kernel's split of f32 x into
- * f16 rows, split-K partial sums) in a fixed array of
+ * beyond the inputs and outputs (x gathered under act-order, as it is or split
+ * into f16 rows, and split-K partial sums) in a fixed array of
  * ST_NOALLOC_SCRATCH_BYTES that the library holds on every GPU it runs on,
  * from the context's creation until the process ends, instead of the
  * context workspace. Allocates nothing. A call whose scratch would exceed
  * the array fails with ST_ERR_WORKSPACE and launches nothing. The check is
- * conservative: for f32 x (and for f16 x under act-order) it counts the
- * f16-MFMA kernel's split rows of one launch, 4 M K + M K / 32 bytes
- * (f16 x with perm: 2 M K), with M capped at 32, whichever kernel the call
- * then takes; split-K partials are not counted (they shrink or go unsplit
+ * conservative: for f32 x (and for f16 x under act-order) it counts two f16
+ * rows per token and a factor per 128 k, 4 M K + M K / 32 bytes (f16 x with
+ * perm: 2 M K), with M capped at 32, whichever kernel the call then takes (f32 x
+ * without perm needs none of it); split-K partials are not counted (they shrink or go unsplit
  * to fit the array). Every call on
  * one GPU shares that GPU's array (nothing in it needs to start at zero;
  * each call overwrites what it reads): calls that overlap on one GPU (other
@@ -278,9 +280,8 @@ int st_bf16_matvec(st_context *ctx, const void *x, int x_dtype, const uint16_t *
 
 /* Prefill GEMM: C[M, N] = A[M, K] . dequant(W), A f16, C in c_dtype (ST_F32
  * or ST_F16). No reference counterpart (the reference prefills token by
- * token, src/inference.rs:93-95). MFMA f16 with integer-valued (q - z)
- * operands, f32 accumulation, per-group scale applied after each group.
- * perm as st_gptq_i4_matvec. */
+ * token, src/inference.rs:93-95). MFMA f16 on weights (q - z) s rounded once to
+ * f16, f32 accumulation (rel-L2 vs f64 ~2e-4). perm as st_gptq_i4_matvec. */
 int st_gptq_i4_gemm(st_context *ctx, const uint16_t *a, const uint32_t *qweight,
                     const uint16_t *scales, const uint32_t *qzeros, const int32_t *perm,
                     void *c, int c_dtype, int M, int K, int N, int group_size,
@@ -288,8 +289,8 @@ int st_gptq_i4_gemm(st_context *ctx, const uint16_t *a, const uint32_t *qweight,
 
 /* Gate and up projections of one MLP for M tokens in one call:
  * c_gate = a . dequant(W_gate) and c_up = a . dequant(W_up), both [M, N],
- * from one pre-processed A and (when no split-K is needed) one launch whose
- * grid holds the tiles of both weights. The M-token form of the gate/up
+ * from one pre-processed A and one launch whose grid holds the tiles of both
+ * weights (short prompts may take a launch for each). The M-token form of the gate/up
  * half of the reference's MLP (src/model.rs:803-811, the separate gate and
  * up matvecs it runs one token at a time); st_gptq_i4_silu_gemm then takes
  * c_gate and c_up for the down projection. Both weights share K, N,

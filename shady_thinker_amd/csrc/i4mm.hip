@@ -30,6 +30,7 @@
 //    chunks of weights, scales and zeros, two in flight while it computes
 //    one. Partial sums meet in LDS in a fixed order.
 #include "common.hpp"
+#include "i4frag.hpp"
 
 #include <algorithm>
 #include <cstdlib>
@@ -37,11 +38,10 @@
 
 namespace {
 
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
+using namespace st::i4;
+
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kWaves = 16;
@@ -50,39 +50,6 @@ constexpr int kTileN = 16;
 constexpr int kRsrcWord3 = 0x00020000;     // raw 32-bit buffer data (gfx9-class)
 constexpr unsigned kNoLoad = 0x80000000u;  // buffer offset past every resource: reads 0, touches no memory
 constexpr int kMaxTilesPerWg = 8;
-
-// v_and_or_b32 with both constants in registers (a VOP3 takes no literal).
-__device__ __forceinline__ unsigned and_or(unsigned a, unsigned m, unsigned c) {
-    unsigned r;
-    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(m), "v"(c));
-    return r;
-}
-
-// GPTQ word (nibbles n0..n7 = k0..k7) -> (n0 - z, n4 - z), (n1 - z, n5 - z),
-// (n2 - z, n6 - z), (n3 - z, n7 - z) in f16, exactly: 1024 + n - (1024 + z),
-// or (1024 + 16 n) / 16 - (64 + z) for the odd nibbles.
-__device__ __forceinline__ half8 word_to_b(unsigned w, half2_t zlo, half2_t zhi) {
-    const unsigned m_lo = 0x000F000Fu, m_hi = 0x00F000F0u, bias = 0x64006400u;
-    const half2_t sixteenth = {(_Float16)0.0625f, (_Float16)0.0625f};
-    const unsigned w8 = w >> 8;
-    const half2_t h0 = __builtin_bit_cast(half2_t, and_or(w, m_lo, bias)) - zlo;
-    const half2_t h1 = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, and_or(w, m_hi, bias)), sixteenth, zhi);
-    const half2_t h2 = __builtin_bit_cast(half2_t, and_or(w8, m_lo, bias)) - zlo;
-    const half2_t h3 = __builtin_elementwise_fma(__builtin_bit_cast(half2_t, and_or(w8, m_hi, bias)), sixteenth, zhi);
-    const u32x4 r = {__builtin_bit_cast(unsigned, h0), __builtin_bit_cast(unsigned, h1), __builtin_bit_cast(unsigned, h2),
-                     __builtin_bit_cast(unsigned, h3)};
-    return __builtin_bit_cast(half8, r);
-}
-
-// 8 halves (k0..k7, as 4 dwords) -> the order of word_to_b: k0,k4,k1,k5,k2,k6,k3,k7.
-__device__ __forceinline__ u32x4 to_b_order(u32x4 a) {
-    u32x4 r;
-    r.x = __builtin_amdgcn_perm(a.z, a.x, 0x05040100u);
-    r.y = __builtin_amdgcn_perm(a.z, a.x, 0x07060302u);
-    r.z = __builtin_amdgcn_perm(a.w, a.y, 0x05040100u);
-    r.w = __builtin_amdgcn_perm(a.w, a.y, 0x07060302u);
-    return r;
-}
 
 // 8 f32 x (k0..k7) times 2^-e (|x 2^-e| < 1) -> hi and lo f16 in the
 // order of word_to_b, |x 2^-e - hi - lo| < 2^-20 |x 2^-e| + 2^-24:
@@ -122,11 +89,6 @@ __device__ __forceinline__ int unit_exponent(const float (&v)[8]) {
     m = max(m, dpp_u<0x140>(m));  // row_mirror
     return m ? __builtin_amdgcn_frexp_expf(__uint_as_float(m)) : 0;  // |x| < 2^e
 }
-
-// silu(v) = v / (1 + exp(-v)) (fused_gate_up_silu_4t.wgsl)
-__device__ __forceinline__ float silu_f(float v) { return __fdividef(v, 1.0f + __expf(-v)); }
-
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
 template <int GS>
 struct Unit {  // what a wave loads for one 128-k unit of its tile and source
@@ -547,38 +509,38 @@ int launch_gs(st_context *ctx, const void *x, const float *pe, const uint32_t *c
                        x, pe, qw[0], sc[0], qz[0], qw[1], sc[1], qz[1], zoff, y, M, K, N, ntiles);    \
     } while (0)
 #define ST_I4MM(KCU_, GW_, NW_) ST_I4MM_P(KCU_, GW_, NW_, false)
-        // gate/up with both sources in a wave: wpt is then waves per tile pair
-        if constexpr (NSRC == 2 && GS != 64) {  // (group 64 with two sources per wave spills)
-            if (pair) {
-                if (wpt >= 4)
-                    ST_I4MM_P(4, 1, 12, true);
-                else
-                    ST_I4MM_P(2, 1, 12, true);
-                return st::launch_check("i4mm_kernel");
-            }
-        }
-        // waves per tile and source = 128-k units per chunk (one unit per wave):
-        // 8 (1024-k chunks), 4 or 2. Group size 64 stops at 4: its 8-unit chunk
-        // spilled 30 VGPRs inside the loop (one source, 16 tokens, 2560 x 6144:
-        // 15.5 -> 13.7 us with 4; gate/up unchanged).
-        if constexpr (GS != 64) {
-            if (wpt >= 8) {
-                ST_I4MM(8, 1, 16);
-                return st::launch_check("i4mm_kernel");
-            }
-        }
-        if (wpt >= 4) {
-            if (nw == 12)
-                ST_I4MM(4, 1, 12);
+    // gate/up with both sources in a wave: wpt is then waves per tile pair
+    if constexpr (NSRC == 2 && GS != 64) {  // (group 64 with two sources per wave spills)
+        if (pair) {
+            if (wpt >= 4)
+                ST_I4MM_P(4, 1, 12, true);
             else
-                ST_I4MM(4, 1, 16);
-        } else {
-            if (nw == 12)
-                ST_I4MM(2, 1, 12);
-            else
-                ST_I4MM(2, 1, 16);
+                ST_I4MM_P(2, 1, 12, true);
+            return st::launch_check("i4mm_kernel");
         }
-        return st::launch_check("i4mm_kernel");
+    }
+    // waves per tile and source = 128-k units per chunk (one unit per wave):
+    // 8 (1024-k chunks), 4 or 2. Group size 64 stops at 4: its 8-unit chunk
+    // spilled 30 VGPRs inside the loop (one source, 16 tokens, 2560 x 6144:
+    // 15.5 -> 13.7 us with 4; gate/up unchanged).
+    if constexpr (GS != 64) {
+        if (wpt >= 8) {
+            ST_I4MM(8, 1, 16);
+            return st::launch_check("i4mm_kernel");
+        }
+    }
+    if (wpt >= 4) {
+        if (nw == 12)
+            ST_I4MM(4, 1, 12);
+        else
+            ST_I4MM(4, 1, 16);
+    } else {
+        if (nw == 12)
+            ST_I4MM(2, 1, 12);
+        else
+            ST_I4MM(2, 1, 16);
+    }
+    return st::launch_check("i4mm_kernel");
 #undef ST_I4MM
 #undef ST_I4MM_P
 }
