@@ -139,6 +139,7 @@ struct XsCall {
     bool y_f16;
     int M, K, N, gs, nsrc;  // nsrc 2: y = silu(gate) * up
     bool round_w = false;   // f16 x, one source: weights rounded to f16 as the prefill GEMM's
+    bool parts = false;     // columns in several launches where the partial sums of all do not fit
     bool gathered = false;  // the workspace holds the act-order gather of this x, by the call before
 };
 int int4_xs(st_context *ctx, const XsCall &c);

@@ -22,12 +22,15 @@ namespace {
 using namespace st::xs;
 
 // y = epilogue(sum over slices s < ks of part[s][src]), the slices added in
-// pairs (a fixed order), the epilogue silu(gate) * up for two sources.
+// pairs (a fixed order), the epilogue silu(gate) * up for two sources. The
+// partials are of pn columns from n0 on.
 template <int NSRC, bool F16OUT>
-__global__ __launch_bounds__(256) void i4xs_reduce_kernel(const float *__restrict__ part, void *__restrict__ y, int MN,
-                                                          int ks, const float *__restrict__ rsc, int N) {
-    const int idx = blockIdx.x * 256 + threadIdx.x;
+__global__ __launch_bounds__(256) void i4xs_reduce_kernel(const float *__restrict__ part, void *__restrict__ y, int M,
+                                                          int ks, const float *__restrict__ rsc, int N, int n0, int pn) {
+    const int idx = blockIdx.x * 256 + threadIdx.x, MN = M * pn;
     if (idx >= MN) return;
+    const int m = idx / pn;
+    const size_t at = (size_t)m * N + n0 + (idx - m * pn);
     float t[NSRC][kMaxSplit];  // every slice's load issued before the first add
 #pragma unroll
     for (int s = 0; s < kMaxSplit; ++s)
@@ -36,11 +39,11 @@ __global__ __launch_bounds__(256) void i4xs_reduce_kernel(const float *__restric
     float v[NSRC];
 #pragma unroll
     for (int sr = 0; sr < NSRC; ++sr) v[sr] = pair_sum(t[sr]);
-    const float r = NSRC == 2 ? silu_f(v[0]) * v[NSRC - 1] : rsc ? v[0] * rsc[idx / N] : v[0];
+    const float r = NSRC == 2 ? silu_f(v[0]) * v[NSRC - 1] : rsc ? v[0] * rsc[m] : v[0];
     if (F16OUT)
-        static_cast<_Float16 *>(y)[idx] = (_Float16)r;
+        static_cast<_Float16 *>(y)[at] = (_Float16)r;
     else
-        static_cast<float *>(y)[idx] = r;
+        static_cast<float *>(y)[at] = r;
 }
 
 // Act-order: xg[t, k] = x[t, perm[k]] (the sorted weight rows' order), or
@@ -188,7 +191,16 @@ int int4_xs(st_context *ctx, const XsCall &c) {
     size_t off, rsc_off;
     if (!pre_pass(ctx, c, &off, &rsc_off)) return -1;
     if (pre && silu && !half) xm = X_F32;
-    const Split sp = plan(ctx, xm, c.gs, c.qz[0] != nullptr, c.M, c.K, c.N, c.nsrc, ctx->ws ? ctx->ws_bytes - off : 0);
+    const bool hz = c.qz[0] != nullptr;
+    const int ntiles = (c.N + kTileN - 1) / kTileN;
+    const size_t left = ctx->ws ? ctx->ws_bytes - off : 0;
+    auto plan_tiles = [&](int tiles) { return plan(ctx, xm, c.gs, hz, c.M, c.K, std::min(tiles * kTileN, c.N), c.nsrc, left); };
+    // Partial sums of all columns that do not fit: half the columns per launch,
+    // a quarter, ..., at least a tile per CU. (8 MiB of workspace, an lm_head of 4608
+    // x 152064, 9 / 32 tokens: 93 / 229 us, on the integer-limb kernels 186 / 463.)
+    int run = ntiles;  // tiles per launch
+    Split sp = plan_tiles(run);
+    while (!sp.ks && c.parts && run >= 2 * ctx->num_cus) sp = plan_tiles(run = (run + 1) / 2);
     if (!sp.ks) return -1;
     Args a{};
     a.x = c.x;
@@ -222,38 +234,44 @@ int int4_xs(st_context *ctx, const XsCall &c) {
         a.sc[i] = c.sc[j];
         a.qz[i] = c.qz[j];
     }
-    const bool hz = c.qz[0] != nullptr;
-    const int units = c.K / 128, ntiles = (c.N + kTileN - 1) / kTileN;
+    const int units = c.K / 128;
     a.y = c.y;
-    a.part = sp.ks > 1 ? reinterpret_cast<float *>(reinterpret_cast<char *>(ctx->ws) + off) : nullptr;
     a.zoff = c.zoff;
     a.M = c.M;
     a.K = c.K;
     a.N = c.N;
-    a.tq = ntiles / sp.groups;
-    a.trem = ntiles % sp.groups;
-    a.uq = units / sp.ks;
-    a.urem = units % sp.ks;
-    a.ks = sp.ks;
     a.tblocks = (c.M + block_tokens(xm) - 1) / block_tokens(xm);
     a.f16out = c.y_f16;
-    int rc;
-    switch (xm) {
-        case X_F32: rc = c.nsrc == 2 ? xs::launch<X_F32, 2>(ctx, a, c.gs, sp.groups, hz) : xs::launch<X_F32, 1>(ctx, a, c.gs, sp.groups, hz); break;
-        case X_F16: rc = c.nsrc == 2 ? xs::launch<X_F16, 2>(ctx, a, c.gs, sp.groups, hz) : xs::launch<X_F16, 1>(ctx, a, c.gs, sp.groups, hz); break;
-        case X_F16G: rc = xs::launch<X_F16G, 1>(ctx, a, c.gs, sp.groups, hz); break;
-        default: rc = xs::launch<X_F32_SILU, 1>(ctx, a, c.gs, sp.groups, hz); break;
+    for (a.tile0 = 0; a.tile0 < ntiles; a.tile0 += run) {
+        const int tiles = std::min(run, ntiles - a.tile0);
+        if (tiles < run) sp = plan_tiles(tiles);  // (the last launch's, which fits where `run` tiles do)
+        a.pn = std::min(tiles * kTileN, c.N - a.tile0 * kTileN);
+        a.part = sp.ks > 1 ? reinterpret_cast<float *>(reinterpret_cast<char *>(ctx->ws) + off) : nullptr;
+        a.tq = tiles / sp.groups;
+        a.trem = tiles % sp.groups;
+        a.uq = units / sp.ks;
+        a.urem = units % sp.ks;
+        a.ks = sp.ks;
+        int rc;
+        switch (xm) {
+            case X_F32: rc = c.nsrc == 2 ? xs::launch<X_F32, 2>(ctx, a, c.gs, sp.groups, hz) : xs::launch<X_F32, 1>(ctx, a, c.gs, sp.groups, hz); break;
+            case X_F16: rc = c.nsrc == 2 ? xs::launch<X_F16, 2>(ctx, a, c.gs, sp.groups, hz) : xs::launch<X_F16, 1>(ctx, a, c.gs, sp.groups, hz); break;
+            case X_F16G: rc = xs::launch<X_F16G, 1>(ctx, a, c.gs, sp.groups, hz); break;
+            default: rc = xs::launch<X_F32_SILU, 1>(ctx, a, c.gs, sp.groups, hz); break;
+        }
+        if (rc) return rc;
+        if (sp.ks == 1) continue;
+        const dim3 g((c.M * a.pn + 255) / 256), b(256);
+        const int n0 = a.tile0 * kTileN;
+        if (c.nsrc == 2)
+            c.y_f16 ? st::launch(ctx, i4xs_reduce_kernel<2, true>, g, b, 0, a.part, a.y, c.M, sp.ks, a.rsc, c.N, n0, a.pn)
+                    : st::launch(ctx, i4xs_reduce_kernel<2, false>, g, b, 0, a.part, a.y, c.M, sp.ks, a.rsc, c.N, n0, a.pn);
+        else
+            c.y_f16 ? st::launch(ctx, i4xs_reduce_kernel<1, true>, g, b, 0, a.part, a.y, c.M, sp.ks, a.rsc, c.N, n0, a.pn)
+                    : st::launch(ctx, i4xs_reduce_kernel<1, false>, g, b, 0, a.part, a.y, c.M, sp.ks, a.rsc, c.N, n0, a.pn);
+        if (int rr = launch_check("i4xs_reduce_kernel")) return rr;
     }
-    if (rc || sp.ks == 1) return rc;
-    const int mn = c.M * c.N;
-    const dim3 g((mn + 255) / 256), b(256);
-    if (c.nsrc == 2)
-        c.y_f16 ? st::launch(ctx, i4xs_reduce_kernel<2, true>, g, b, 0, a.part, a.y, mn, sp.ks, a.rsc, c.N)
-                : st::launch(ctx, i4xs_reduce_kernel<2, false>, g, b, 0, a.part, a.y, mn, sp.ks, a.rsc, c.N);
-    else
-        c.y_f16 ? st::launch(ctx, i4xs_reduce_kernel<1, true>, g, b, 0, a.part, a.y, mn, sp.ks, a.rsc, c.N)
-                : st::launch(ctx, i4xs_reduce_kernel<1, false>, g, b, 0, a.part, a.y, mn, sp.ks, a.rsc, c.N);
-    return launch_check("i4xs_reduce_kernel");
+    return ST_OK;
 }
 
 // Fitted to 1800 drawn calls of 33-256 tokens (MI355X, cold weights: within 6% rms).

@@ -28,7 +28,8 @@
 //    that XCD's L2 after (on any XCDs, in grids that are no multiple of 8: 3
 //    blocks 6% slower over 307 drawn prompts, up to 13%, 5 blocks 8%).
 //  * Few tiles, or K beyond what the waves hold: K slices across workgroups,
-//    f32 partials in the workspace, added in a fixed order by a reduce launch.
+//    f32 partials in the workspace, added in a fixed order by a reduce launch;
+//    where those of all columns do not fit, the columns in several launches.
 #pragma once
 #include "common.hpp"
 #include "i4frag.hpp"
@@ -78,6 +79,7 @@ struct Args {
     float *part;  // K slices' partial sums (ks > 1)
     const float *rsc;  // or nullptr: factor of each token's y (one source)
     int zoff, M, K, N, tq, trem, uq, urem, ks, tblocks, f16out;  // tq, trem: tiles / runs; uq, urem: 128-k units / K slices
+    int tile0, pn;  // the launch's first tile; columns of the partial sums
 };
 
 // launch_gs<XM, NSRC, GS> for the group size; groups: runs of tiles
@@ -154,7 +156,7 @@ __global__ __launch_bounds__(64 * kWaves) void i4xs_kernel(Args a) {
     const int ksl = id % a.ks, grp = id / a.ks;
     // (the first ntiles % groups runs are one tile longer; likewise the K
     // slices' units, and the units of a slice over its waves)
-    const int t0 = grp * a.tq + min(grp, a.trem), nt = a.tq + (grp < a.trem ? 1 : 0);
+    const int t0 = a.tile0 + grp * a.tq + min(grp, a.trem), nt = a.tq + (grp < a.trem ? 1 : 0);
     const int G = a.K / GS, K = a.K, N = a.N;
     const int us = a.uq + (ksl < a.urem ? 1 : 0);
     const int nu = us / kWaves + (wave < us % kWaves ? 1 : 0);  // this wave's units: U or U - 1 (less in short slices)
@@ -459,7 +461,7 @@ __global__ __launch_bounds__(64 * kWaves) void i4xs_kernel(Args a) {
             if (t + rt >= nt || m >= a.M || nc >= N) continue;
             if (a.ks > 1) {
 #pragma unroll
-                for (int sr = 0; sr < NSRC; ++sr) a.part[((size_t)(ksl * NSRC + sr) * a.M + m) * N + nc] = y[sr];
+                for (int sr = 0; sr < NSRC; ++sr) a.part[((size_t)(ksl * NSRC + sr) * a.M + m) * a.pn + nc - kTileN * a.tile0] = y[sr];
                 continue;
             }
             const float yv = NSRC == 2 ? silu_f(y[0]) * y[NSRC - 1] : a.rsc ? y[0] * a.rsc[m] : y[0];

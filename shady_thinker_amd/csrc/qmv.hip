@@ -126,7 +126,7 @@ int launch_f16(st_context *ctx, const QmvParams &p, bool tiled, int nsrc, int xm
     if (use_i4mm(ctx, p, ntiles, nsrc, xm))
         return st::int4_mm_f16(ctx, p.x, xm == XM_F32, p.perm, p.qw, p.sc, p.qz, p.zoff, p.y, p.M, p.K, p.N, p.gs, nsrc);
     const st::XsCall c{p.x, xm == XM_SILU ? p.xb : nullptr, xm == XM_F16, p.perm, {p.qw[0], p.qw[1]}, {p.sc[0], p.sc[1]},
-                       {p.qz[0], p.qz[1]}, p.zoff, p.y, false, p.M, p.K, p.N, p.gs, nsrc};
+                       {p.qz[0], p.qz[1]}, p.zoff, p.y, false, p.M, p.K, p.N, p.gs, nsrc, false, true};
     return st::int4_xs(ctx, c);
 }
 

@@ -10,7 +10,7 @@ import pytest
 import torch
 
 import shady_thinker_amd as sta
-from shady_thinker_amd._lib import ST_ERR_WORKSPACE, ST_F32, call, lib
+from shady_thinker_amd._lib import ST_ERR_WORKSPACE, ST_F32, call, launches, lib
 
 pytestmark = pytest.mark.gpu
 
@@ -46,6 +46,29 @@ def test_noalloc_matches_matvec(gpu, orc, first, second):
         assert torch.equal(y, y_ref), (Mr, K, N)
         ref = orc.gptq_matvec_f64(c["x"], c["qweight"], c["scales"], K, N, 128, qzeros=c["qzeros"])
         assert orc.rel_l2(y.cpu().numpy(), ref) < TOL
+
+
+@pytest.mark.parametrize("Mr,K,N,gs,zeros", [(32, 4608, 33032, 128, False), (9, 5120, 120016, 64, True)])
+def test_noalloc_wide_long_k(gpu, orc, Mr, K, N, gs, zeros):
+    """K slices whose partial sums of all columns exceed the scratch: the
+    columns in several launches (not the integer-limb kernels), each column
+    what the plain call gives up to its K split."""
+    c = orc.gptq_case(410 + Mr, K, N, gs, zeros=zeros, M=Mr)
+    w = sta.GptqWeight.upload(gpu, c["qweight"], c["scales"], gs, qzeros=c["qzeros"])
+    x = torch.from_numpy(c["x"]).cuda()
+    y_ref, y = (torch.full((Mr, N), float("nan"), device="cuda") for _ in range(2))
+    _mv(gpu, "st_gptq_i4_matvec", x, w, y_ref)
+    launches()
+    _mv(gpu, "st_gptq_i4_matvec_noalloc", x, w, y)
+    ran = launches()
+    torch.cuda.synchronize()
+    assert set(ran) == {"i4xs_kernel", "i4xs_reduce_kernel"} and ran.count("i4xs_kernel") > 1, ran
+    assert ((y - y_ref).norm() / y_ref.norm()).item() < 5e-7  # f32 sums in another order
+    for n0 in (0, N // 16 // 2 * 16 - 64, N - 136):  # (the first columns, around a launch's end, the last)
+        n1 = n0 + 136
+        ref = orc.gptq_matvec_f64(c["x"], np.ascontiguousarray(c["qweight"][:, n0:n1]), np.ascontiguousarray(c["scales"][:, n0:n1]),
+                                  K, n1 - n0, gs, qzeros=None if not zeros else np.ascontiguousarray(c["qzeros"][:, n0 // 8:n1 // 8]))
+        assert orc.rel_l2(y[:, n0:n1].cpu().numpy(), ref) < 1e-6
 
 
 def test_noalloc_rejects_beyond_scratch(gpu):
