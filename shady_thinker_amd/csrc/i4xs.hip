@@ -157,7 +157,8 @@ Split plan(const st_context *ctx, int xm, int gs, bool hz, int M, int K, int N, 
         int groups = std::min(ntiles, std::max(1, ctx->num_cus / (ks * tb)));
         const int tq = (ntiles + groups - 1) / groups;
         const double waves = std::max(1.0, (double)groups * ks * tb / ctx->num_cus);  // (more token blocks than CUs)
-        const double us = waves * U * (x_us + tile_us * nsrc * tq) + (ks > 1 ? 1.7 + bytes * 2 / 3e6 : 0.0);
+        const double us = waves * U * (x_us + tile_us * nsrc * tq) * (spills(xm, nsrc, gs, hz, U) ? 1.55 : 1.0) +
+                          (ks > 1 ? 1.7 + bytes * 2 / 3e6 : 0.0);
         if (us < least) {
             least = us;
             best.ks = ks;

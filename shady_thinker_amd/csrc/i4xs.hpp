@@ -57,16 +57,21 @@ constexpr bool is_half(int xm) { return xm == X_F16 || xm == X_F16G; }  // one f
 constexpr int kWaves = 8;                   // waves per workgroup
 // 128-k units per wave at most: their weights, fragments and sums are in
 // registers, two f32 inputs of silu(a) * b at first too, and where they spill
-// one unit less is faster or the same. us at 4 / 3 units (128), 3 / 2 (64):
-// gate/up with zero points 4096 x 14336, 32 tokens, f32 x, group 128 36.8 /
-// 31.8, group 256 38.5 / 33.4, f16 x 26.9 / 24.9 and 29.0 / 25.8; 5632 x 9728
-// group 64 f32 x 51.5 / 37.8, f16 x 31.6 / 26.7. One source with zero points:
-// 4 in groups 128 and 256 (f16 x: 8 registers spilled; f32 x, two units at a
-// time, none; from 5% slower than 3 units, 3328 x 4096, to 5% faster, 4096 x
-// 14336), 3 in groups of 64 (20-28 spilled at 4: 4096 x 14336, f16 x, 23.1 /
-// 16.6).
+// one unit less is faster or the same. us at 4 / 3 units: gate/up with zero
+// points 4096 x 14336, 32 tokens, f32 x, group 128 36.8 / 31.8, group 256 38.5 /
+// 33.4, f16 x 26.9 / 24.9 and 29.0 / 25.8. One source with zero points: 4 in
+// groups 128 and 256 (f16 x: 8 registers spilled; f32 x, two units at a time,
+// none; from 5% slower than 3 units, 3328 x 4096, to 5% faster, 4096 x 14336), 3
+// in groups of 64 (20-28 spilled at 4: 4096 x 14336, f16 x, 23.1 / 16.6).
 constexpr int max_units(int xm, int nsrc, int gs, bool hz) {
-    return xm == X_F32_SILU ? 2 : xm == X_F16G || !hz ? 4 : 4 - (nsrc == 2) - (gs == 64);
+    return xm == X_F32_SILU ? 2 : xm == X_F16G || !hz ? 4 : gs == 64 || nsrc == 2 ? 3 : 4;
+}
+// Gate/up with zero points in groups of 64: three units spill 8-10 registers and
+// take half as long again. Faster than two all the same where two need K slices
+// for many columns (plan; 2560 x 12656, 31 tokens, 2 / 3 units 31.1 / 26.7 us,
+// 2816 x 10160, 13 tokens, 16.4 / 19.7, 5632 x 9728 37.8 / 51.5).
+constexpr bool spills(int xm, int nsrc, int gs, bool hz, int U) {
+    return (xm == X_F32 || xm == X_F16) && nsrc == 2 && gs == 64 && hz && U == 3;
 }
 constexpr int block_tokens(int xm) { return is_half(xm) ? 32 : 16; }
 
@@ -373,7 +378,7 @@ __global__ __launch_bounds__(64 * kWaves) void i4xs_kernel(Args a) {
         // itself, was rounded to lo's steps at every MFMA. Four units of them go
         // two by two: with all eight sums and zero points live six registers
         // spilled (3840 x 75936, 12 tokens, 45.6 / 40.0 us).
-        constexpr int PU = SCALED && NU == 4 ? 2 : NU;  // units at a time
+        constexpr int PU = SCALED && (NU == 4 || (NU == 3 && spills(XM, NSRC, GS, HZ, NU))) ? 2 : NU;  // units at a time
         constexpr int NA = ROUND ? (NU < 2 ? NU : 2) : PU;  // (ROUND: units may share accumulators)
         f32x4 acc[NA][2];
 #pragma unroll
@@ -388,20 +393,20 @@ __global__ __launch_bounds__(64 * kWaves) void i4xs_kernel(Args a) {
                     const int step = EK * j + e;
                     half8 b[PU];
 #pragma unroll
-                    for (int u = 0; u < PU; ++u) {
+                    for (int u = 0; u < PU && p + u < NU; ++u) {
                         b[u] = word_to_b(ring[rr][p + u][step], zlo[p + u][j], zhi[p + u][j]);
                         if constexpr (ROUND) b[u] *= (_Float16)sf[p + u][j];  // (sf: an f16 value)
                     }
 #pragma unroll
-                    for (int u = 0; u < PU; ++u)
+                    for (int u = 0; u < PU && p + u < NU; ++u)
                         acc[u % NA][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[p + u][step][0], b[u], acc[u % NA][0], 0, 0, 0);
 #pragma unroll
-                    for (int u = 0; u < PU; ++u)
+                    for (int u = 0; u < PU && p + u < NU; ++u)
                         acc[u % NA][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xa[p + u][step][1], b[u], acc[u % NA][1], 0, 0, 0);
                 }
                 if constexpr (!ROUND)
 #pragma unroll
-                    for (int u = 0; u < PU; ++u)
+                    for (int u = 0; u < PU && p + u < NU; ++u)
 #pragma unroll
                         for (int mb = 0; mb < MB; ++mb)
 #pragma unroll

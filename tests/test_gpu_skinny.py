@@ -109,7 +109,9 @@ def test_skinny_silu_matvec(gpu, orc, Mr, K, N, gs, zeros, act):
     (9, 1536, 4120, 128, True, False, False),
     (32, 4096, 1032, 64, False, False, False),
     (17, 5120, 776, 256, True, True, True),
-    (12, 3328, 1032, 64, True, False, False),  # group 64 with zero points: three units a wave at most
+    (12, 3328, 1032, 64, True, False, False),  # group 64 with zero points: two units a wave, K slices
+    (32, 2304, 14336, 64, True, False, False),  # three (many columns of two token blocks): K in one piece
+    (27, 2560, 13064, 64, True, True, True),
 ])
 def test_skinny_gate_up(gpu, orc, Mr, K, N, gs, zeros, act, f16):
     c = _case(orc, 900 + Mr, K, N, gs, zeros, act, Mr, f16)
@@ -118,8 +120,11 @@ def test_skinny_gate_up(gpu, orc, Mr, K, N, gs, zeros, act, f16):
     g, u = _up(gpu, c, gs), _up(gpu, c2, gs)
     x = torch.from_numpy(c["x"]).cuda()
     y = torch.full((Mr, N), float("nan"), device="cuda")
+    launches()
     M.fused_gate_up_silu(gpu, x, g.qweight, g.scales, u.qweight, u.scales, y, K, N, gs, gate_qz=g.qzeros, up_qz=u.qzeros,
                          perm=g.perm, flags=g.flags)
+    ran = launches()
+    assert "i4xs_kernel" in ran and (N < 13064 or "i4xs_reduce_kernel" not in ran)
     torch.cuda.synchronize()
     ref = orc.silu_gate_f64(_ref(orc, c, c["x"], K, N, gs, act), _ref(orc, c2, c["x"], K, N, gs, act))
     assert orc.rel_l2(y.cpu().numpy(), ref) < 3e-6  # silu and the product add their own f32 steps
